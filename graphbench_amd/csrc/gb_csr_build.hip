@@ -4,60 +4,447 @@
 // pass (scan_csr_idx, graph/csr.c:133-202) and a scatter in file order
 // (read_graph_csr, graph/csr.c:4-66; read_csr_bin, graph/csr.c:211-299).  Here
 // the edge list is on the device and the CSR is one stable radix sort of the
-// row keys (edges of a row keep their input order, as the reference's scatter
-// does), a histogram and a prefix sum.  The transpose of a CSR is the same
-// construction with the endpoints swapped.
+// edges by row (edges of a row keep their input order, as the reference's
+// scatter does) that carries the other endpoint and the weight along, and a
+// search of the sorted rows for the row offsets.  The transpose of a CSR is
+// the same construction with the endpoints swapped.
+//
+// What bounds it: bytes.  A pass reads and writes an edge once (12 bytes with
+// 4-byte weights each way) and reads its key once more for the histogram.
+// Against a sort of (row, index) pairs, a gather of the payload through the
+// sorted indices and one atomic per edge for the row counts, a CSR of R-MAT 20
+// (16.8 M edges) takes 0.53 ms instead of 5.4 ms: the row counts took 2.6 ms
+// of it, serialised on the hubs' counters, the gather 0.64 ms, a 64-byte line
+// per 4-byte value, and allocations 1.5 ms.
 #include <hip/hip_runtime.h>
 #include <hipcub/device/device_radix_sort.hpp>
 #include <hipcub/device/device_scan.hpp>
 
+#include <algorithm>
+#include <atomic>
+#include <thread>
+
+#include "gb_device.hpp"
 #include "graphbench.h"
 #include "gb_internal.hpp"
 
 namespace {
 
-__global__ void iota_kernel(int64_t n, int32_t *__restrict__ a) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    a[i] = (int32_t)i;
+// ---- stable radix sort by row, payload carried -----------------------------
+// Least significant digit first, digits of at most RS_MAX_BITS bits, a tile of
+// RS_TILE consecutive edges per block.  A pass is four launches: the tiles'
+// digit counts, two levels of scan over the tiles (groups of RS_GROUP), and
+// the scatter.  Tile-major counts keep every access of the scans coalesced.
+constexpr int RS_BLOCK = 256;
+constexpr int RS_WAVES = RS_BLOCK / GB_WAVE;
+constexpr int RS_TILE = 8192;
+constexpr int RS_ITEMS = RS_TILE / RS_BLOCK;       // edges per thread
+// the scatter: 8 waves per tile, each over RS_SEG consecutive edges
+constexpr int RS_SBLOCK = 1024;
+constexpr int RS_SWAVES = RS_SBLOCK / GB_WAVE;
+constexpr int RS_SITEMS = RS_TILE / RS_SBLOCK;
+constexpr int RS_SEG = RS_TILE / RS_SWAVES;
+constexpr int RS_MAX_BITS = 11;
+constexpr int RS_GROUP = 64;                       // tiles per scan group
+
+// Digit counts of every tile: hist[tile * D + digit].  The first pass also
+// checks the endpoints: a bad one sets *bad, which makes every later kernel
+// of the build return at once (nothing is written); its digit is masked, so
+// the count stays inside the table.
+template <bool CHECK>
+__global__ __launch_bounds__(RS_BLOCK) void rs_hist_kernel(
+    int64_t E, int32_t V, const int32_t *__restrict__ key, const int32_t *__restrict__ other,
+    int shift, int bits, uint32_t *__restrict__ hist, int *__restrict__ bad) {
+  __shared__ uint32_t s_cnt[1 << RS_MAX_BITS];
+  if (!CHECK && *bad) return;
+  const int D = 1 << bits;
+  for (int d = threadIdx.x; d < D; d += RS_BLOCK) s_cnt[d] = 0;
+  __syncthreads();
+  const int64_t t0 = (int64_t)blockIdx.x * RS_TILE;
+  bool wrong = false;
+  for (int k0 = 0; k0 < RS_ITEMS; k0 += 8) {
+    int32_t a[8], b[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {  // clamped: the reads stay one batch
+      const int64_t e = min(t0 + (int64_t)(k0 + k) * RS_BLOCK + threadIdx.x, E - 1);
+      a[k] = key[e];
+      if (CHECK) b[k] = other[e];
+    }
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const bool in = t0 + (int64_t)(k0 + k) * RS_BLOCK + threadIdx.x < E;
+      if (CHECK) wrong |= a[k] < 0 || a[k] >= V || b[k] < 0 || b[k] >= V;
+      if (in) atomicAdd(&s_cnt[((uint32_t)a[k] >> shift) & (D - 1)], 1u);
+    }
+  }
+  if (CHECK && wrong) *bad = 1;
+  __syncthreads();
+  for (int d = threadIdx.x; d < D; d += RS_BLOCK)
+    hist[(int64_t)blockIdx.x * D + d] = s_cnt[d];
 }
 
-__global__ void count_rows_kernel(int64_t E, const int32_t *__restrict__ key,
-                                  int32_t *__restrict__ deg) {
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < E;
-       e += (int64_t)gridDim.x * blockDim.x)
-    atomicAdd(&deg[key[e]], 1);
+// Exclusive scan of the counts over the RS_GROUP tiles of a group, in place;
+// the group's totals to gsum[group * D + digit].  A block takes 64 digits, a
+// wave 16 of the tiles.
+__global__ __launch_bounds__(RS_BLOCK) void rs_scan_kernel(int64_t ntiles, int D,
+                                                           uint32_t *__restrict__ hist,
+                                                           uint32_t *__restrict__ gsum,
+                                                           const int *__restrict__ bad) {
+  constexpr int PER = RS_GROUP / RS_WAVES;
+  __shared__ uint32_t s_sum[RS_WAVES][GB_WAVE];
+  if (*bad) return;
+  const int w = threadIdx.x >> 6, lane = gb_lane();
+  const int d = blockIdx.x * GB_WAVE + lane;
+  const int64_t t0 = (int64_t)blockIdx.y * RS_GROUP + w * PER;
+  uint32_t x[PER], sum = 0;
+#pragma unroll
+  for (int k = 0; k < PER; k++)
+    x[k] = d < D && t0 + k < ntiles ? hist[(t0 + k) * D + d] : 0u;
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    const uint32_t v = x[k];
+    x[k] = sum;
+    sum += v;
+  }
+  s_sum[w][lane] = sum;
+  __syncthreads();
+  uint32_t base = 0, tot = 0;
+  for (int q = 0; q < RS_WAVES; q++) {
+    if (q < w) base += s_sum[q][lane];
+    tot += s_sum[q][lane];
+  }
+#pragma unroll
+  for (int k = 0; k < PER; k++)
+    if (d < D && t0 + k < ntiles) hist[(t0 + k) * D + d] = base + x[k];
+  if (w == 0 && d < D) gsum[(int64_t)blockIdx.y * D + d] = tot;
 }
 
-template <int WB>
-__global__ void gather_cols_kernel(int64_t E, const int32_t *__restrict__ perm,
-                                   const int32_t *__restrict__ dst, const void *__restrict__ w,
-                                   int32_t *__restrict__ col, void *__restrict__ w_out) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < E;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int32_t p = perm[i];
-    col[i] = dst[p];
-    if (WB == 4) ((uint32_t *)w_out)[i] = ((const uint32_t *)w)[p];
-    if (WB == 8) ((double *)w_out)[i] = ((const double *)w)[p];
+// Exclusive scan of the groups' totals over the groups, in place; the digits'
+// totals to total[digit].
+__global__ __launch_bounds__(GB_WAVE) void rs_groups_kernel(int64_t ngroups, int D,
+                                                            uint32_t *__restrict__ gsum,
+                                                            uint32_t *__restrict__ total,
+                                                            const int *__restrict__ bad) {
+  if (*bad) return;
+  const int d = blockIdx.x * GB_WAVE + threadIdx.x;
+  if (d >= D) return;
+  uint32_t sum = 0;
+  for (int64_t g0 = 0; g0 < ngroups; g0 += 16) {
+    uint32_t x[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) x[k] = g0 + k < ngroups ? gsum[(g0 + k) * D + d] : 0u;
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+      if (g0 + k < ngroups) gsum[(g0 + k) * D + d] = sum;
+      sum += x[k];
+    }
+  }
+  total[d] = sum;
+}
+
+// Exclusive scan of s[0 .. N) by a block of NB threads (N a power of two).
+template <int NB, int N>
+__device__ __forceinline__ void rs_block_scan(uint32_t *s) {
+  constexpr int PER = N > NB ? N / NB : 1, NW = NB / GB_WAVE;
+  __shared__ uint32_t s_w[NW];
+  const int b = threadIdx.x * PER;
+  uint32_t x[PER], sum = 0;
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    x[k] = b + k < N ? s[b + k] : 0u;
+    sum += x[k];
+  }
+  uint32_t wt;
+  uint32_t ex = gb_wave_excl_sum(sum, &wt);
+  if (gb_lane() == 0) s_w[threadIdx.x >> 6] = wt;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NW; q++) ex += q < (int)(threadIdx.x >> 6) ? s_w[q] : 0u;
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    if (b + k < N) s[b + k] = ex;
+    ex += x[k];
+  }
+  __syncthreads();
+}
+
+// Moves a tile's edges to their digits' places, keeping their order.  A wave
+// owns RS_SEG consecutive edges and ranks them 64 at a time: the lanes with
+// the same digit find each other with one ballot per digit bit, and the
+// wave's own counter of the digit (LDS, one writer) gives the rank of the
+// first.  The tile is then put in digit order in LDS, one array after the
+// other, so that a digit's edges leave as one run of consecutive addresses:
+// written straight from the ranking lanes, each edge was a write request of
+// its own and a pass over 16.8 M edges took 426 us instead of
+// 173 us (2.3 TB/s).
+// Digits have BITS bits; LDS is 34, 40 or 80 KiB at 8, 10 or 11.  At 10 and 11
+// bits the kernel keeps its 89 registers (one block of 16 waves per CU): held
+// to 64 for two blocks it spills, 205 us a pass.  At 8 bits it spills little
+// and two blocks win (R-MAT 24 with 134 M edges, a CSR and its reverse: 8.4
+// against 9.2 ms).
+template <int WB, int BITS>
+__global__ __launch_bounds__(RS_SBLOCK)
+__attribute__((amdgpu_waves_per_eu(BITS == 8 ? 8 : 4))) void rs_scatter_kernel(
+    int64_t E, const int32_t *__restrict__ key, const int32_t *__restrict__ val,
+    const void *__restrict__ w, int shift, const uint32_t *__restrict__ hist,
+    const uint32_t *__restrict__ gsum, const uint32_t *__restrict__ total,
+    int32_t *__restrict__ key_out, int32_t *__restrict__ val_out, void *__restrict__ w_out,
+    const int *__restrict__ bad) {
+  constexpr int D = 1 << BITS;
+  __shared__ uint32_t s_delta[D];  // global minus tile place of a digit
+  __shared__ uint32_t s_place[D];  // tile place of a digit
+  // the tile takes the counters' place once the ranks are known
+  constexpr int CNT_WORDS = RS_SWAVES * D / 2;
+  __shared__ uint32_t s_tile[RS_TILE > CNT_WORDS ? RS_TILE : CNT_WORDS];
+  uint16_t *s_cnt = (uint16_t *)s_tile;  // [RS_SWAVES][D]
+  if (*bad) return;
+  for (int d = threadIdx.x; d < D; d += RS_SBLOCK) s_delta[d] = total[d];
+  for (int d = threadIdx.x; d < RS_SWAVES * D / 2; d += RS_SBLOCK) ((uint32_t *)s_cnt)[d] = 0;
+  __syncthreads();
+  rs_block_scan<RS_SBLOCK, D>(s_delta);
+  const int wv = threadIdx.x >> 6, lane = gb_lane();
+  const uint64_t below = (1ull << lane) - 1;
+  const int64_t t0 = (int64_t)blockIdx.x * RS_TILE;
+  const int n = (int)min((int64_t)RS_TILE, E - t0);
+  const int32_t *tkey = key + t0, *tval = val + t0;
+  const int i0 = wv * RS_SEG + lane;  // this lane's first edge in the tile
+  volatile uint16_t *cnt = s_cnt + wv * D;
+  uint32_t at[RS_SITEMS];  // digit | rank << 16, then the place in the tile
+  int32_t kk[RS_SITEMS];
+#pragma unroll
+  for (int r = 0; r < RS_SITEMS; r++) kk[r] = tkey[(uint32_t)min(i0 + r * GB_WAVE, n - 1)];
+#pragma unroll
+  for (int r = 0; r < RS_SITEMS; r++) {
+    const bool in = i0 + r * GB_WAVE < n;
+    const uint32_t d = ((uint32_t)kk[r] >> shift) & (D - 1);
+    uint64_t peers = __ballot(in);
+#pragma unroll
+    for (int b = 0; b < BITS; b++) {
+      const bool one = (d >> b) & 1u;
+      const uint64_t m = __ballot(one);
+      peers &= one ? m : ~m;
+    }
+    uint32_t old = 0;
+    if (in) old = cnt[d];
+    __builtin_amdgcn_wave_barrier();
+    if (in && (peers & below) == 0) cnt[d] = (uint16_t)(old + (uint32_t)__popcll(peers));
+    __builtin_amdgcn_wave_barrier();
+    at[r] = d | (old + (uint32_t)__popcll(peers & below)) << 16;
+  }
+  __syncthreads();
+  // the tile's counts of each digit, their scan, and each wave's first place
+  for (int d = threadIdx.x; d < D; d += RS_SBLOCK) {
+    uint32_t c = 0;
+    for (int q = 0; q < RS_SWAVES; q++) c += s_cnt[q * D + d];
+    s_place[d] = c;
+  }
+  __syncthreads();
+  rs_block_scan<RS_SBLOCK, D>(s_place);
+  const int64_t g = blockIdx.x / RS_GROUP;
+  for (int d = threadIdx.x; d < D; d += RS_SBLOCK) {
+    uint32_t p = s_place[d];
+    s_delta[d] += gsum[g * D + d] + hist[(int64_t)blockIdx.x * D + d] - p;
+    for (int q = 0; q < RS_SWAVES; q++) {
+      const uint32_t c = s_cnt[q * D + d];
+      s_cnt[q * D + d] = (uint16_t)p;  // < RS_TILE where c > 0
+      p += c;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < RS_SITEMS; r++) at[r] = s_cnt[wv * D + (at[r] & 0xFFFFu)] + (at[r] >> 16);
+  __syncthreads();  // the counters give way to the tile
+  // the keys give every place its address; the other arrays follow
+  uint32_t dest[RS_SITEMS];
+#pragma unroll
+  for (int r = 0; r < RS_SITEMS; r++)
+    if (i0 + r * GB_WAVE < n) s_tile[at[r]] = (uint32_t)kk[r];
+  __syncthreads();
+  int32_t x[RS_SITEMS];
+#pragma unroll
+  for (int r = 0; r < RS_SITEMS; r++) x[r] = tval[(uint32_t)min(i0 + r * GB_WAVE, n - 1)];
+#pragma unroll
+  for (int r = 0; r < RS_SITEMS; r++) {
+    const int i = r * RS_SBLOCK + threadIdx.x;
+    if (i < n) {
+      const uint32_t k = s_tile[i];
+      dest[r] = (uint32_t)i + s_delta[(k >> shift) & (D - 1)];
+      key_out[dest[r]] = (int32_t)k;
+    }
+  }
+  // one 4-byte array through the tile: out word dest * step + off
+  auto move = [&](uint32_t *out, int step, int off) {
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RS_SITEMS; r++)
+      if (i0 + r * GB_WAVE < n) s_tile[at[r]] = (uint32_t)x[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RS_SITEMS; r++) {
+      const int i = r * RS_SBLOCK + threadIdx.x;
+      if (i < n) out[(uint64_t)dest[r] * step + off] = s_tile[i];
+    }
+  };
+  move((uint32_t *)val_out, 1, 0);
+  for (int h = 0; h < WB / 4; h++) {
+    const int32_t *ws = (const int32_t *)w + t0 * (WB / 4) + h;
+#pragma unroll
+    for (int r = 0; r < RS_SITEMS; r++)
+      x[r] = ws[(uint32_t)(min(i0 + r * GB_WAVE, n - 1) * (WB / 4))];
+    move((uint32_t *)w_out, WB / 4, h);
   }
 }
 
-// out-of-range endpoints are reported, not written
-__global__ void check_ids_kernel(int64_t E, int32_t V, const int32_t *__restrict__ a,
-                                 const int32_t *__restrict__ b, int *__restrict__ bad) {
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < E;
-       e += (int64_t)gridDim.x * blockDim.x)
-    if (a[e] < 0 || a[e] >= V || b[e] < 0 || b[e] >= V) *bad = 1;
+// row_ptr[r] = first index whose row is >= r, for r in [0, V]: a binary search
+// per row in the sorted rows, inside the edges that share its high digit
+// (total: the last pass's digit counts, `shift` its shift).
+__global__ __launch_bounds__(RS_BLOCK) void rs_rows_kernel(int32_t V, int64_t E,
+                                                           const int32_t *__restrict__ row,
+                                                           int shift, int bits,
+                                                           const uint32_t *__restrict__ total,
+                                                           int32_t *__restrict__ row_ptr,
+                                                           const int *__restrict__ bad) {
+  constexpr int MAXD = 1 << RS_MAX_BITS;
+  __shared__ uint32_t s_base[MAXD + 1];
+  if (*bad) return;
+  const int D = 1 << bits;
+  for (int d = threadIdx.x; d < MAXD; d += RS_BLOCK) s_base[d] = d < D ? total[d] : 0u;
+  __syncthreads();
+  rs_block_scan<RS_BLOCK, MAXD>(s_base);
+  if (threadIdx.x == 0) s_base[D] = (uint32_t)E;
+  __syncthreads();
+  for (int64_t r = (int64_t)blockIdx.x * RS_BLOCK + threadIdx.x; r <= V;
+       r += (int64_t)gridDim.x * RS_BLOCK) {
+    const int64_t d = r >> shift;  // r = V may lie past the last digit
+    uint32_t lo = d < D ? s_base[d] : (uint32_t)E, hi = d < D ? s_base[d + 1] : (uint32_t)E;
+    while (lo < hi) {
+      const uint32_t mid = lo + (hi - lo) / 2;
+      if (row[mid] < r)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    row_ptr[r] = (int32_t)lo;
+  }
 }
 
-// row id of every edge of a CSR
-__global__ void expand_rows_kernel(int32_t V, const int32_t *__restrict__ rp,
-                                   int32_t *__restrict__ row) {
-  const int lane = threadIdx.x & 63;
-  const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> 6;
-  for (int64_t v = wave; v < V; v += nwaves)
-    for (int32_t e = rp[v] + lane; e < rp[v + 1]; e += 64) row[e] = (int32_t)v;
+// Row id of every edge of a CSR.  A block takes EX_TILE consecutive edges:
+// the rows that begin inside the tile leave their ids at their first edges
+// (the largest where several begin at one edge: all but the last are empty),
+// and a running maximum over the tile fills the rest.  The first edge's row
+// is found by binary search.  One wave per row had left hub rows to one wave
+// (R-MAT 20: 201 us, now 48 us).
+constexpr int EX_ITEMS = 16;
+constexpr int EX_TILE = RS_BLOCK * EX_ITEMS;
+__global__ __launch_bounds__(RS_BLOCK) void expand_rows_kernel(int32_t V, int64_t E,
+                                                               const int32_t *__restrict__ rp,
+                                                               int32_t *__restrict__ row) {
+  __shared__ int32_t s_row[EX_TILE];
+  __shared__ int32_t s_wmax[RS_WAVES];
+  __shared__ int32_t s_lim[2];
+  const int64_t t0 = (int64_t)blockIdx.x * EX_TILE;
+  const int64_t t1 = min(t0 + EX_TILE, E);
+  for (int i = threadIdx.x; i < EX_TILE; i += RS_BLOCK) s_row[i] = 0;
+  if (threadIdx.x < 2) {
+    // thread 0: last row with rp <= t0 (the first edge's row); thread 1: last
+    // row with rp < t1
+    const int64_t x = threadIdx.x ? t1 - 1 : t0;
+    int32_t lo = 0, hi = V;  // rp[lo] <= x < rp[hi] = E
+    while (hi - lo > 1) {
+      const int32_t mid = lo + (hi - lo) / 2;
+      if (rp[mid] <= x)
+        lo = mid;
+      else
+        hi = mid;
+    }
+    s_lim[threadIdx.x] = lo;
+  }
+  __syncthreads();
+  const int32_t first = s_lim[0], last = s_lim[1];
+  if (last - first > 8 * EX_TILE) {
+    // mostly empty rows: a search per edge instead of a visit per row
+    for (int64_t e = t0 + threadIdx.x; e < t1; e += RS_BLOCK) {
+      int32_t lo = first, hi = last + 1;
+      while (hi - lo > 1) {
+        const int32_t mid = lo + (hi - lo) / 2;
+        if (rp[mid] <= e)
+          lo = mid;
+        else
+          hi = mid;
+      }
+      row[e] = lo;
+    }
+    return;
+  }
+  for (int64_t v = (int64_t)first + 1 + threadIdx.x; v <= last; v += RS_BLOCK) {
+    // rp[v] in (t0, t1) or, for an empty row, at the tile's first edge or
+    // equal to a later row's
+    const int64_t o = rp[v] - t0;
+    if (o >= 0 && o < EX_TILE) atomicMax(&s_row[o], (int32_t)v);
+  }
+  if (threadIdx.x == 0) atomicMax(&s_row[0], first);
+  __syncthreads();
+  // thread i holds EX_ITEMS consecutive edges
+  int32_t m = 0, x[EX_ITEMS];
+#pragma unroll
+  for (int k = 0; k < EX_ITEMS; k++) {
+    m = max(m, s_row[threadIdx.x * EX_ITEMS + k]);
+    x[k] = m;
+  }
+  int32_t incl = m;
+#pragma unroll
+  for (int d = 1; d < GB_WAVE; d <<= 1) {
+    const int32_t y = __shfl_up(incl, d, GB_WAVE);
+    if (gb_lane() >= d) incl = max(incl, y);
+  }
+  if (gb_lane() == GB_WAVE - 1) s_wmax[threadIdx.x >> 6] = incl;
+  int32_t before = __shfl_up(incl, 1, GB_WAVE);
+  if (gb_lane() == 0) before = 0;
+  __syncthreads();
+  for (int q = 0; q < (int)(threadIdx.x >> 6); q++) before = max(before, s_wmax[q]);
+#pragma unroll
+  for (int k = 0; k < EX_ITEMS; k++) s_row[threadIdx.x * EX_ITEMS + k] = max(x[k], before);
+  __syncthreads();
+  for (int64_t e = t0 + threadIdx.x; e < t1; e += RS_BLOCK) row[e] = s_row[e - t0];
+}
+
+// Scratch of the builds, kept between calls up to CSR_KEEP bytes (allocating
+// and freeing it took 1.5 ms of a 5.4 ms build).  One build uses it at a time,
+// on any thread and stream: a build waits for its stream before it lets go of
+// the scratch.  An allocation that would fail elsewhere takes it back first
+// (gb_csr_trim).
+constexpr size_t CSR_KEEP = (size_t)4 << 30;
+struct CsrWork {
+  std::atomic<int> busy{0};
+  DevBuf rows, k[2], v, w, hist, gsum, total, flag;
+  size_t held() const {
+    return rows.bytes + k[0].bytes + k[1].bytes + v.bytes + w.bytes + hist.bytes + gsum.bytes +
+           total.bytes + flag.bytes;
+  }
+  void release() {
+    for (DevBuf *b : {&rows, &k[0], &k[1], &v, &w, &hist, &gsum, &total, &flag}) b->release();
+  }
+};
+// Holds the scratch for one build; at most CSR_KEEP bytes outlive it.
+struct CsrHold {
+  CsrWork &k;
+  explicit CsrHold(CsrWork &work) : k(work) {
+    int idle = 0;
+    while (!k.busy.compare_exchange_weak(idle, 1)) {
+      idle = 0;
+      std::this_thread::yield();
+    }
+  }
+  ~CsrHold() {
+    if (k.held() > CSR_KEEP) k.release();
+    k.busy.store(0);
+  }
+};
+// Heap singleton, never destroyed (no device memory freed from a static
+// destructor).
+CsrWork &csr_work() {
+  static CsrWork *w = new CsrWork();
+  return *w;
 }
 
 int grid_for(int64_t n) {
@@ -157,6 +544,113 @@ extern "C" gb_status gb_edges_unique(int64_t E, const int32_t *d_src, const int3
   return GB_OK;
 }
 
+namespace {
+
+// The build on the workspace (its lock held): edges sorted by d_src.
+template <int WB>
+gb_status csr_build(CsrWork &k, int32_t V, int64_t E, const int32_t *d_src, const int32_t *d_dst,
+                    const void *d_w, int32_t *d_row_ptr, int32_t *d_col, void *d_w_out,
+                    hipStream_t st) {
+  GB_TRY(k.flag.ensure(sizeof(int)));
+  if (E == 0) {
+    GB_HIP(hipMemsetAsync(d_row_ptr, 0, sizeof(int32_t) * ((size_t)V + 1), st));
+    GB_HIP(hipStreamSynchronize(st));
+    return GB_OK;
+  }
+  int bits = 1;
+  while (bits < 31 && ((int64_t)1 << bits) < (int64_t)V) bits++;
+  // as few passes as 11-bit digits allow, with the smallest of 8, 10 and 11
+  // bits that needs no more: a pass costs about as much at each (13, 16 and 10
+  // us per million edges at 10, 11 and 8 bits on R-MAT 20, 22 and 24)
+  const int passes = (bits + RS_MAX_BITS - 1) / RS_MAX_BITS;
+  const int even = (bits + passes - 1) / passes;
+  const int db = even <= 8 ? 8 : even <= 10 ? 10 : 11;
+  const int D = 1 << db;
+  const int64_t ntiles = (E + RS_TILE - 1) / RS_TILE;
+  const int64_t ngroups = (ntiles + RS_GROUP - 1) / RS_GROUP;
+  // the endpoints and weights alternate between the scratch and the caller's
+  // arrays so that the last pass ends in the latter
+  GB_TRY(k.k[0].ensure(sizeof(int32_t) * E));
+  if (passes > 1) {
+    GB_TRY(k.k[1].ensure(sizeof(int32_t) * E));
+    GB_TRY(k.v.ensure(sizeof(int32_t) * E));
+    if (WB) GB_TRY(k.w.ensure((size_t)WB * E));
+  }
+  GB_TRY(k.hist.ensure(sizeof(uint32_t) * ntiles * D));
+  GB_TRY(k.gsum.ensure(sizeof(uint32_t) * ngroups * D));
+  GB_TRY(k.total.ensure(sizeof(uint32_t) * D));
+  int *bad = k.flag.as<int>();
+  uint32_t *hist = k.hist.as<uint32_t>(), *gsum = k.gsum.as<uint32_t>(),
+           *total = k.total.as<uint32_t>();
+  GB_HIP(hipMemsetAsync(bad, 0, sizeof(int), st));
+  const int32_t *key = d_src, *val = d_dst;
+  const void *w = d_w;
+  for (int p = 0; p < passes; p++) {
+    const int shift = p * db;
+    const bool to_caller = (passes - 1 - p) % 2 == 0;
+    if (p == 0)
+      hipLaunchKernelGGL(rs_hist_kernel<true>, dim3((unsigned)ntiles), dim3(RS_BLOCK), 0, st, E, V,
+                         key, val, shift, db, hist, bad);
+    else
+      hipLaunchKernelGGL(rs_hist_kernel<false>, dim3((unsigned)ntiles), dim3(RS_BLOCK), 0, st, E,
+                         V, key, val, shift, db, hist, bad);
+    hipLaunchKernelGGL(rs_scan_kernel, dim3((D + GB_WAVE - 1) / GB_WAVE, (unsigned)ngroups),
+                       dim3(RS_BLOCK), 0, st, ntiles, D, hist, gsum, bad);
+    hipLaunchKernelGGL(rs_groups_kernel, dim3((D + GB_WAVE - 1) / GB_WAVE), dim3(GB_WAVE), 0, st,
+                       ngroups, D, gsum, total, bad);
+    int32_t *ko = k.k[p & 1].as<int32_t>();
+    int32_t *vo = to_caller ? d_col : k.v.as<int32_t>();
+    void *wo = to_caller ? d_w_out : k.w.p;
+    auto scatter = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)ntiles), dim3(RS_SBLOCK), 0, st, E, key, val, w,
+                         shift, hist, gsum, total, ko, vo, wo, bad);
+    };
+    if (db == 8)
+      scatter(rs_scatter_kernel<WB, 8>);
+    else if (db == 10)
+      scatter(rs_scatter_kernel<WB, 10>);
+    else
+      scatter(rs_scatter_kernel<WB, 11>);
+    GB_HIP(hipGetLastError());
+    key = ko;
+    val = vo;
+    w = wo;
+  }
+  hipLaunchKernelGGL(rs_rows_kernel, dim3(grid_for((int64_t)V + 1)), dim3(RS_BLOCK), 0, st, V, E,
+                     key, (passes - 1) * db, db, total, d_row_ptr, bad);
+  GB_HIP(hipGetLastError());
+  int h_bad = 0;
+  GB_HIP(hipMemcpyAsync(&h_bad, bad, sizeof(int), hipMemcpyDeviceToHost, st));
+  GB_HIP(hipStreamSynchronize(st));  // the scratch is idle from here on
+  if (h_bad) return gb_fail(GB_ERR_INVALID, "gb_csr_from_edges: endpoint outside [0, V)");
+  return GB_OK;
+}
+
+gb_status csr_build_any(CsrWork &k, int32_t V, int64_t E, const int32_t *d_src,
+                        const int32_t *d_dst, const void *d_w, int32_t w_bytes, int32_t *d_row_ptr,
+                        int32_t *d_col, void *d_w_out, hipStream_t st) {
+  const gb_status s =
+      w_bytes == 8   ? csr_build<8>(k, V, E, d_src, d_dst, d_w, d_row_ptr, d_col, d_w_out, st)
+      : w_bytes == 4 ? csr_build<4>(k, V, E, d_src, d_dst, d_w, d_row_ptr, d_col, d_w_out, st)
+                     : csr_build<0>(k, V, E, d_src, d_dst, d_w, d_row_ptr, d_col, d_w_out, st);
+  if (s != GB_OK) (void)hipStreamSynchronize(st);  // launches before an error end first
+  return s;
+}
+
+}  // namespace
+
+// Gives the kept scratch back unless a build is using it; returns whether it
+// held anything.
+bool gb_csr_trim() {
+  CsrWork &k = csr_work();
+  int idle = 0;
+  if (!k.busy.compare_exchange_strong(idle, 2)) return false;
+  const bool had = k.held() > 0;
+  k.release();
+  k.busy.store(0);
+  return had;
+}
+
 extern "C" gb_status gb_csr_from_edges(int32_t V, int64_t E, const int32_t *d_src,
                                        const int32_t *d_dst, const void *d_w, int32_t w_bytes,
                                        int32_t *d_row_ptr, int32_t *d_col, void *d_w_out,
@@ -167,57 +661,10 @@ extern "C" gb_status gb_csr_from_edges(int32_t V, int64_t E, const int32_t *d_sr
     return gb_fail(GB_ERR_INVALID, "gb_csr_from_edges: w_bytes must be 0, 4 or 8");
   if (w_bytes && E > 0 && (!d_w || !d_w_out))
     return gb_fail(GB_ERR_INVALID, "gb_csr_from_edges: weights without a weight buffer");
-  hipStream_t st = gb_stream(stream);
-  DevBuf deg, keys_out, ids, perm, flag, tmp;
-  GB_TRY(deg.ensure(sizeof(int32_t) * ((size_t)V + 1)));
-  GB_TRY(flag.ensure(sizeof(int)));
-  GB_HIP(hipMemsetAsync(deg.p, 0, sizeof(int32_t) * ((size_t)V + 1), st));
-  GB_HIP(hipMemsetAsync(flag.p, 0, sizeof(int), st));
-  if (E > 0) {
-    hipLaunchKernelGGL(check_ids_kernel, dim3(grid_for(E)), dim3(256), 0, st, E, V, d_src, d_dst,
-                       flag.as<int>());
-    int bad = 0;
-    GB_HIP(hipMemcpyAsync(&bad, flag.p, sizeof(int), hipMemcpyDeviceToHost, st));
-    GB_HIP(hipStreamSynchronize(st));
-    if (bad) return gb_fail(GB_ERR_INVALID, "gb_csr_from_edges: endpoint outside [0, V)");
-    GB_TRY(keys_out.ensure(sizeof(int32_t) * E));
-    GB_TRY(ids.ensure(sizeof(int32_t) * E));
-    GB_TRY(perm.ensure(sizeof(int32_t) * E));
-    hipLaunchKernelGGL(iota_kernel, dim3(grid_for(E)), dim3(256), 0, st, E, ids.as<int32_t>());
-    hipLaunchKernelGGL(count_rows_kernel, dim3(grid_for(E)), dim3(256), 0, st, E, d_src,
-                       deg.as<int32_t>() + 1);
-    GB_HIP(hipGetLastError());
-    // stable sort of the edge indices by row (LSD radix sort keeps ties in input order)
-    int bits = 1;
-    while (bits < 31 && ((int64_t)1 << bits) < (int64_t)V) bits++;
-    size_t tb_sort = 0, tb_scan = 0;
-    const uint32_t *ukeys = (const uint32_t *)d_src;  // checked non-negative above
-    GB_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb_sort, ukeys, keys_out.as<uint32_t>(),
-                                              ids.as<int32_t>(), perm.as<int32_t>(), (int)E, 0,
-                                              bits, st));
-    GB_HIP(hipcub::DeviceScan::InclusiveSum(nullptr, tb_scan, deg.as<int32_t>(), d_row_ptr,
-                                            V + 1, st));
-    GB_TRY(tmp.ensure(std::max(tb_sort, tb_scan) + 16));
-    GB_HIP(hipcub::DeviceRadixSort::SortPairs(tmp.p, tb_sort, ukeys, keys_out.as<uint32_t>(),
-                                              ids.as<int32_t>(), perm.as<int32_t>(), (int)E, 0,
-                                              bits, st));
-    GB_HIP(hipcub::DeviceScan::InclusiveSum(tmp.p, tb_scan, deg.as<int32_t>(), d_row_ptr, V + 1,
-                                            st));
-    if (w_bytes == 8)
-      hipLaunchKernelGGL(gather_cols_kernel<8>, dim3(grid_for(E)), dim3(256), 0, st, E,
-                         perm.as<int32_t>(), d_dst, d_w, d_col, d_w_out);
-    else if (w_bytes == 4)
-      hipLaunchKernelGGL(gather_cols_kernel<4>, dim3(grid_for(E)), dim3(256), 0, st, E,
-                         perm.as<int32_t>(), d_dst, d_w, d_col, d_w_out);
-    else
-      hipLaunchKernelGGL(gather_cols_kernel<0>, dim3(grid_for(E)), dim3(256), 0, st, E,
-                         perm.as<int32_t>(), d_dst, d_w, d_col, d_w_out);
-    GB_HIP(hipGetLastError());
-  } else {
-    GB_HIP(hipMemsetAsync(d_row_ptr, 0, sizeof(int32_t) * ((size_t)V + 1), st));
-  }
-  GB_HIP(hipStreamSynchronize(st));  // scratch buffers are freed on return
-  return GB_OK;
+  CsrHold hold(csr_work());
+  CsrWork &k = hold.k;
+  return csr_build_any(k, V, E, d_src, d_dst, d_w, w_bytes, d_row_ptr, d_col, d_w_out,
+                       gb_stream(stream));
 }
 
 extern "C" gb_status gb_csr_transpose(int32_t V, int64_t E, const int32_t *d_row_ptr,
@@ -226,17 +673,21 @@ extern "C" gb_status gb_csr_transpose(int32_t V, int64_t E, const int32_t *d_row
                                       void *stream) {
   if (V < 0 || E < 0 || !d_row_ptr || !d_trow_ptr || (E > 0 && (!d_col || !d_tcol)))
     return gb_fail(GB_ERR_INVALID, "gb_csr_transpose: bad arguments");
+  if (E >= ((int64_t)1 << 31) || (w_bytes != 0 && w_bytes != 4 && w_bytes != 8) ||
+      (w_bytes && E > 0 && (!d_w || !d_tw)))
+    return gb_fail(GB_ERR_INVALID, "gb_csr_transpose: bad arguments");
   hipStream_t st = gb_stream(stream);
-  DevBuf rows;
-  GB_TRY(rows.ensure(sizeof(int32_t) * ((size_t)E + 1)));
+  CsrHold hold(csr_work());
+  CsrWork &k = hold.k;
+  GB_TRY(k.rows.ensure(sizeof(int32_t) * ((size_t)E + 1)));
   if (E > 0 && V > 0) {
-    hipLaunchKernelGGL(expand_rows_kernel, dim3(grid_for((int64_t)V * 64)), dim3(256), 0, st, V,
-                       d_row_ptr, rows.as<int32_t>());
-    GB_HIP(hipGetLastError());
+    hipLaunchKernelGGL(expand_rows_kernel, dim3((unsigned)((E + EX_TILE - 1) / EX_TILE)),
+                       dim3(RS_BLOCK), 0, st, V, E, d_row_ptr, k.rows.as<int32_t>());
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return gb_fail(GB_ERR_HIP, "expand_rows: %s", hipGetErrorString(e));
   }
   // transposed rows are keyed by the column; edges of a transposed row keep
   // the order of their source rows
-  GB_TRY(gb_csr_from_edges(V, E, d_col, rows.as<int32_t>(), d_w, w_bytes, d_trow_ptr, d_tcol,
-                           d_tw, stream));
-  return GB_OK;
+  return csr_build_any(k, V, E, d_col, k.rows.as<int32_t>(), d_w, w_bytes, d_trow_ptr, d_tcol,
+                       d_tw, st);
 }

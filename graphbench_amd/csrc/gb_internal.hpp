@@ -194,5 +194,7 @@ void gb_bc_release();
 void gb_msbc_release();
 void gb_mlp_release();
 void gb_learned_release();
+// Gives back the scratch kept for CSR builds unless one is running.
+bool gb_csr_trim();
 
 #endif

@@ -37,6 +37,12 @@ hipStream_t gb_stream(void *s) { return (hipStream_t)s; }
 int gb_num_cus() { return g_cus; }
 
 gb_status gb_dmalloc(void **p, size_t bytes) {
+  auto over = [&]() {
+    std::lock_guard<std::mutex> lk(g_mem_mu);
+    return g_mem_cap && g_mem_used + bytes > g_mem_cap;
+  };
+  // scratch kept for later CSR builds makes room first
+  if (over()) (void)gb_csr_trim();
   {
     std::lock_guard<std::mutex> lk(g_mem_mu);
     if (g_mem_cap && g_mem_used + bytes > g_mem_cap)
@@ -45,6 +51,10 @@ gb_status gb_dmalloc(void **p, size_t bytes) {
   }
   void *raw = nullptr;
   hipError_t e = hipMalloc(&raw, bytes);
+  if (e != hipSuccess && gb_csr_trim()) {
+    (void)hipGetLastError();
+    e = hipMalloc(&raw, bytes);
+  }
   if (e != hipSuccess) {
     (void)hipGetLastError();
     return gb_fail(GB_ERR_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
@@ -101,6 +111,7 @@ void gb_release_workspaces(void) {
   gb_msbc_release();
   gb_mlp_release();
   gb_learned_release();
+  (void)gb_csr_trim();
   split_release();
 }
 
