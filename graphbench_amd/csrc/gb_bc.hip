@@ -26,6 +26,7 @@
 
 #include "gb_device.hpp"
 #include "gb_internal.hpp"
+#include "gb_sssp_small.hpp"
 
 namespace {
 
@@ -201,10 +202,176 @@ __global__ void bc_accum_kernel(int32_t V, int32_t nslots, const int32_t *__rest
   bc[v] = acc;
 }
 
+// ---- a source's whole solve in one workgroup -------------------------------
+// Graphs whose FP64 distances fit the LDS of a CU (gb_sssp_small.hpp): one
+// workgroup per source finds the distances, the tight in-degree counts, the
+// DAG depths with the path counts, and the dependencies, with block barriers
+// between the levels.  The engine's form below launches three kernels and
+// waits for the host twice per level, after thousands of launches for the
+// distances: R-MAT 13 with 16 sources 22.5 ms, now 0.6 ms; 16384 vertices with
+// 196 K edges and 32 sources 28 ms, now 1.3 ms.  The steps and the operand
+// order of the dependencies are the kernels' above; sigma is added
+// instead of pulled (exact in any order below 2^53), a dependency is summed by
+// 8 lanes, or by a wave from BCS_HUB out-edges on, in a fixed order.
+constexpr int BCS_G = 8;        // lanes per vertex in the backward pass
+constexpr int BCS_HUB = 128;
+constexpr int BCS_SOURCES = 256;  // sources per launch, passed by value
+struct BcsSources {
+  int32_t s[BCS_SOURCES];
+};
+// what a workgroup reports: reached vertices, ordered vertices, levels
+struct BcsOut {
+  uint32_t reached, ordered, depth, pad;
+};
+struct BcsCtx {
+  double *sigma, *delta;  // [slot][V]
+  int32_t *indeg;         // [slot][V]
+  uint32_t *order;        // [slot][V] vertices by depth
+  uint32_t *loff;         // [slot][V + 1] first entry of each level
+  BcsOut *out;
+};
+
+template <int VCAP>
+__global__ __launch_bounds__(SM_BLOCK) void bcw_small_kernel(SmGraph<double> G, BcsSources src,
+                                                             double width, BcsCtx c) {
+  __shared__ SmLds<SmF64, VCAP> s;
+  __shared__ uint32_t s_n;
+  const int tid = threadIdx.x, lane = gb_lane(), wv = tid >> 6;
+  const int64_t base = (int64_t)blockIdx.x * G.V;
+  double *sigma = c.sigma + base, *delta = c.delta + base;
+  int32_t *indeg = c.indeg + base;
+  uint32_t *order = c.order + base, *loff = c.loff + (int64_t)blockIdx.x * (G.V + 1);
+  const int32_t s0 = src.s[blockIdx.x];
+  SmStats st;
+  uint32_t sweep = 0;
+  sm_solve(s, G, s0, width, sweep, st);
+  // s.dist is only read from here on
+  for (int v = tid; v < G.V; v += SM_BLOCK) {
+    sigma[v] = 0.0;
+    delta[v] = 0.0;
+    indeg[v] = 0;
+  }
+  if (tid == 0) s_n = 0;
+  __syncthreads();
+  // the reached vertices, in any order, and their tight in-degrees
+  for (int v0 = tid & ~63; v0 < G.V; v0 += SM_BLOCK) {
+    const int v = v0 + lane;
+    const bool on = v < G.V && s.dist[v] != SmF64::inf_bits();
+    const uint64_t m = __ballot(on);
+    uint32_t b = 0;
+    if (lane == 0 && m) b = atomicAdd(&s_n, (uint32_t)__popcll(m));
+    b = __shfl(b, 0, GB_WAVE);
+    if (on) order[b + (uint32_t)__popcll(m & ((1ull << lane) - 1))] = (uint32_t)v;
+  }
+  __syncthreads();
+  const uint32_t reached = s_n;
+  auto tight = [&](uint32_t u, uint32_t x, double w) {
+    return SmF64::bits(__dadd_rn(SmF64::val(s.dist[u]), w)) == s.dist[x];
+  };
+  sm_expand(
+      s, G, reached, sweep, [&](uint32_t i) { return order[i]; },
+      [&](auto &in, auto &u, auto &x, auto &w) {
+        constexpr int U = sizeof(in) / sizeof(in[0]);
+#pragma unroll
+        for (int k = 0; k < U; k++)
+          if (in[k] && tight(u[k], x[k], w[k]))
+            __hip_atomic_fetch_add(&indeg[x[k]], 1, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+      });
+  if (tid == 0) {
+    order[0] = (uint32_t)s0;
+    sigma[s0] = 1.0;
+    loff[0] = 0;
+    loff[1] = 1;
+    s_n = 1;
+  }
+  __syncthreads();
+  // Kahn's order: the last tight in-edge of a vertex appends it to the next level
+  uint32_t lo = 0, hi = 1, depth = 1;
+  for (;;) {
+    sm_expand(
+        s, G, hi - lo, sweep, [&](uint32_t i) { return order[lo + i]; },
+        [&](auto &in, auto &u, auto &x, auto &w) {
+          constexpr int U = sizeof(in) / sizeof(in[0]);
+          double su[U];
+          int32_t left[U];
+#pragma unroll
+          for (int k = 0; k < U; k++) su[k] = sigma[u[k]];
+#pragma unroll
+          for (int k = 0; k < U; k++) {
+            left[k] = 0;
+            if (in[k] && x[k] != (uint32_t)s0 && tight(u[k], x[k], w[k])) {
+              __hip_atomic_fetch_add(&sigma[x[k]], su[k], __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_WORKGROUP);
+              left[k] = __hip_atomic_fetch_add(&indeg[x[k]], -1, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+          }
+#pragma unroll
+          for (int k = 0; k < U; k++)
+            if (left[k] == 1) order[atomicAdd(&s_n, 1u)] = x[k];
+        });
+    lo = hi;
+    hi = s_n;
+    __syncthreads();  // s_n is read before the next level appends
+    if (hi == lo) break;
+    depth++;
+    if (tid == 0) loff[depth] = hi;
+  }
+  if (tid == 0) c.out[blockIdx.x] = BcsOut{reached, hi, depth, 0};
+  if (hi != reached) return;  // a cycle of tight edges: the caller refuses
+  // dependencies, deepest level first
+  const int sub = lane / BCS_G, sl = lane % BCS_G;
+  constexpr int PER = GB_WAVE / BCS_G;
+  for (int32_t d = (int32_t)depth - 1; d >= 0; d--) {
+    const uint32_t l0 = loff[d], l1 = loff[d + 1];
+    for (uint32_t i0 = l0 + wv * PER; i0 < l1; i0 += SM_WAVES * PER) {
+      const bool on = i0 + sub < l1;
+      const uint32_t v = on ? order[i0 + sub] : 0u;
+      const int32_t beg = on ? G.rp[v] : 0, end = on ? G.rp[v + 1] : 0;
+      const double sv = on ? sigma[v] : 0.0;
+      const bool hub = end - beg >= BCS_HUB;
+      auto sum = [&](uint32_t vv, double svv, int32_t e0, int32_t e1, int step) {
+        double acc = 0.0;
+        for (int32_t e = e0; e < e1; e += 4 * step) {
+          int32_t x[4];
+          double w[4];
+#pragma unroll
+          for (int k = 0; k < 4; k++) {
+            const int32_t ee = min(e + k * step, e1 - 1);
+            x[k] = G.col[ee];
+            w[k] = G.w[ee];
+          }
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+            if (e + k * step < e1 && tight(vv, (uint32_t)x[k], w[k]))
+              acc += __ddiv_rn(__dmul_rn(__dadd_rn(1.0, delta[x[k]]), svv), sigma[x[k]]);
+        }
+        return acc;
+      };
+      double acc = hub ? 0.0 : sum(v, sv, beg + sl, end, BCS_G);
+#pragma unroll
+      for (int k = BCS_G / 2; k >= 1; k >>= 1) acc += __shfl_xor(acc, k, GB_WAVE);
+      if (on && !hub && sl == 0) delta[v] = acc;
+      uint64_t hubs = __ballot(hub && sl == 0);
+      while (hubs) {
+        const int l = __ffsll((unsigned long long)hubs) - 1;
+        hubs &= hubs - 1;
+        const uint32_t hv = __shfl(v, l, GB_WAVE);
+        const double a = gb_wave_sum_f64(sum(hv, __shfl(sv, l, GB_WAVE),
+                                             __shfl(beg, l, GB_WAVE) + lane,
+                                             __shfl(end, l, GB_WAVE), GB_WAVE));
+        if (lane == 0) delta[hv] = a;
+      }
+    }
+    __syncthreads();
+  }
+}
+
 struct BcWork {
-  DevBuf level, sigma, delta, order, src, cnt, indeg, dist;
+  DevBuf level, sigma, delta, order, src, cnt, indeg, dist, loff;
   void release() {
-    for (DevBuf *b : {&level, &sigma, &delta, &order, &src, &cnt, &indeg, &dist}) b->release();
+    for (DevBuf *b : {&level, &sigma, &delta, &order, &src, &cnt, &indeg, &dist, &loff}) b->release();
   }
 };
 // Heap singleton, never destroyed: device memory must not be freed from a
@@ -227,6 +394,13 @@ int fill_grid(int64_t n) {
   int64_t cap = (int64_t)gb_num_cus() * 32;
   if (b > cap) b = cap;
   return b < 1 ? 1 : (int)b;
+}
+
+gb_status bcw_refuse(uint64_t n) {
+  return gb_fail(GB_ERR_INVALID,
+                 "gb_bc_weighted: %llu reached vertices lie on a cycle of tight edges "
+                 "(weights must be positive and not vanish against the distances)",
+                 (unsigned long long)n);
 }
 
 // Forward levels for nslots sources; returns level offsets (size depth+2).
@@ -265,6 +439,46 @@ gb_status forward_levels(gb_graph g, int32_t nslots, hipStream_t st,
   return GB_OK;
 }
 
+// Where the workgroup form serves: distances in LDS, and edges that one CU
+// reads in less time than the engine's launches take.
+constexpr int32_t BCS_MAX_V = 16384;
+constexpr int64_t BCS_MAX_E = (int64_t)1 << 20;
+
+// The dependencies of one batch, w.delta[slot][V], by one workgroup per source.
+gb_status bcs_batch(gb_graph g, const int32_t *h_sources, int32_t ns, int32_t *max_depth,
+                    hipStream_t st) {
+  static BcsOut *res = nullptr;  // pinned, kept for the process's life
+  if (!res)
+    GB_HIP(hipHostMalloc((void **)&res, sizeof(BcsOut) * BCS_SOURCES, hipHostMallocDefault));
+  BcWork &w = g_bcw;
+  const int32_t V = g->V;
+  const double width = g->split64_valid ? g->split64_delta : 0.1;
+  GB_TRY(w.loff.ensure(sizeof(uint32_t) * (size_t)BCS_SOURCES * (V + 1)));
+  for (int32_t g0 = 0; g0 < ns; g0 += BCS_SOURCES) {
+    const int n = std::min<int32_t>(BCS_SOURCES, ns - g0);
+    BcsSources src{};
+    for (int i = 0; i < n; i++) src.s[i] = h_sources[g0 + i];
+    const int64_t o = (int64_t)g0 * V;
+    const BcsCtx c{w.sigma.as<double>() + o,  w.delta.as<double>() + o,
+                   w.indeg.as<int32_t>() + o, w.order.as<uint32_t>() + o,
+                   w.loff.as<uint32_t>(),     res};
+    const SmGraph<double> G{g->rp, g->col, g->w64, V};
+    if (V <= BCS_MAX_V / 4)
+      hipLaunchKernelGGL(bcw_small_kernel<BCS_MAX_V / 4>, dim3(n), dim3(SM_BLOCK), 0, st, G, src,
+                         width, c);
+    else
+      hipLaunchKernelGGL(bcw_small_kernel<BCS_MAX_V>, dim3(n), dim3(SM_BLOCK), 0, st, G, src,
+                         width, c);
+    GB_HIP(hipGetLastError());
+    GB_HIP(hipStreamSynchronize(st));
+    for (int i = 0; i < n; i++) {
+      if (res[i].reached != res[i].ordered) return bcw_refuse(res[i].reached - res[i].ordered);
+      *max_depth = std::max(*max_depth, (int32_t)res[i].depth);
+    }
+  }
+  return GB_OK;
+}
+
 gb_status bc_run(gb_graph g, const int32_t *h_sources, int32_t nsrc, int32_t batch, double *d_bc,
                  gb_bc_stats *stats, void *stream) {
   if (!g || (!h_sources && nsrc > 0) || nsrc < 0 || !d_bc)
@@ -294,11 +508,20 @@ gb_status bc_run(gb_graph g, const int32_t *h_sources, int32_t nsrc, int32_t bat
   GB_HIP(hipEventRecord(e0, st));
   GB_HIP(hipMemsetAsync(d_bc, 0, sizeof(double) * V, st));
   int32_t max_depth = 0, batches = 0;
+  const bool small = V <= BCS_MAX_V && g->E <= BCS_MAX_E && gb_sssp_small_enabled();
   std::vector<uint64_t> off;
   for (int32_t b0 = 0; b0 < nsrc; b0 += batch) {
     const int32_t ns = std::min(batch, nsrc - b0);
     const int64_t nn = (int64_t)ns * V;
     GB_HIP(hipMemcpyAsync(w.src.p, h_sources + b0, sizeof(int32_t) * ns, hipMemcpyHostToDevice, st));
+    if (small) {
+      GB_TRY(bcs_batch(g, h_sources + b0, ns, &max_depth, st));
+      hipLaunchKernelGGL(bc_accum_kernel, dim3((V + 255) / 256), dim3(256), 0, st, V, ns,
+                         w.src.as<int32_t>(), w.delta.as<double>(), d_bc);
+      GB_HIP(hipGetLastError());
+      batches++;
+      continue;
+    }
     // exact distances of the batch, then tight in-degree counts; bucket
     // width: the last f64 split of this graph, else the reference's BC
     // constant (run_sspath(gs, pred, source, 0.1), csr_bc.c:43)
@@ -330,11 +553,7 @@ gb_status bc_run(gb_graph g, const int32_t *h_sources, int32_t nsrc, int32_t bat
       unsigned long long reached = 0;
       GB_HIP(hipMemcpyAsync(&reached, rc, sizeof(reached), hipMemcpyDeviceToHost, st));
       GB_HIP(hipStreamSynchronize(st));
-      if (reached != off.back())
-        return gb_fail(GB_ERR_INVALID,
-                       "gb_bc_weighted: %llu reached vertices lie on a cycle of tight edges "
-                       "(weights must be positive and not vanish against the distances)",
-                       (unsigned long long)(reached - off.back()));
+      if (reached != off.back()) return bcw_refuse(reached - off.back());
     }
     const int32_t depth = (int32_t)off.size() - 2;  // number of non-empty levels
     max_depth = std::max(max_depth, depth);

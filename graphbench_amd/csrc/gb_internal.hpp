@@ -185,6 +185,9 @@ gb_status gb_msssp_run(gb_graph g, uint32_t delta, const int32_t *h_sources, int
                        int64_t *expanded, bool *ovf, hipStream_t st);
 gb_status gb_msssp_count(gb_graph g, int32_t nsrc, const uint32_t *d_dist, int64_t *reached,
                          int64_t *traversed, hipStream_t st);
+// Whether solves in one workgroup per source (gb_sssp_small.hpp) are allowed by
+// the environment.
+bool gb_sssp_small_enabled();
 // Adds the per-wave statistics slots (nwaves * GB_WSTAT, gb_device.hpp) to
 // the counters: cnt[idx[k]] += sum over waves of slot k (k < 4; idx3 < 0
 // leaves slot 3 out).

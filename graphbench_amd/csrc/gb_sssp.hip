@@ -31,6 +31,7 @@
 #include "gb_device.hpp"
 #include "gb_internal.hpp"
 #include "gb_sssp_ctl.hpp"
+#include "gb_sssp_small.hpp"
 
 namespace {
 
@@ -725,6 +726,108 @@ gb_status sssp_engine(const std::vector<SGraph<typename Tr::W>> &hg,
   return status;
 }
 
+// ---- graphs whose distances fit one workgroup's LDS ------------------------
+// One workgroup per source (gb_sssp_small.hpp); a launch takes up to
+// SM_SOURCES sources by value, so nothing is uploaded, and each workgroup
+// leaves its counters in pinned host memory, so nothing is copied back.
+constexpr int SM_SOURCES = 256;
+struct SmSources {
+  int32_t s[SM_SOURCES];
+};
+
+template <class Tr, int VCAP>
+__global__ __launch_bounds__(SM_BLOCK) void sssp_small_kernel(SmGraph<typename Tr::W> G,
+                                                              SmSources src, typename Tr::T width,
+                                                              typename Tr::D *dist,
+                                                              SmStats *out) {
+  __shared__ SmLds<Tr, VCAP> s;
+  SmStats st;
+  uint32_t sweep = 0;
+  sm_solve(s, G, src.s[blockIdx.x], width, sweep, st);
+  typename Tr::D *row = dist + (int64_t)blockIdx.x * G.V;
+  for (int v = threadIdx.x; v < G.V; v += SM_BLOCK) row[v] = Tr::val(s.dist[v]);
+  if (threadIdx.x == 0) out[blockIdx.x] = st;
+}
+
+// One CU relaxes about one edge per ns, whatever the chip could do beside it,
+// so the form serves graphs of up to 2^18 edges, and up to 2^20 when enough
+// sources keep many CUs busy.  Measured against the engines (us, plain width /
+// width 128): R-MAT 12, 65 K edges, one source 193 against 1433 / 171 against
+// 737; 16384 vertices, 262 K edges 474 against 1669 / 462 against 758; 32768
+// vertices, 1 M edges, one source 1329 against 2309 / 1655 against 812 (the
+// engine), 64 sources 1939 against 13363 / 2450 against 2813.
+constexpr int64_t SM_MAX_E = (int64_t)1 << 18, SM_MAX_E_MANY = (int64_t)1 << 20;
+constexpr int32_t SM_MANY = 32;
+template <class Tr>
+bool sm_fits(int32_t V, int64_t E, int32_t nsrc) {
+  const int32_t max_v = sizeof(typename Tr::D) == 4 ? 32768 : 16384;
+  return nsrc > 0 && V <= max_v && E <= (nsrc >= SM_MANY ? SM_MAX_E_MANY : SM_MAX_E) &&
+         gb_sssp_small_enabled();
+}
+
+template <class Tr, int VCAP>
+void sm_launch(int n, const SmGraph<typename Tr::W> &G, const SmSources &src, typename Tr::T width,
+               typename Tr::D *dist, SmStats *out, hipStream_t st) {
+  hipLaunchKernelGGL((sssp_small_kernel<Tr, VCAP>), dim3(n), dim3(SM_BLOCK), 0, st, G, src, width,
+                     dist, out);
+}
+
+// Solves all sources; *ovf set when some sum overflowed (the distances are
+// then not to be used: the caller repeats the solve with an engine, whose
+// narrower buckets decide whether the call fails).
+template <class Tr>
+gb_status sm_run(const SmGraph<typename Tr::W> &G, typename Tr::T width, const int32_t *h_sources,
+                 int32_t nsrc, typename Tr::D *d_dist, gb_sssp_stats *stats, bool *ovf,
+                 hipStream_t st) {
+  static SmStats *res = nullptr;  // pinned, kept for the process's life
+  if (!res)
+    GB_HIP(hipHostMalloc((void **)&res, sizeof(SmStats) * SM_SOURCES, hipHostMallocDefault));
+  gb_sssp_stats tot{};
+  *ovf = false;
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  if (stats) {
+    GB_HIP(hipEventCreate(&e0));
+    GB_HIP(hipEventCreate(&e1));
+    GB_HIP(hipEventRecord(e0, st));
+  }
+  hipError_t err = hipSuccess;
+  for (int32_t g0 = 0; g0 < nsrc && err == hipSuccess; g0 += SM_SOURCES) {
+    const int n = std::min<int32_t>(SM_SOURCES, nsrc - g0);
+    SmSources src{};
+    for (int i = 0; i < n; i++) src.s[i] = h_sources[g0 + i];
+    typename Tr::D *rows = d_dist + (int64_t)g0 * G.V;
+    constexpr int BIG = sizeof(typename Tr::D) == 4 ? 32768 : 16384;
+    if (G.V <= BIG / 4)
+      sm_launch<Tr, BIG / 4>(n, G, src, width, rows, res, st);
+    else
+      sm_launch<Tr, BIG>(n, G, src, width, rows, res, st);
+    err = hipGetLastError();
+    if (stats && g0 + n >= nsrc) (void)hipEventRecord(e1, st);
+    if (err == hipSuccess) err = hipStreamSynchronize(st);
+    for (int i = 0; i < n && err == hipSuccess; i++) {
+      tot.buckets = std::max(tot.buckets, (int64_t)res[i].buckets);
+      tot.phases = std::max(tot.phases, (int64_t)res[i].phases);
+      tot.relax_edges += (int64_t)res[i].relax;
+      tot.improved_near += (int64_t)res[i].imp_near;
+      tot.improved_far += (int64_t)res[i].imp_far;
+      tot.reached += (int64_t)res[i].reached;
+      tot.traversed += (int64_t)res[i].traversed;
+      if (res[i].ovf) *ovf = true;
+    }
+  }
+  if (stats) {
+    float ms = 0.0f;
+    if (err == hipSuccess) (void)hipEventElapsedTime(&ms, e0, e1);
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    tot.ms = ms;
+    tot.expanded_edges = tot.relax_edges;  // one source per expansion
+    *stats = tot;
+  }
+  if (err != hipSuccess) return gb_fail(GB_ERR_HIP, "sssp: %s", hipGetErrorString(err));
+  return GB_OK;
+}
+
 // Queue entries carry a 16-bit chunk index: a vertex may have at most
 // 65535 chunks of CHUNK edges.
 gb_status check_degree(gb_graph g, hipStream_t st) {
@@ -771,6 +874,17 @@ gb_status light_rows(gb_graph g, uint32_t lm, hipStream_t st, SGraph<uint32_t> &
 
 }  // namespace
 
+// The workgroup form serves a call unless the environment asks for one of the
+// engines (GB_SSSP_PER_SOURCE, a fixed GB_MSSSP_ shape) or GB_SSSP_SMALL=0.
+bool gb_sssp_small_enabled() {
+  for (const char *k : {"GB_SSSP_PER_SOURCE", "GB_MSSSP_SCAN", "GB_MSSSP_GRID", "GB_MSSSP_CHUNK"}) {
+    const char *e = getenv(k);
+    if (e && e[0]) return false;
+  }
+  const char *e = getenv("GB_SSSP_SMALL");
+  return !(e && e[0] == '0');
+}
+
 void gb_sssp_release() { g_ssw.release(); }
 
 extern "C" gb_status gb_sssp(gb_graph g, const gb_sssp_params *p, const int32_t *h_sources,
@@ -789,6 +903,12 @@ extern "C" gb_status gb_sssp(gb_graph g, const gb_sssp_params *p, const int32_t 
     delta = plain_delta(mw, g->V, g->E);
   }
   if (lmax == 0) lmax = delta;
+  if (!(p && p->max_phases > 0) && sm_fits<SmU32>(g->V, g->E, nsrc)) {
+    bool ovf = false;
+    GB_TRY(sm_run<SmU32>(SmGraph<uint32_t>{g->rp, g->col, g->w, g->V}, delta, h_sources, nsrc,
+                         d_dist, stats, &ovf, st));
+    if (!ovf) return GB_OK;
+  }
   if (nsrc >= 2 && ms_enabled()) {
     // several sources: the batched engine (one entry per vertex and source mask)
     gb_sssp_stats s{};
@@ -837,6 +957,11 @@ extern "C" gb_status gb_sssp_f64(gb_graph g, double delta, const int32_t *h_sour
     if (h_sources[i] < 0 || h_sources[i] >= g->V)
       return gb_fail(GB_ERR_INVALID, "gb_sssp_f64: source %d out of range", h_sources[i]);
   hipStream_t st = gb_stream(stream);
+  if (sm_fits<SmF64>(g->V, g->E, nsrc)) {
+    bool ovf = false;
+    return sm_run<SmF64>(SmGraph<double>{g->rp, g->col, g->w64, g->V}, delta, h_sources, nsrc,
+                         d_dist, stats, &ovf, st);
+  }
   GB_TRY(check_degree(g, st));
   GB_TRY(gb_graph_split64(g, delta, st));
   std::vector<SGraph<double>> hg(1);
