@@ -195,6 +195,12 @@ gb_status gb_wstat_fold(int64_t nwaves, const unsigned long long *slots, unsigne
                         int idx0, int idx1, int idx2, hipStream_t st, int idx3 = -1);
 void gb_bc_release();
 void gb_msbc_release();
+// Unweighted Brandes with one workgroup per source (gb_bc_small.hip): adds the
+// dependencies to d_bc, *depth the most levels of a source.
+bool gb_bc_small_fits(gb_graph g);
+gb_status gb_bc_small_run(gb_graph g, const int32_t *h_sources, int32_t nsrc, double *d_bc,
+                          int32_t *depth, hipStream_t st);
+void gb_bc_small_release();
 void gb_mlp_release();
 void gb_learned_release();
 // Gives back the scratch kept for CSR builds unless one is running.

@@ -1141,6 +1141,12 @@ extern "C" gb_status gb_bc(gb_graph g, const int32_t *h_sources, int32_t nsrc, i
   for (int32_t b0 = 0; b0 < nsrc && V > 0; b0 += (int32_t)per) {
     const int32_t ns = (int32_t)std::min<int64_t>(per, nsrc - b0);
     int32_t depth = 0;
+    if (gb_bc_small_fits(g)) {
+      GB_TRY(gb_bc_small_run(g, h_sources + b0, ns, d_bc, &depth, st));
+      max_depth = std::max(max_depth, depth - 1);
+      batches++;
+      continue;
+    }
     GB_TRY(bc_tune(g, h_sources + b0, ns, st));
     GB_TRY(ms_run(g, h_sources + b0, ns, true, d_bc, nullptr, st, &depth,
                   bc_shape(g, (ns + 63) / 64, nullptr)));

@@ -109,6 +109,7 @@ void gb_release_workspaces(void) {
   gb_msssp_release();
   gb_bc_release();
   gb_msbc_release();
+  gb_bc_small_release();
   gb_mlp_release();
   gb_learned_release();
   (void)gb_csr_trim();

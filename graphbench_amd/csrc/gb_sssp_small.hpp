@@ -22,6 +22,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "gb_device.hpp"
 
 constexpr int SM_BLOCK = 1024;
@@ -78,6 +80,7 @@ struct SmF64 {
   static __device__ __forceinline__ T widen(T width) { return width * 2.0; }
 };
 
+// W void: no weights
 template <class W>
 struct SmGraph {
   const int32_t *rp;
@@ -85,22 +88,27 @@ struct SmGraph {
   const W *w;
   int32_t V;
 };
+template <class W>
+using sm_weight = std::conditional_t<std::is_void<W>::value, uint32_t, W>;
 
 struct SmStats {
   unsigned long long buckets, phases, relax, imp_near, imp_far, reached, traversed, ovf;
 };
 
-// LDS of one workgroup; VCAP a multiple of 2048.
-template <class Tr, int VCAP>
-struct SmLds {
-  typename Tr::Bits dist[VCAP];
-  uint32_t pend[VCAP / 32];
-  uint16_t queue[SM_QCAP];
+// LDS of the edge spreading
+struct SmShare {
   // of a batch's vertices with edges: edge index minus edge slot, vertex
   uint2 own[SM_BLOCK];
   unsigned long long start[3][SM_SWEEP / 64];  // slots where a vertex's edges begin
   uint32_t wsum[SM_WAVES], wcnt[SM_WAVES];
-  uint32_t n, lim, total, edges;
+};
+// LDS of one workgroup; VCAP a multiple of 2048.
+template <class Tr, int VCAP>
+struct SmLds : SmShare {
+  typename Tr::Bits dist[VCAP];
+  uint32_t pend[VCAP / 32];
+  uint16_t queue[SM_QCAP];
+  uint32_t n, lim, edges;
   unsigned long long lo;  // bits of the smallest waiting distance
   unsigned long long acc[6];
 };
@@ -111,14 +119,13 @@ struct SmLds {
 // bits; pre: the start bits before that word plus those of earlier sweeps.
 // The owner of slot k is the last start at or before k: the wave's 64
 // consecutive slots are one word, held by one lane.
-template <int U, class Tr, int VCAP, class F>
-__device__ __forceinline__ void sm_edges(const SmLds<Tr, VCAP> &s,
-                                         const SmGraph<typename Tr::W> &G, uint32_t k0,
+template <int U, class W, class F>
+__device__ __forceinline__ void sm_edges(const SmShare &s, const SmGraph<W> &G, uint32_t k0,
                                          uint32_t total, uint64_t bits, uint32_t pre, F f) {
   const int wv = threadIdx.x >> 6;
   const uint64_t upto = ~0ull >> (63 - gb_lane());
   uint32_t v[U], x[U];
-  typename Tr::W w[U];
+  sm_weight<W> w[U];
   bool in[U];
   uint2 o[U];
 #pragma unroll
@@ -135,7 +142,8 @@ __device__ __forceinline__ void sm_edges(const SmLds<Tr, VCAP> &s,
     const int32_t e = (int32_t)k + (int32_t)o[u].x;
     v[u] = o[u].y;
     x[u] = in[u] ? (uint32_t)G.col[e] : 0u;
-    w[u] = in[u] ? G.w[e] : (typename Tr::W)0;
+    w[u] = 0;
+    if constexpr (!std::is_void<W>::value) w[u] = in[u] ? G.w[e] : (W)0;
   }
   f(in, v, x, w);
 }
@@ -147,9 +155,9 @@ __device__ __forceinline__ void sm_edges(const SmLds<Tr, VCAP> &s,
 // Every lane searching the batch's first slots instead (10 LDS reads per edge)
 // measured 3 to 10% slower (32768 vertices, 31 edges each, 32 sources: 1762
 // against 1608 us).
-template <class Tr, int VCAP, class Vert, class F>
-__device__ __forceinline__ void sm_expand(SmLds<Tr, VCAP> &s, const SmGraph<typename Tr::W> &G,
-                                          uint32_t n, uint32_t &sweep, Vert vert, F f) {
+template <class W, class Vert, class F>
+__device__ __forceinline__ void sm_expand(SmShare &s, const SmGraph<W> &G, uint32_t n,
+                                          uint32_t &sweep, Vert vert, F f) {
   const int tid = threadIdx.x, lane = gb_lane(), wv = tid >> 6;
   for (uint32_t b = 0; b < n; b += SM_BLOCK) {
     int32_t beg = 0;

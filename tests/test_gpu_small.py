@@ -115,3 +115,27 @@ def test_bc_weighted(gpu, kind, V, nsrc, batch):
     bc = gb.bc(g, srcs, batch=batch, weighted=True).cpu().numpy()
     ref = oracle.brandes_weighted(h.row_ptr, h.col, w64, r.row_ptr, r.col, rw64, srcs)
     np.testing.assert_allclose(bc, ref, rtol=1e-12, atol=1e-9 * max(1.0, np.abs(ref).max()) * 1e-3)
+
+
+# 4096 / 14336 vertices are the two LDS sizes; past them the batched engine
+@pytest.mark.parametrize("kind,V,nsrc,batch", [("random", 1, 1, 0), ("random", 64, 9, 0),
+                                               ("random", 4096, 70, 64), ("random", 4097, 6, 0),
+                                               ("random", 14336, 3, 0), ("random", 14337, 3, 0),
+                                               ("star", 14000, 2, 0), ("path", 900, 3, 0),
+                                               ("random", 150, 300, 0)])
+def test_bc_unweighted(gpu, kind, V, nsrc, batch):
+    """Directed graphs with parallel edges, self-loops and unreached vertices:
+    hubs past 128 out-edges, levels wider than a batch of the edge spreading,
+    one level per vertex, more sources than a launch."""
+    gb = gpu
+    rng = np.random.default_rng(V + 3)
+    h = _graph(gb, kind, V, rng)
+    h = gb.HostCSR(h.row_ptr, h.col)
+    r = h.transpose()
+    g = gb.Graph.from_host(h, reverse=r)
+    srcs = [int(x) for x in rng.integers(0, V, nsrc)]
+    bc, st = gb.bc(g, srcs, batch=batch, stats=True)
+    ref = oracle.brandes_bfs(h.row_ptr, h.col, srcs, r.row_ptr, r.col)
+    np.testing.assert_allclose(bc.cpu().numpy(), ref, rtol=1e-12, atol=1e-12)
+    depth = max(int(oracle.bfs_levels(h.row_ptr, h.col, s).max()) for s in srcs)
+    assert st["max_depth"] == depth
