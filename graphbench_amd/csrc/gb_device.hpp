@@ -24,6 +24,18 @@ __device__ __forceinline__ uint64_t gb_shfl_u64(uint64_t v, int src) {
   uint32_t hi = __shfl((uint32_t)(v >> 32), src, GB_WAVE);
   return ((uint64_t)hi << 32) | lo;
 }
+// A value that is the same in every lane (read from LDS, say), as the compiler
+// can know it: kept in scalar registers, loops and loads that depend on it stay
+// scalar.
+__device__ __forceinline__ uint32_t gb_uniform(uint32_t v) {
+  return __builtin_amdgcn_readfirstlane(v);
+}
+__device__ __forceinline__ uint64_t gb_uniform(uint64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return ((uint64_t)hi << 32) | lo;
+}
+
 // Reserve `cnt` consecutive slots of a device queue for this lane.  One
 // atomicAdd per wave.  Must be reached by every active lane of the wave.
 __device__ __forceinline__ uint64_t gb_wave_reserve(unsigned long long *counter, uint32_t cnt) {
@@ -150,6 +162,25 @@ __device__ __forceinline__ void gb_wstat_add(unsigned long long *slots, int k, u
   if (v) {
     const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     atomicAdd(&slots[wave * GB_WSTAT + k], (unsigned long long)v);
+  }
+}
+
+// What a phase loop on the device tells the host, in pinned memory: the number
+// of phases begun and, once done, the loop's totals.
+struct GbProgress {
+  uint32_t started, done;
+  int64_t phases, buckets;
+  int32_t capped, pad;
+};
+__device__ __forceinline__ void gb_progress(GbProgress *p, uint32_t k, bool done, int64_t phases,
+                                            int64_t buckets, int32_t capped) {
+  if (done) {
+    __hip_atomic_store(&p->phases, phases, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&p->buckets, buckets, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&p->capped, capped, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&p->done, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  } else {
+    __hip_atomic_store(&p->started, k + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 

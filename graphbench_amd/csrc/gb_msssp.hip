@@ -28,19 +28,19 @@
 // The scan costs a pass over V per phase.  Small graphs with many short
 // phases use the append form instead (SCAN = false): the lane whose atomicOr
 // turns a target's next-phase mask from empty to non-empty (its return value)
-// reads the target's row bounds and appends its chunks at once; the masks
-// are double-buffered (the phase reads its input mask array, which is
-// cleared by queue entry after the phase) and entries carry no mask.
-// All sources step through bucket indices in lockstep: light phases while the
-// near queue is non-empty, then a far scan that moves the next non-empty
-// bucket's (vertex, source) pairs to the near queue.  There is no light/heavy
-// split: an expansion relaxes all edges of the vertex.  Delta-stepping is
-// exact for any bucket width, so distances equal the per-source engine's.
-// The bucket loop is the state machine ms_ctl_advance (gb_sssp_ctl.hpp),
-// replayed from a captured hipGraph as in the per-source engine.  A phase of
-// the scan form is three launches (step, compaction, state advance); of the
-// append form two (the state advance fused with the clear of the previous
-// phase's input masks, then the step).
+// reads the target's row bounds and appends its chunks at once; masks and
+// queues rotate through three buffers (a phase reads one, fills the next and
+// clears the one before by its queue entries) and entries carry no mask.
+// All sources step through ranges of buckets in lockstep (gb_sssp_ctl.hpp):
+// light phases while the near queue is non-empty, then a far scan that moves
+// the next non-empty range's (vertex, source) pairs to the near queue.  There
+// is no light/heavy split: an expansion relaxes all edges of the vertex.
+// Delta-stepping is exact for any bucket widths, so distances equal the
+// per-source engine's.  The loop is the state machine ms_ctl_advance, driven by
+// launches that run ahead of the device (gb_drive_phases).  A phase of the
+// scan form is three launches (step, compaction, state advance), of the append
+// form one.  R-MAT 16 with 8 sources: 1.2 ms in 38 phases, against 3.1 ms in
+// 169 phases of two launches from a hipGraph captured per call.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -102,11 +102,13 @@ struct MsCtx {
   int64_t E;
   int32_t ntask;                   // sources in this group (<= W)
   uint32_t *dist;                  // [V][W]
-  // next-phase masks: scan form mask[0] only (zero between phases), append
-  // form one per near queue
-  unsigned long long *mask[2];
+  // next-phase masks and near queues (chunks).  Scan form: mask[0] (zero
+  // between phases), queues 0/1.  Append form: three of each in turn, phase k
+  // reading k % 3, appending to (k + 1) % 3 and clearing the masks that phase
+  // k - 1 read.
+  unsigned long long *mask[3];
   unsigned long long *far;         // far masks
-  MsEnt *qn[2];                    // near queues 0/1 (chunks)
+  MsEnt *qn[3];
   uint64_t *qf[2];                 // far queues 0/1 (vertices)
   unsigned long long *cnt;         // MS_* counters
   unsigned long long *wstat;       // per-wave statistics slots (GB_WSTAT per wave)
@@ -118,16 +120,11 @@ __device__ __forceinline__ uint64_t ms_bucket(uint32_t d, uint64_t magic) {
   return magic ? __umul64hi((uint64_t)d, magic) : (uint64_t)d;
 }
 
-__global__ void ms_fill_kernel(int64_t n, uint32_t *__restrict__ dist) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    dist[i] = 0xFFFFFFFFu;
-}
-
 // One wave (blockDim 64): lane t seeds source t; the lowest lane holding a
 // vertex writes its chunks with the mask of every lane holding it.
 template <int W, bool SCAN>
-__global__ void ms_seed_kernel(MsCtx c, const int32_t *__restrict__ src) {
+__global__ void ms_seed_kernel(MsCtx c, const int32_t *__restrict__ src,
+                               unsigned long long *__restrict__ n_near) {
   const int t = threadIdx.x;
   const bool on = t < c.ntask;
   const int32_t s = on ? src[t] : -1;
@@ -146,10 +143,22 @@ __global__ void ms_seed_kernel(MsCtx c, const int32_t *__restrict__ src) {
   const int32_t r0 = c.rp[s], r1 = c.rp[s + 1];
   if (lowest && r1 > r0) {
     const uint32_t k = ms_nchunks(r1 - r0, c.cshift);
-    const unsigned long long b = atomicAdd(&c.cnt[MS_NEAR0], (unsigned long long)k);
+    const unsigned long long b = atomicAdd(n_near, (unsigned long long)k);
     for (uint32_t i = 0; i < k; i++) c.qn[0][b + i] = ms_chunk(m, (uint32_t)s, r0, r1, i, c.cshift);
   }
 }
+
+// Where a phase reads and appends.
+struct MsIo {
+  const MsEnt *in;                // light: the near queue
+  const unsigned long long *min_;  // append form: its masks
+  unsigned long long *mout;       // next-phase masks
+  MsEnt *near_out;                // append form
+  const uint64_t *far_in;
+  uint64_t *far_out;
+  uint64_t n;                     // entries of the queue read
+  unsigned long long *n_near, *n_far, *minb;
+};
 
 // What a wave loads for one near entry: the entry's source mask, this lane's
 // source distance at the vertex, and the chunk's edges (lane r holds edge
@@ -177,8 +186,8 @@ __device__ __forceinline__ MsIn ms_load(const MsCtx &c, const unsigned long long
 // pipelined: entry i is expanded while entry i + nwaves's loads and entry
 // i + 2 nwaves's descriptor are in flight.
 template <int W, bool SCAN>
-__device__ __forceinline__ void ms_light(const MsCtx &c, const MsCtl &a, MsEnt *lds_near,
-                                         uint64_t *lds_far, uint32_t &relax, uint32_t &imp_near,
+__device__ __forceinline__ void ms_light(const MsCtx &c, const MsIo &io, uint64_t b, bool all,
+                                         MsEnt *lds_near, uint64_t *lds_far, uint32_t &relax, uint32_t &imp_near,
                                          uint32_t &imp_far, uint32_t &expanded, bool &ovf) {
   using S = MsShape<W>;
   constexpr int ES = S::ES, UNROLL = S::UNROLL, G = S::G;
@@ -187,13 +196,12 @@ __device__ __forceinline__ void ms_light(const MsCtx &c, const MsCtl &a, MsEnt *
   // the lane that issues the mask update of (step lane / ES, slot lane % ES)
   const int kj = lane / ES, ej = lane % ES;
   const uint64_t wmask = W == 64 ? ~0ull : ((1ull << W) - 1);
-  const MsEnt *in = c.qn[a.a_in - MS_NEAR0];
-  const unsigned long long *min_ = c.mask[a.a_in - MS_NEAR0];
-  unsigned long long *mout = SCAN ? c.mask[0] : c.mask[a.a_near - MS_NEAR0];
-  gb_wave_queue<MsEnt, MS_NCAP> nq(lds_near, c.qn[a.a_near - MS_NEAR0], &c.cnt[a.a_near]);
-  gb_wave_queue<uint64_t, MS_FCAP> fq(lds_far, c.qf[a.a_far - MS_FAR0], &c.cnt[a.a_far]);
-  const uint64_t n = c.cnt[a.a_in];
-  const uint64_t b = a.a_bucket;
+  const MsEnt *in = io.in;
+  const unsigned long long *min_ = io.min_;
+  unsigned long long *mout = io.mout;
+  gb_wave_queue<MsEnt, MS_NCAP> nq(lds_near, io.near_out, io.n_near);
+  gb_wave_queue<uint64_t, MS_FCAP> fq(lds_far, io.far_out, io.n_far);
+  const uint64_t n = io.n;
   // wave-uniform indices (readfirstlane): the entries are read with scalar
   // loads and live in scalar registers
   const uint64_t wave = __builtin_amdgcn_readfirstlane(
@@ -257,6 +265,18 @@ __device__ __forceinline__ void ms_light(const MsCtx &c, const MsCtl &a, MsEnt *
 #pragma unroll
       for (int k = 0; k < UNROLL; k++)
         if (ok[k]) atomicMin(&c.dist[(int64_t)x[k] * W + t], nd[k]);
+      // the counters tell the buckets of the caller's width apart, also within
+      // a range of several
+      if (all) {
+        const uint64_t bu = ms_bucket(cur.du, c.magic);
+#pragma unroll
+        for (int k = 0; k < UNROLL; k++) {
+          const uint64_t bk = ms_bucket(nd[k], c.magic);
+          const uint32_t moved = ok[k] & (bk <= b) & (bk > bu);
+          imp_near -= moved;
+          imp_far += moved;
+        }
+      }
       nm = (nm >> (ej * W)) & wmask;
       fm = (fm >> (ej * W)) & wmask;
       const uint32_t xj = (uint32_t)__shfl(cur.x, (g0 + lane) & (GB_WAVE - 1), GB_WAVE);
@@ -303,18 +323,17 @@ __device__ __forceinline__ void ms_light(const MsCtx &c, const MsCtl &a, MsEnt *
 // next-phase masks (queued by the compaction), later buckets stay (far queue
 // a_far), settled ones are dropped.
 template <int W, bool SCAN>
-__device__ __forceinline__ void ms_far(const MsCtx &c, const MsCtl &a, MsEnt *lds_near,
-                                       uint64_t *lds_far) {
+__device__ __forceinline__ void ms_far(const MsCtx &c, const MsIo &io, uint64_t first,
+                                       uint64_t last, MsEnt *lds_near, uint64_t *lds_far) {
   constexpr int ES = GB_WAVE / W;
   const int lane = gb_lane();
   const int es = lane / W, t = lane % W;
   const uint64_t wmask = W == 64 ? ~0ull : ((1ull << W) - 1);
-  const uint64_t *in = c.qf[a.a_in - MS_FAR0];
-  unsigned long long *mout = SCAN ? c.mask[0] : c.mask[a.a_near - MS_NEAR0];
-  gb_wave_queue<MsEnt, MS_NCAP> nq(lds_near, c.qn[a.a_near - MS_NEAR0], &c.cnt[a.a_near]);
-  gb_wave_queue<uint64_t, MS_FCAP> fq(lds_far, c.qf[a.a_far - MS_FAR0], &c.cnt[a.a_far]);
-  const uint64_t n = c.cnt[a.a_in];
-  const uint64_t bnext = a.a_bucket;
+  const uint64_t *in = io.far_in;
+  unsigned long long *mout = io.mout;
+  gb_wave_queue<MsEnt, MS_NCAP> nq(lds_near, io.near_out, io.n_near);
+  gb_wave_queue<uint64_t, MS_FCAP> fq(lds_far, io.far_out, io.n_far);
+  const uint64_t n = io.n;
   const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) >> 6;
   uint64_t minb = ~0ull;
@@ -327,9 +346,9 @@ __device__ __forceinline__ void ms_far(const MsCtx &c, const MsCtl &a, MsEnt *ld
       const unsigned long long m = c.far[x];
       if ((m >> t) & 1ull) {
         const uint64_t bk = ms_bucket(c.dist[(int64_t)x * W + t], c.magic);
-        if (bk == bnext) {
+        if (bk >= first && bk <= last) {
           near = true;
-        } else if (bk > bnext) {
+        } else if (bk > last) {
           keep = true;
           minb = bk < minb ? bk : minb;
         }
@@ -361,16 +380,13 @@ __device__ __forceinline__ void ms_far(const MsCtx &c, const MsCtl &a, MsEnt *ld
     gb_block_flush(fq);
   else
     gb_block_flush(nq, fq);
-  gb_block_atomic_min(minb, ~0ull, &c.cnt[MS_MINB]);
+  gb_block_atomic_min(minb, ~0ull, io.minb);
 }
 
+// The action (ACT_LIGHT or ACT_FAR) of one phase.
 template <int W, bool SCAN>
-__global__ __launch_bounds__(MS_BLOCK)
-__attribute__((amdgpu_waves_per_eu(MsShape<W>::MIN_WAVES))) void ms_step_kernel(MsCtx c,
-                                                           const MsCtl *__restrict__ ctl) {
-  const int act = ctl->action;
-  if (act == ACT_NONE) return;
-  const MsCtl a = *ctl;
+__device__ __forceinline__ void ms_phase(const MsCtx &c, const MsIo &io, int act, uint64_t first,
+                                         uint64_t last, bool all) {
   __shared__ uint64_t s_far[MS_BLOCK / GB_WAVE][MS_FCAP];
   __shared__ MsEnt s_near[MS_BLOCK / GB_WAVE][SCAN ? 1 : MS_NCAP];
   uint64_t *lf = s_far[threadIdx.x / GB_WAVE];
@@ -378,7 +394,7 @@ __attribute__((amdgpu_waves_per_eu(MsShape<W>::MIN_WAVES))) void ms_step_kernel(
   if (act == ACT_LIGHT) {
     uint32_t relax = 0, imp_near = 0, imp_far = 0, expanded = 0;
     bool ovf = false;
-    ms_light<W, SCAN>(c, a, ln, lf, relax, imp_near, imp_far, expanded, ovf);
+    ms_light<W, SCAN>(c, io, last, all, ln, lf, relax, imp_near, imp_far, expanded, ovf);
     uint32_t tot, tn, tf, te;
     (void)gb_wave_excl_sum(relax, &tot);
     (void)gb_wave_excl_sum(imp_near, &tn);
@@ -392,38 +408,149 @@ __attribute__((amdgpu_waves_per_eu(MsShape<W>::MIN_WAVES))) void ms_step_kernel(
     }
     if (__ballot(ovf) && gb_lane() == 0) atomicOr(&c.cnt[MS_OVF], 1ull);
   } else {
-    ms_far<W, SCAN>(c, a, ln, lf);
+    ms_far<W, SCAN>(c, io, first, last, ln, lf);
   }
 }
 
-// The state machine between two phases (one thread).
-__global__ void ms_ctrl_kernel(MsCtx c, MsCtl *__restrict__ ctl) {
+// Scan form: the step; the state machine advances in a launch of its own.
+template <int W>
+__global__ __launch_bounds__(MS_BLOCK)
+__attribute__((amdgpu_waves_per_eu(MsShape<W>::MIN_WAVES))) void ms_step_kernel(MsCtx c,
+                                                           const MsCtl *__restrict__ ctl) {
+  const int act = ctl->action;
+  if (act == ACT_NONE) return;
+  MsIo io{};
+  const int in = ctl->a_in, fr = ctl->a_far - MS_FAR0;
+  if (act == ACT_LIGHT)
+    io.in = c.qn[in - MS_NEAR0];
+  else
+    io.far_in = c.qf[in - MS_FAR0];
+  io.mout = c.mask[0];
+  io.near_out = c.qn[ctl->a_near - MS_NEAR0];
+  io.far_out = c.qf[fr];
+  io.n = c.cnt[in];
+  io.n_near = &c.cnt[ctl->a_near];
+  io.n_far = &c.cnt[ctl->a_far];
+  io.minb = &c.cnt[MS_MINB];
+  ms_phase<W, true>(c, io, act, ctl->a_first, ctl->a_bucket, ctl->a_all != 0);
+}
+
+// Scan form, between two phases: one thread.
+__global__ void ms_ctrl_kernel(MsCtx c, MsCtl *__restrict__ ctl, uint32_t k, GbProgress *prog) {
   MsCtl s = *ctl;
   ms_ctl_advance(s, c.cnt);
   *ctl = s;
+  gb_progress(prog, k, s.done != 0, s.phases, s.buckets, s.capped);
 }
 
-// Append form, between two phases, one launch: thread 0 computes the next
-// action from the previous state `prev` into `next`, and, when the previous
-// action was a light phase, every thread clears that phase's input masks (the
-// buffer is the output of the phase after next).  The two states are
-// distinct buffers, alternating per phase, and the clear takes its entry
-// count from `prev` rather than the counter, which the advance may reset.
-__global__ void ms_clear_ctrl_kernel(MsCtx c, const MsCtl *__restrict__ prev,
-                                     MsCtl *__restrict__ next) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    MsCtl s = *prev;
-    ms_ctl_advance(s, c.cnt);
-    *next = s;
+// Append form: a phase is one launch.  Every block advances the state from
+// what the phase before left and performs the action it finds; block 0 writes
+// the state for the next phase (two buffers in turn).  Appends are counted in
+// one of three MsAdds in turn: the phase before's is read, this phase's is
+// written, the next one's is cleared.  The masks that the phase before read
+// are cleared through its queue, which is not reused until the phase after
+// this one.  With the advance and the clear in a launch of their own a phase
+// had taken another 5 us.
+struct MsAdds {
+  unsigned long long near, far, minb;
+};
+struct MsDev {
+  MsCtl ctl;
+  unsigned long long n[MS_MINB + 1];  // queue lengths, smallest far bucket
+};
+struct MsLoop {
+  MsDev st[2];
+  MsAdds adds[3];
+};
+
+template <int W>
+__global__ __launch_bounds__(MS_BLOCK)
+__attribute__((amdgpu_waves_per_eu(MsShape<W>::MIN_WAVES))) void ms_append_kernel(
+    MsCtx c, MsLoop *__restrict__ L, uint32_t k, GbProgress *prog) {
+  __shared__ MsDev s_dev;
+  __shared__ MsAdds s_add;
+  __shared__ unsigned long long s_clear;
+  constexpr int DW = sizeof(MsDev) / 4, AW = sizeof(MsAdds) / 4;
+  static_assert(DW + AW <= MS_BLOCK && sizeof(MsDev) % 4 == 0, "one load per thread");
+  const int t = threadIdx.x;
+  {
+    const uint32_t *ds = (const uint32_t *)&L->st[(k + 1) & 1];
+    const uint32_t *as = (const uint32_t *)&L->adds[(k + 2) % 3];
+    if (t < DW)
+      ((uint32_t *)&s_dev)[t] = ds[t];
+    else if (t < DW + AW)
+      ((uint32_t *)&s_add)[t - DW] = as[t - DW];
   }
-  if (prev->action != ACT_LIGHT) return;
-  const int in = prev->a_in;
-  const uint64_t n = prev->a_in_n;
-  unsigned long long *m = c.mask[in - MS_NEAR0];
-  const MsEnt *q = c.qn[in - MS_NEAR0];
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * blockDim.x)
-    m[q[i].v] = 0;
+  __syncthreads();
+  if (t == 0) {
+    const int act = s_dev.ctl.action;
+    s_clear = act == ACT_LIGHT && !s_dev.ctl.done ? s_dev.ctl.a_in_n : 0ull;
+    if (!s_dev.ctl.done) {
+      // before phase 0 the seeds went to near queue 0
+      s_dev.n[act == ACT_NONE ? MS_NEAR0 : s_dev.ctl.a_near] += s_add.near;
+      if (act != ACT_NONE) s_dev.n[s_dev.ctl.a_far] += s_add.far;
+      s_dev.n[MS_MINB] = s_add.minb;
+      ms_ctl_advance(s_dev.ctl, s_dev.n);
+    }
+  }
+  __syncthreads();
+  if (blockIdx.x == 0) {
+    if (t < DW) ((uint32_t *)&L->st[k & 1])[t] = ((uint32_t *)&s_dev)[t];
+    if (t == 0) {
+      L->adds[(k + 1) % 3] = MsAdds{0, 0, ~0ull};
+      gb_progress(prog, k, s_dev.ctl.done != 0, s_dev.ctl.phases, s_dev.ctl.buckets,
+                  s_dev.ctl.capped);
+    }
+  }
+  const int act = (int)gb_uniform((uint32_t)s_dev.ctl.action);
+  if (s_dev.ctl.done || act == ACT_NONE) return;
+  const int a_in = (int)gb_uniform((uint32_t)s_dev.ctl.a_in);
+  const int a_far = (int)gb_uniform((uint32_t)s_dev.ctl.a_far);
+  const int rin = k % 3, rout = (k + 1) % 3, rold = (k + 2) % 3;
+  const uint64_t old_n = gb_uniform((uint64_t)s_clear);
+  for (uint64_t i = (uint64_t)blockIdx.x * MS_BLOCK + t; i < old_n;
+       i += (uint64_t)gridDim.x * MS_BLOCK)
+    c.mask[rold][c.qn[rold][i].v] = 0;
+  MsAdds *add = &L->adds[k % 3];
+  MsIo io;
+  io.in = c.qn[rin];
+  io.min_ = c.mask[rin];
+  io.mout = c.mask[rout];
+  io.near_out = c.qn[rout];
+  io.far_in = act == ACT_FAR ? c.qf[a_in - MS_FAR0] : nullptr;
+  // a far scan's output queue starts empty
+  io.far_out = c.qf[a_far - MS_FAR0] + gb_uniform((uint64_t)s_dev.n[a_far]);
+  io.n = gb_uniform((uint64_t)s_dev.n[a_in]);
+  io.n_near = &add->near;
+  io.n_far = &add->far;
+  io.minb = &add->minb;
+  ms_phase<W, false>(c, io, act, gb_uniform(s_dev.ctl.a_first), gb_uniform(s_dev.ctl.a_bucket),
+                     gb_uniform((uint32_t)s_dev.ctl.a_all) != 0);
+}
+
+// Before the seeds: distances infinite, masks, far masks, counters and
+// statistics zero.
+__global__ void ms_begin_kernel(MsCtx c, int W, int nmask, MsLoop *__restrict__ L, MsCtl ctl,
+                                MsCtl *__restrict__ scan_ctl, int64_t nstat) {
+  const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t step = (int64_t)gridDim.x * blockDim.x;
+  const int64_t n4 = (int64_t)c.V * W / 4;  // W is a multiple of 8
+  uint4 *d4 = (uint4 *)c.dist;
+  for (int64_t i = i0; i < n4; i += step)
+    d4[i] = make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu);
+  for (int64_t i = i0; i < c.V; i += step) {
+    c.far[i] = 0;
+    for (int k = 0; k < nmask; k++) c.mask[k][i] = 0;
+  }
+  for (int64_t i = i0; i < nstat; i += step) c.wstat[i] = 0;
+  if (i0 < MS_N) c.cnt[i0] = 0;
+  if (i0 == 0) {
+    MsDev d{};
+    d.ctl = ctl;
+    L->st[1] = d;
+    for (int k = 0; k < 3; k++) L->adds[k] = MsAdds{0, 0, ~0ull};
+    *scan_ctl = ctl;
+  }
 }
 
 // After a phase: every vertex whose next-phase mask is set gets one near-queue
@@ -649,10 +776,21 @@ int ms_compact_grid(int64_t V) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)gb_num_cus() * 16));
 }
 
+// Queue entries per phase of a range below which the next range is wider (by 8
+// below an eighth of it), and above 16 times of which it is half as wide.  The
+// more sources share an expansion, the more a wide range saves: a vertex is
+// expanded fewer times, for more sources at once.  At 2^18 / 2^19 entries:
+// R-MAT 20 with 2 sources 2.8 / 3.7 ms (single buckets 3.7), with 32 sources
+// 20.2 / 14.5 ms (32.2); R-MAT 18 with 64 sources 10.9 / 10.9 ms (29.9); a
+// uniform graph of 2^20 vertices with 32 sources 12.1 / 12.1 ms (20.0).
+constexpr uint32_t ms_few(int W) { return W <= 16 ? 1u << 18 : 1u << 19; }
+constexpr int MS_AHEAD = 8;  // phases launched ahead of the device
+
 struct MsWork {
-  DevBuf dist, m0, m1, far, q[4], cnt, ctl, src, wstat;
+  DevBuf dist, mask[3], far, q[5], cnt, ctl, src, wstat;
   void release() {
-    for (DevBuf *b : {&dist, &m0, &m1, &far, &cnt, &ctl, &src, &wstat}) b->release();
+    for (DevBuf *b : {&dist, &mask[0], &mask[1], &mask[2], &far, &cnt, &ctl, &src, &wstat})
+      b->release();
     for (auto &b : q) b.release();
   }
 };
@@ -678,100 +816,64 @@ struct MsStats {
   }
 };
 
+// One group's solve.  spans: merge buckets while they hold little work.
 template <int W, bool SCAN>
-gb_status ms_group(MsCtx c, const int32_t *d_src, int max_phases, int grid, hipStream_t st,
-                   uint32_t *out_rows, MsStats &sx) {
+gb_status ms_group(MsCtx c, const int32_t *d_src, int max_phases, bool spans, int grid,
+                   hipStream_t st, uint32_t *out_rows, MsStats &sx) {
   MsWork &w = g_msw;
   const int64_t V = c.V;
-  hipLaunchKernelGGL(ms_fill_kernel, dim3((unsigned)std::min<int64_t>((V * W + 255) / 256, 65536)),
-                     dim3(256), 0, st, V * W, c.dist);
-  GB_HIP(hipMemsetAsync(c.mask[0], 0, sizeof(unsigned long long) * V, st));
-  if (!SCAN) GB_HIP(hipMemsetAsync(c.mask[1], 0, sizeof(unsigned long long) * V, st));
-  GB_HIP(hipMemsetAsync(c.far, 0, sizeof(unsigned long long) * V, st));
-  GB_HIP(hipMemsetAsync(c.cnt, 0, sizeof(unsigned long long) * MS_N, st));
+  const int64_t qn = V + c.E / MS_MIN_CHUNK + 1;
+  const int nm = SCAN ? 1 : 3, nq = SCAN ? 2 : 3;
+  for (int k = 0; k < nm; k++) {
+    GB_TRY(w.mask[k].ensure(sizeof(unsigned long long) * V));
+    c.mask[k] = w.mask[k].as<unsigned long long>();
+  }
+  for (int k = 0; k < nq; k++) {
+    GB_TRY(w.q[k].ensure(sizeof(MsEnt) * qn));
+    c.qn[k] = w.q[k].as<MsEnt>();
+  }
   const int64_t nwaves = (int64_t)grid * (MS_BLOCK / GB_WAVE);
-  GB_HIP(hipMemsetAsync(c.wstat, 0, sizeof(unsigned long long) * GB_WSTAT * nwaves, st));
-  hipLaunchKernelGGL((ms_seed_kernel<W, SCAN>), dim3(1), dim3(64), 0, st, c, d_src);
-  GB_HIP(hipGetLastError());
-  // the loop state.  Scan form: one state in ctl[0], advanced to the first
-  // action here, then after every phase's compaction.  Append form: two
-  // states alternating per phase: phase k acts on ctl[k % 2], which the launch
-  // before it computed from ctl[(k + 1) % 2]; the first launch starts from the
-  // initial state in ctl[1] (no action taken yet)
+  GbProgress *prog = nullptr;
+  GB_TRY(gb_progress_begin(&prog));
   MsCtl hc{};
   hc.max_phases = max_phases > 0 ? max_phases : ((int64_t)1 << 40);
   hc.state = MS_ST_LIGHT;
   hc.buckets = 1;
   hc.action = ACT_NONE;
-  MsCtl *ctl = w.ctl.as<MsCtl>();
-  MsCtl *hstate = SCAN ? ctl : ctl + 1;  // where a replay leaves the state
-  GB_HIP(hipMemcpyAsync(hstate, &hc, sizeof(hc), hipMemcpyHostToDevice, st));
-  if (SCAN) {
-    hipLaunchKernelGGL(ms_ctrl_kernel, dim3(1), dim3(1), 0, st, c, ctl);
-    GB_HIP(hipGetLastError());
-  }
-  const int cgrid = SCAN ? ms_compact_grid(c.V) : gb_num_cus() * 2;
+  hc.sp.adapt = spans ? 1 : 0;
+  hc.sp.few = ms_few(W);
+  hc.sp.many = 16 * ms_few(W);
+  hc.sp.leap = 8;
+  MsLoop *loop = w.ctl.as<MsLoop>();
+  MsCtl *ctl = (MsCtl *)(loop + 1);
+  const int64_t fill = std::max<int64_t>(V * W / 4, GB_WSTAT * nwaves);
+  hipLaunchKernelGGL(ms_begin_kernel, dim3((unsigned)std::min<int64_t>((fill + 255) / 256, 65536)),
+                     dim3(256), 0, st, c, W, nm, loop, hc, ctl, GB_WSTAT * nwaves);
+  // the append form's seeds count as appended by the phase before phase 0
+  hipLaunchKernelGGL((ms_seed_kernel<W, SCAN>), dim3(1), dim3(64), 0, st, c, d_src,
+                     SCAN ? &c.cnt[MS_NEAR0] : &loop->adds[2].near);
+  if (SCAN) hipLaunchKernelGGL(ms_ctrl_kernel, dim3(1), dim3(1), 0, st, c, ctl, 0u, prog);
+  GB_HIP(hipGetLastError());
+  const int cgrid = ms_compact_grid(c.V);
   // vertices per compaction block: a multiple of MS_CSPAN, cgrid blocks cover V
   const int64_t crange = ((c.V + cgrid - 1) / cgrid + MS_CSPAN - 1) / MS_CSPAN * MS_CSPAN;
-  constexpr int PH = 16;  // phases per replay (even: the append form ends on ctl[1])
-  hipStream_t cs = st, own = nullptr;
-  if (!st) {  // the null stream cannot be captured
-    GB_HIP(hipStreamCreate(&own));
-    cs = own;
-    hipEvent_t ready;
-    GB_HIP(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
-    GB_HIP(hipEventRecord(ready, st));
-    GB_HIP(hipStreamWaitEvent(cs, ready, 0));
-    (void)hipEventDestroy(ready);
-  }
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  gb_status gst = GB_OK;
-  hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
-  if (e == hipSuccess) {
-    for (int k = 0; k < PH; k++) {
-      if (SCAN) {
-        hipLaunchKernelGGL((ms_step_kernel<W, true>), dim3(grid), dim3(MS_BLOCK), 0, cs, c,
-                           (const MsCtl *)ctl);
-        hipLaunchKernelGGL(ms_compact_kernel<W>, dim3(cgrid), dim3(MS_BLOCK), 0, cs, c,
-                           (const MsCtl *)ctl, crange);
-        hipLaunchKernelGGL(ms_ctrl_kernel, dim3(1), dim3(1), 0, cs, c, ctl);
-      } else {
-        MsCtl *cur = ctl + (k % 2), *prev = ctl + ((k + 1) % 2);
-        hipLaunchKernelGGL(ms_clear_ctrl_kernel, dim3(cgrid), dim3(256), 0, cs, c,
-                           (const MsCtl *)prev, cur);
-        hipLaunchKernelGGL((ms_step_kernel<W, false>), dim3(grid), dim3(MS_BLOCK), 0, cs, c,
-                           (const MsCtl *)cur);
-      }
+  const gb_status gst = gb_drive_phases(prog, MS_AHEAD, st, [&](uint32_t k) {
+    if (SCAN) {
+      hipLaunchKernelGGL(ms_step_kernel<W>, dim3(grid), dim3(MS_BLOCK), 0, st, c,
+                         (const MsCtl *)ctl);
+      hipLaunchKernelGGL(ms_compact_kernel<W>, dim3(cgrid), dim3(MS_BLOCK), 0, st, c,
+                         (const MsCtl *)ctl, crange);
+      hipLaunchKernelGGL(ms_ctrl_kernel, dim3(1), dim3(1), 0, st, c, ctl, k, prog);
+    } else {
+      hipLaunchKernelGGL(ms_append_kernel<W>, dim3(grid), dim3(MS_BLOCK), 0, st, c, loop, k, prog);
     }
-    e = hipStreamEndCapture(cs, &graph);
+    return hipGetLastError();
+  });
+  if (gst != GB_OK) {
+    (void)hipStreamSynchronize(st);  // launches before an error end first
+    return gst;
   }
-  if (e == hipSuccess) e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-  if (e != hipSuccess) gst = gb_fail(GB_ERR_HIP, "msssp: graph capture failed: %s", hipGetErrorString(e));
-  MsCtl hs{};
-  int64_t last = -1;
-  while (gst == GB_OK) {
-    if (hipGraphLaunch(exec, cs) != hipSuccess ||
-        hipMemcpyAsync(&hs, hstate, sizeof(hs), hipMemcpyDeviceToHost, cs) != hipSuccess ||
-        hipStreamSynchronize(cs) != hipSuccess) {
-      gst = gb_fail(GB_ERR_HIP, "msssp: phase replay failed");
-      break;
-    }
-    if (hs.done) break;
-    if (hs.phases == last) {
-      gst = gb_fail(GB_ERR_HIP, "msssp: bucket loop made no progress");
-      break;
-    }
-    last = hs.phases;
-  }
-  if (exec) (void)hipGraphExecDestroy(exec);
-  if (graph) (void)hipGraphDestroy(graph);
-  if (own) {
-    (void)hipStreamSynchronize(own);
-    (void)hipStreamDestroy(own);
-  }
-  GB_TRY(gst);
-  if (hs.capped) return gb_fail(GB_ERR_NOT_CONVERGED, "sssp: phase cap reached");
+  if (prog->capped) return gb_fail(GB_ERR_NOT_CONVERGED, "sssp: phase cap reached");
   constexpr int VT = 4096 / W;
   hipLaunchKernelGGL(ms_unpack_kernel<W>, dim3((unsigned)((V + VT - 1) / VT)), dim3(256), 0, st,
                      V, c.ntask, (const uint32_t *)c.dist, out_rows);
@@ -781,8 +883,8 @@ gb_status ms_group(MsCtx c, const int32_t *d_src, int max_phases, int grid, hipS
   unsigned long long h[MS_N];
   GB_HIP(hipMemcpyAsync(h, c.cnt, sizeof(h), hipMemcpyDeviceToHost, st));
   GB_HIP(hipStreamSynchronize(st));
-  sx.phases = hs.phases;
-  sx.buckets = hs.buckets;
+  sx.phases = prog->phases;
+  sx.buckets = prog->buckets;
   sx.relax = h[MS_RELAX];
   sx.imp_near = (int64_t)h[MS_IMP_NEAR];
   sx.imp_far = (int64_t)h[MS_IMP_FAR];
@@ -797,8 +899,19 @@ gb_status ms_group_shape(MsCtx c, const int32_t *d_src, int max_phases, const Ms
                          hipStream_t st, uint32_t *out_rows, MsStats &sx) {
   c.cshift = sh.cshift;
   const int grid = gb_num_cus() * sh.per_cu;
-  return sh.scan ? ms_group<W, true>(c, d_src, max_phases, grid, st, out_rows, sx)
-                 : ms_group<W, false>(c, d_src, max_phases, grid, st, out_rows, sx);
+  auto run = [&](bool spans) {
+    return sh.scan ? ms_group<W, true>(c, d_src, max_phases, spans, grid, st, out_rows, sx)
+                   : ms_group<W, false>(c, d_src, max_phases, spans, grid, st, out_rows, sx);
+  };
+  // Buckets are merged unless the caller caps the phases (a count of its own
+  // width's) or GB_SSSP_SPANS=0.  A wider range may add a weight to a distance
+  // that is not final yet: when a sum overflows in a solve with ranges, the
+  // solve with single buckets decides.
+  const char *e = getenv("GB_SSSP_SPANS");
+  const bool spans = max_phases <= 0 && !(e && e[0] == '0');
+  GB_TRY(run(spans));
+  if (sx.ovf && spans) GB_TRY(run(false));
+  return GB_OK;
 }
 
 // The shape for a group of width W on graph g: the environment's fixed parts,
@@ -852,7 +965,9 @@ gb_status ms_group_tuned(gb_graph g, MsCtx c, const int32_t *d_src, int max_phas
   auto consider = [&](MsShapeRt s) -> gb_status {
     double ms = 0;
     MsStats o;
-    GB_TRY(timed(s, ms, o));
+    const gb_status r = timed(s, ms, o);
+    if (r == GB_ERR_NOMEM) return GB_OK;  // no room for the other form's buffers
+    GB_TRY(r);
     if (ms < best_ms) {
       best = s;
       best_ms = ms;
@@ -915,23 +1030,17 @@ gb_status gb_msssp_run(gb_graph g, uint32_t delta, const int32_t *h_sources, int
                        int64_t *expanded, bool *ovf, hipStream_t st) {
   MsWork &w = g_msw;
   const int64_t V = g->V, E = g->E;
-  // queue capacity: a vertex enters a near queue at most once per phase with
-  // ceil(deg / chunk) entries, a far queue at most once
-  const int64_t qn = V + E / MS_MIN_CHUNK + 1;
+  // queue capacities: a vertex enters a near queue at most once per phase with
+  // ceil(deg / chunk) entries (ms_group), a far queue at most once
   const int Wmax = nsrc >= 64 ? 64 : (nsrc > 32 ? 64 : nsrc > 16 ? 32 : nsrc > 8 ? 16 : 8);
   GB_TRY(w.dist.ensure(sizeof(uint32_t) * (size_t)V * Wmax));
-  // both forms' buffers: the autotuner may try either
-  GB_TRY(w.m0.ensure(sizeof(unsigned long long) * V));
-  GB_TRY(w.m1.ensure(sizeof(unsigned long long) * V));
   GB_TRY(w.far.ensure(sizeof(unsigned long long) * V));
-  GB_TRY(w.q[0].ensure(sizeof(MsEnt) * qn));
-  GB_TRY(w.q[1].ensure(sizeof(MsEnt) * qn));
-  GB_TRY(w.q[2].ensure(sizeof(uint64_t) * (V + 1)));
   GB_TRY(w.q[3].ensure(sizeof(uint64_t) * (V + 1)));
+  GB_TRY(w.q[4].ensure(sizeof(uint64_t) * (V + 1)));
   GB_TRY(w.cnt.ensure(sizeof(unsigned long long) * MS_N));
   GB_TRY(w.wstat.ensure(sizeof(unsigned long long) * GB_WSTAT * gb_num_cus() * MS_MAX_PER_CU *
                         (MS_BLOCK / GB_WAVE)));
-  GB_TRY(w.ctl.ensure(2 * sizeof(MsCtl)));
+  GB_TRY(w.ctl.ensure(sizeof(MsLoop) + sizeof(MsCtl)));
   GB_TRY(w.src.ensure(sizeof(int32_t) * 64));
   MsCtx c{};
   c.rp = g->rp;
@@ -940,13 +1049,9 @@ gb_status gb_msssp_run(gb_graph g, uint32_t delta, const int32_t *h_sources, int
   c.V = g->V;
   c.E = g->E;
   c.dist = w.dist.as<uint32_t>();
-  c.mask[0] = w.m0.as<unsigned long long>();
-  c.mask[1] = w.m1.as<unsigned long long>();
   c.far = w.far.as<unsigned long long>();
-  c.qn[0] = w.q[0].as<MsEnt>();
-  c.qn[1] = w.q[1].as<MsEnt>();
-  c.qf[0] = w.q[2].as<uint64_t>();
-  c.qf[1] = w.q[3].as<uint64_t>();
+  c.qf[0] = w.q[3].as<uint64_t>();
+  c.qf[1] = w.q[4].as<uint64_t>();
   c.cnt = w.cnt.as<unsigned long long>();
   c.wstat = w.wstat.as<unsigned long long>();
   c.delta = delta;

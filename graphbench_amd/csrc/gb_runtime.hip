@@ -81,6 +81,14 @@ void gb_dfree(void *p) {
   (void)hipFree(p);
 }
 
+gb_status gb_progress_begin(GbProgress **p) {
+  static GbProgress *rec = nullptr;  // pinned, kept for the process's life
+  if (!rec) GB_HIP(hipHostMalloc((void **)&rec, sizeof(GbProgress), hipHostMallocDefault));
+  *rec = GbProgress{};
+  *p = rec;
+  return GB_OK;
+}
+
 extern "C" {
 
 const char *gb_version(void) { return "graphbench-mi355x 0.1 (gfx950)"; }

@@ -226,17 +226,15 @@ __device__ __forceinline__ double gb_shfl_any<double>(double v, int src) {
 template <class Tr, bool HEAVY, bool SINGLE>
 __device__ __forceinline__ void expand_body(
     const Ctx<Tr> &c, const SGraph<typename Tr::W> &G0, uint64_t *lds_near, uint64_t *lds_far,
-    uint64_t *lds_s, uint64_t *lds_imp, const uint64_t *__restrict__ in,
-    const unsigned long long *__restrict__ n_in, uint64_t *__restrict__ near_out,
+    uint64_t *lds_s, uint64_t *lds_imp, const uint64_t *__restrict__ in, uint64_t n, uint64_t *__restrict__ near_out,
     unsigned long long *n_near, uint64_t *__restrict__ s_out, unsigned long long *n_s,
-    uint64_t *__restrict__ far_out, unsigned long long *n_far, uint64_t bucket,
+    uint64_t *__restrict__ far_out, unsigned long long *n_far, uint64_t bucket, bool all,
     uint32_t gen_next, uint32_t sround, uint32_t fepoch, uint32_t epw) {
   using D = typename Tr::D;
   const int lane = gb_lane();
   gb_wave_queue<uint64_t, NEAR_CAP> nearq(lds_near, near_out, n_near);
   gb_wave_queue<uint64_t, FAR_CAP> farq(lds_far, far_out, n_far);
   gb_wave_queue<uint64_t, S_CAP> sq(lds_s, s_out, n_s);
-  const uint64_t n = *n_in;
   const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) >> 6;
   uint32_t relax = 0, imp_near = 0, imp_far = 0;
@@ -259,9 +257,9 @@ __device__ __forceinline__ void expand_body(
       const int32_t rs = tk.G.rp[u], le = tk.G.le[u], re = tk.G.rp[u + 1];
       if (!HEAVY) {
         beg = rs + (int32_t)(ch << CHUNK_SHIFT);
-        end = min(le, beg + CHUNK);
+        end = min(all ? re : le, beg + CHUNK);
         // remember_arr: the first chunk records u in S (heavy edges pending)
-        if (ch == 0 && re > le && atomicExch(&c.sst[tk.s(u)], sround) != sround)
+        if (!all && ch == 0 && re > le && atomicExch(&c.sst[tk.s(u)], sround) != sround)
           scnt = nchunks(re - le);
       } else {
         beg = le + (int32_t)(ch << CHUNK_SHIFT);
@@ -310,7 +308,7 @@ __device__ __forceinline__ void expand_body(
         wv[s] = tk.G.w[e[s]];
       }
       D *dp[EXP_U];
-      bool isfar[EXP_U];
+      bool isfar[EXP_U], later[EXP_U];
 #pragma unroll
       for (int s = 0; s < EXP_U; s++) {
         const TaskView<Tr, SINGLE> tk(c, G0, tj[s]);
@@ -318,7 +316,12 @@ __device__ __forceinline__ void expand_body(
         nd[s] = Tr::add(duj[s], wv[s], o);
         ovf |= o & ok[s];
         relax += ok[s];
-        isfar[s] = Tr::bucket(nd[s], tk.delta, tk.magic) > bucket;
+        const uint64_t bk = Tr::bucket(nd[s], tk.delta, tk.magic);
+        isfar[s] = bk > bucket;
+        // the counters tell the buckets of the caller's width apart, also
+        // within a range (a division per edge that single buckets do without)
+        later[s] = isfar[s];
+        if (all) later[s] = bk > Tr::bucket(duj[s], tk.delta, tk.magic);
         dp[s] = tk.d(v[s]);
         old[s] = *dp[s];
       }
@@ -331,8 +334,8 @@ __device__ __forceinline__ void expand_body(
       uint32_t nimp = 0;
 #pragma unroll
       for (int s = 0; s < EXP_U; s++) {
-        imp_near += ok[s] & !isfar[s];
-        imp_far += ok[s] & isfar[s];
+        imp_near += ok[s] & !later[s];
+        imp_far += ok[s] & later[s];
         uint32_t cnt_s;
         const uint32_t pos = gb_wave_excl_sum(ok[s] ? 1u : 0u, &cnt_s);
         if (ok[s])
@@ -362,7 +365,7 @@ __device__ __forceinline__ void expand_body(
           if (isfar) {
             far = re > rs;
           } else {
-            ncnt = nchunks(tk.G.le[vi] - rs);
+            ncnt = nchunks((all ? re : tk.G.le[vi]) - rs);
             if (ncnt == 0 && re > rs) ncnt = 1;
           }
         }
@@ -389,13 +392,13 @@ __device__ __forceinline__ void expand_body(
 template <class Tr, bool SINGLE>
 __device__ __forceinline__ void far_scan_body(
     const Ctx<Tr> &c, const SGraph<typename Tr::W> &G0, uint64_t *lds_near, uint64_t *lds_far,
-    const uint64_t *__restrict__ in, const unsigned long long *__restrict__ n_in,
-    uint64_t *__restrict__ near_out, unsigned long long *n_near, uint64_t *__restrict__ far_out,
-    unsigned long long *n_far, uint64_t bnext, uint32_t gen_next, uint32_t fepoch_next) {
+    const uint64_t *__restrict__ in, uint64_t n, uint64_t *__restrict__ near_out,
+    unsigned long long *n_near, uint64_t *__restrict__ far_out, unsigned long long *n_far,
+    unsigned long long *minb_out, uint64_t first, uint64_t last, bool all, uint32_t gen_next,
+    uint32_t fepoch_next) {
   const int lane = gb_lane();
   gb_wave_queue<uint64_t, NEAR_CAP> nearq(lds_near, near_out, n_near);
   gb_wave_queue<uint64_t, FAR_CAP> farq(lds_far, far_out, n_far);
-  const uint64_t n = *n_in;
   const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) >> 6;
   uint64_t minb = ~0ull;
@@ -410,13 +413,13 @@ __device__ __forceinline__ void far_scan_body(
       v = (uint32_t)ent;
       const TaskView<Tr, SINGLE> tk(c, G0, t);
       const uint64_t bk = Tr::bucket(*tk.d(v), tk.delta, tk.magic);
-      if (bk == bnext) {
+      if (bk >= first && bk <= last) {
         if (atomicExch(&c.nst[tk.s(v)], gen_next) != gen_next) {
           const SGraph<typename Tr::W> &G = tk.G;
-          ncnt = nchunks(G.le[v] - G.rp[v]);
+          ncnt = nchunks((all ? G.rp[v + 1] : G.le[v]) - G.rp[v]);
           if (ncnt == 0) ncnt = 1;
         }
-      } else if (bk > bnext) {
+      } else if (bk > last) {
         if (atomicExch(&c.fst[tk.s(v)], fepoch_next) != fepoch_next) far = true;
         minb = bk < minb ? bk : minb;
       }
@@ -425,37 +428,105 @@ __device__ __forceinline__ void far_scan_body(
     farq.push(far ? 1u : 0u, [&](uint32_t) { return mk_entry(t, 0, v); });
   }
   gb_block_flush(nearq, farq);
-  gb_block_atomic_min(minb, ~0ull, &c.cnt[C_MINB]);
+  gb_block_atomic_min(minb, ~0ull, minb_out);
 }
 
 // ---- device-driven phase loop ----------------------------------------------
 // The bucket loop runs as a state machine on the device, so that the host
-// neither reads queue sizes nor chooses launches: sssp_ctrl_kernel (one lane)
-// looks at the counters left by the previous phase, advances the loop state,
-// clears the counters the next phase appends to, and writes the next action;
-// sssp_step_kernel (fixed grid) performs that action.  Pairs of the two are
-// captured in a hipGraph and replayed until the state says done.
+// neither reads queue sizes nor chooses launches.  A phase is one launch:
+// every block advances the state from what the phase before left (thread 0,
+// a few hundred cycles) and performs the action it finds; block 0 writes the
+// new state for the next phase.  A launch of its own for the advance had cost
+// another 4 us per phase.  Nothing a phase reads is written in the same phase:
+//   * the state alternates between two buffers,
+//   * appends are counted in one of three SsspAdds in turn: the phase before's
+//     is read, this phase's is written, the next one's is cleared.
 // Queues: 0/1 near (double-buffered), 2 settled set S, 3/4 far (double-
-// buffered); queue k's length is counter k.
+// buffered).
+// The host launches ahead of the device by at most SSSP_AHEAD phases, following
+// the phase number that block 0 leaves in pinned memory; launches past the end
+// find the state done.
 struct Queues {
   uint64_t *q[5];
 };
+struct SsspAdds {
+  unsigned long long near, s, far, minb;
+};
+struct SsspDev {
+  SsspCtl ctl;
+  unsigned long long n[C_MINB + 1];  // queue lengths and the smallest far bucket
+};
+struct SsspLoop {
+  SsspDev st[2];
+  SsspAdds adds[3];
+};
+constexpr int SSSP_AHEAD = 8;
 
-__global__ void sssp_ctrl_kernel(unsigned long long *__restrict__ cnt, SsspCtl *__restrict__ ctl,
-                                 uint32_t cus) {
-  if (threadIdx.x != 0) return;
-  SsspCtl s = *ctl;
-  sssp_ctl_advance(s, cnt, cus);
-  *ctl = s;
+// State before phase 0 (the seeds follow), counters and statistics cleared.
+__global__ void sssp_begin_kernel(SsspLoop *__restrict__ L, SsspCtl ctl, int64_t nstat,
+                                  unsigned long long *__restrict__ wstat,
+                                  unsigned long long *__restrict__ cnt) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < nstat) wstat[i] = 0;
+  if (i < C_N + 2) cnt[i] = 0;
+  if (i == 0) {
+    SsspDev d{};
+    d.ctl = ctl;
+    L->st[1] = d;
+    for (int k = 0; k < 3; k++) L->adds[k] = SsspAdds{0, 0, 0, ~0ull};
+  }
 }
 
 template <class Tr, bool SINGLE>
 __global__ __launch_bounds__(SS_BLOCK) void sssp_step_kernel(Ctx<Tr> c, Queues q,
-                                                              const SsspCtl *__restrict__ ctl) {
-  const int act = ctl->action;
-  if (act == ACT_NONE) return;
-  unsigned long long *cnt = c.cnt;
-  const int in = ctl->a_in, nr = ctl->a_near, fr = ctl->a_far;
+                                                              SsspLoop *__restrict__ L, uint32_t k,
+                                                              uint32_t cus, GbProgress *prog) {
+  __shared__ SsspDev s_dev;
+  __shared__ SsspAdds s_add;
+  constexpr int DW = sizeof(SsspDev) / 4, AW = sizeof(SsspAdds) / 4;
+  static_assert(DW + AW <= SS_BLOCK && sizeof(SsspDev) % 4 == 0, "one load per thread");
+  {
+    const uint32_t *ds = (const uint32_t *)&L->st[(k + 1) & 1];
+    const uint32_t *as = (const uint32_t *)&L->adds[(k + 2) % 3];
+    const int t = threadIdx.x;
+    if (t < DW)
+      ((uint32_t *)&s_dev)[t] = ds[t];
+    else if (t < DW + AW)
+      ((uint32_t *)&s_add)[t - DW] = as[t - DW];
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && !s_dev.ctl.done) {
+    const int act = s_dev.ctl.action;
+    // the phase before appended to the queues its action names; before phase
+    // 0 the seeds went to near queue 0
+    s_dev.n[act == ACT_NONE ? C_NEAR0 : s_dev.ctl.a_near] += s_add.near;
+    s_dev.n[C_S] += s_add.s;
+    if (act != ACT_NONE) s_dev.n[s_dev.ctl.a_far] += s_add.far;
+    s_dev.n[C_MINB] = s_add.minb;
+    sssp_ctl_advance(s_dev.ctl, s_dev.n, cus);
+  }
+  __syncthreads();
+  if (blockIdx.x == 0) {
+    if (threadIdx.x < DW) ((uint32_t *)&L->st[k & 1])[threadIdx.x] = ((uint32_t *)&s_dev)[threadIdx.x];
+    if (threadIdx.x == 0) {
+      L->adds[(k + 1) % 3] = SsspAdds{0, 0, 0, ~0ull};
+      gb_progress(prog, k, s_dev.ctl.done, s_dev.ctl.phases, s_dev.ctl.buckets, s_dev.ctl.capped);
+    }
+  }
+  const SsspCtl &ctl = s_dev.ctl;
+  const int act = (int)gb_uniform((uint32_t)ctl.action);
+  if (ctl.done || act == ACT_NONE) return;
+  const int in = (int)gb_uniform((uint32_t)ctl.a_in);
+  const int nr = (int)gb_uniform((uint32_t)ctl.a_near), fr = (int)gb_uniform((uint32_t)ctl.a_far);
+  SsspAdds *add = &L->adds[k % 3];
+  const uint64_t n = gb_uniform((uint64_t)s_dev.n[in]);
+  // the near queue and, in a far scan, the far queue start empty
+  uint64_t *far_out = q.q[fr] + gb_uniform((uint64_t)s_dev.n[fr]);
+  uint64_t *s_out = q.q[C_S] + gb_uniform((uint64_t)s_dev.n[C_S]);
+  const uint64_t first = gb_uniform(ctl.a_first), last = gb_uniform(ctl.a_bucket);
+  const bool all = gb_uniform((uint32_t)ctl.a_all) != 0;
+  const uint32_t a_gen = gb_uniform(ctl.a_gen), a_sround = gb_uniform(ctl.a_sround);
+  const uint32_t a_fepoch = gb_uniform(ctl.a_fepoch), a_epw = gb_uniform(ctl.a_epw);
   SGraph<typename Tr::W> G0{};
   if constexpr (SINGLE) G0 = c.graphs[0];
   __shared__ uint64_t s_near[SS_BLOCK / GB_WAVE][NEAR_CAP];
@@ -465,16 +536,16 @@ __global__ __launch_bounds__(SS_BLOCK) void sssp_step_kernel(Ctx<Tr> c, Queues q
   uint64_t *ln = s_near[threadIdx.x / GB_WAVE], *lf = s_far[threadIdx.x / GB_WAVE];
   uint64_t *ls = s_set[threadIdx.x / GB_WAVE], *li = s_imp[threadIdx.x / GB_WAVE];
   if (act == ACT_FAR) {
-    far_scan_body<Tr, SINGLE>(c, G0, ln, lf, q.q[in], cnt + in, q.q[nr], cnt + nr, q.q[fr],
-                              cnt + fr, ctl->a_bucket, ctl->a_gen, ctl->a_fepoch);
+    far_scan_body<Tr, SINGLE>(c, G0, ln, lf, q.q[in], n, q.q[nr], &add->near, far_out, &add->far,
+                              &add->minb, first, last, all, a_gen, a_fepoch);
   } else if (act == ACT_LIGHT) {
-    expand_body<Tr, false, SINGLE>(c, G0, ln, lf, ls, li, q.q[in], cnt + in, q.q[nr], cnt + nr,
-                                   q.q[C_S], cnt + C_S, q.q[fr], cnt + fr, ctl->a_bucket,
-                                   ctl->a_gen, ctl->a_sround, ctl->a_fepoch, ctl->a_epw);
+    expand_body<Tr, false, SINGLE>(c, G0, ln, lf, ls, li, q.q[in], n, q.q[nr], &add->near, s_out,
+                                   &add->s, far_out, &add->far, last, all, a_gen, a_sround,
+                                   a_fepoch, a_epw);
   } else {
-    expand_body<Tr, true, SINGLE>(c, G0, ln, lf, ls, li, q.q[in], cnt + in, q.q[nr], cnt + nr,
-                                  q.q[C_S], cnt + C_S, q.q[fr], cnt + fr, ctl->a_bucket,
-                                  ctl->a_gen, ctl->a_sround, ctl->a_fepoch, ctl->a_epw);
+    expand_body<Tr, true, SINGLE>(c, G0, ln, lf, ls, li, q.q[in], n, q.q[nr], &add->near, s_out,
+                                  &add->s, far_out, &add->far, last, false, a_gen, a_sround,
+                                  a_fepoch, a_epw);
   }
 }
 
@@ -517,9 +588,9 @@ __global__ __launch_bounds__(SS_BLOCK) void sssp_count_kernel(Ctx<Tr> c, int32_t
 }
 
 struct SsspWork {
-  DevBuf graphs, tasks, nst, sst, fst, q[5], cnt, counts, ctl, wstat;
+  DevBuf graphs, tasks, nst, sst, fst, q[5], cnt, loop, wstat;
   void release() {
-    for (DevBuf *b : {&graphs, &tasks, &nst, &sst, &fst, &cnt, &counts, &ctl, &wstat}) b->release();
+    for (DevBuf *b : {&graphs, &tasks, &nst, &sst, &fst, &cnt, &loop, &wstat}) b->release();
     for (auto &b : q) b.release();
   }
 };
@@ -531,10 +602,18 @@ SsspWork &g_ssw_ref() {
 }
 #define g_ssw (g_ssw_ref())
 
+// Queue entries per phase of a range below which the next range is twice as
+// wide, and above which it is half as wide.  One source, at 4096 / 16384 /
+// 65536 entries: R-MAT 20 1.87 / 1.10 / 0.97 ms (2.9 with single buckets),
+// R-MAT 16 0.51 / 0.52 / 0.53 ms (1.9); growing by 4 or 8 instead of 2 relaxes
+// twice the edges of a uniform graph (2^20 vertices: 1.8 against 1.4 ms).
+constexpr uint32_t SSSP_FEW = 65536, SSSP_MANY = 524288;
+
 template <class Tr>
-gb_status sssp_engine(const std::vector<SGraph<typename Tr::W>> &hg,
-                      std::vector<STask<Tr>> &ht, int max_phases, gb_sssp_stats *stats,
-                      hipStream_t st) {
+gb_status sssp_engine_run(const std::vector<SGraph<typename Tr::W>> &hg,
+                          std::vector<STask<Tr>> &ht, int max_phases, bool spans,
+                          gb_sssp_stats *stats, bool *ovf, hipStream_t st) {
+  *ovf = false;
   using G = SGraph<typename Tr::W>;
   const int32_t ntasks = (int32_t)ht.size();
   if (ntasks <= 0) return GB_OK;
@@ -564,7 +643,8 @@ gb_status sssp_engine(const std::vector<SGraph<typename Tr::W>> &hg,
   GB_TRY(w.sst.ensure(sizeof(uint32_t) * total));
   GB_TRY(w.fst.ensure(sizeof(uint32_t) * total));
   for (int k = 0; k < 5; k++) GB_TRY(w.q[k].ensure(sizeof(uint64_t) * qcap));
-  GB_TRY(w.cnt.ensure(sizeof(unsigned long long) * C_N));
+  // counters, then the reached pairs and their out-edges
+  GB_TRY(w.cnt.ensure(sizeof(unsigned long long) * (C_N + 2)));
   // Step-kernel blocks per CU: 4 while the largest graph has fewer than 2^27
   // edges, 16 beyond.  Measured at 4 / 16: one source of R-MAT 16 / 20 / 22
   // 1.93 / 3.09 / 4.61 ms against 2.30 / 4.11 / 5.85 ms, the 512-graph batch
@@ -574,156 +654,113 @@ gb_status sssp_engine(const std::vector<SGraph<typename Tr::W>> &hg,
   const int grid = gb_num_cus() * (max_e < ((int64_t)1 << 27) ? 4 : 16);
   const int64_t nwaves = (int64_t)grid * (SS_BLOCK / GB_WAVE);
   GB_TRY(w.wstat.ensure(sizeof(unsigned long long) * GB_WSTAT * nwaves));
-  GB_TRY(w.ctl.ensure(sizeof(SsspCtl)));
+  GB_TRY(w.loop.ensure(sizeof(SsspLoop)));
   GB_HIP(hipMemcpyAsync(w.graphs.p, hg.data(), sizeof(G) * hg.size(), hipMemcpyHostToDevice, st));
   GB_HIP(hipMemcpyAsync(w.tasks.p, ht.data(), sizeof(STask<Tr>) * ht.size(),
                         hipMemcpyHostToDevice, st));
   unsigned long long *cnt = w.cnt.as<unsigned long long>();
-  GB_HIP(hipMemsetAsync(cnt, 0, sizeof(unsigned long long) * C_N, st));
   unsigned long long *wstat = w.wstat.as<unsigned long long>();
-  GB_HIP(hipMemsetAsync(wstat, 0, sizeof(unsigned long long) * GB_WSTAT * nwaves, st));
   Ctx<Tr> c{w.graphs.as<G>(), w.tasks.as<STask<Tr>>(), w.nst.as<uint32_t>(), w.sst.as<uint32_t>(),
             w.fst.as<uint32_t>(), cnt, wstat, ht[0].dist, ht[0].delta, ht[0].magic};
-
-  hipEvent_t e0, e1;
-  GB_HIP(hipEventCreate(&e0));
-  GB_HIP(hipEventCreate(&e1));
-  GB_HIP(hipEventRecord(e0, st));
-  {
-    int gx = (int)std::min<int64_t>((maxV + SS_BLOCK - 1) / SS_BLOCK, 1024);
-    if (gx < 1) gx = 1;
-    if (single)
-      hipLaunchKernelGGL((sssp_fill_kernel<Tr, true>), dim3(gx, ntasks), dim3(SS_BLOCK), 0, st, c,
-                         ntasks);
-    else
-      hipLaunchKernelGGL((sssp_fill_kernel<Tr, false>), dim3(gx, ntasks), dim3(SS_BLOCK), 0, st, c,
-                         ntasks);
-  }
-  const uint32_t gen = 1;
-  if (single)
-    hipLaunchKernelGGL((sssp_seed_kernel<Tr, true>), dim3((ntasks + 255) / 256), dim3(256), 0, st,
-                       c, ntasks, w.q[0].as<uint64_t>(), cnt + C_NEAR0, gen);
-  else
-    hipLaunchKernelGGL((sssp_seed_kernel<Tr, false>), dim3((ntasks + 255) / 256), dim3(256), 0, st,
-                       c, ntasks, w.q[0].as<uint64_t>(), cnt + C_NEAR0, gen);
-  GB_HIP(hipGetLastError());
+  GbProgress *prog = nullptr;
+  GB_TRY(gb_progress_begin(&prog));
+  struct Events {
+    hipEvent_t e[2] = {nullptr, nullptr};
+    ~Events() {
+      for (hipEvent_t x : e)
+        if (x) (void)hipEventDestroy(x);
+    }
+  } ev;
+  for (hipEvent_t &x : ev.e) GB_HIP(hipEventCreate(&x));
+  GB_HIP(hipEventRecord(ev.e[0], st));
   // the loop state starts at bucket 0 with the seeds in near queue 0
+  SsspLoop *loop = w.loop.as<SsspLoop>();
+  const uint32_t gen = 1;
   SsspCtl hc{};
   hc.gen = gen;
-  hc.sround = 0;
   hc.fepoch = 1;
   hc.max_phases = max_phases > 0 ? max_phases : ((int64_t)1 << 40);
   hc.state = ST_BUCKET;
-  GB_HIP(hipMemcpyAsync(w.ctl.p, &hc, sizeof(hc), hipMemcpyHostToDevice, st));
-  SsspCtl *ctl = w.ctl.as<SsspCtl>();
+  hc.sp.adapt = spans ? 1 : 0;
+  hc.sp.few = SSSP_FEW;
+  hc.sp.many = SSSP_MANY;
+  hc.sp.leap = 2;
+  const int64_t nstat = GB_WSTAT * nwaves;
+  hipLaunchKernelGGL(sssp_begin_kernel, dim3((unsigned)((nstat + 255) / 256)), dim3(256), 0, st,
+                     loop, hc, nstat, wstat, cnt);
+  int fx = (int)std::min<int64_t>((maxV + SS_BLOCK - 1) / SS_BLOCK, 1024);
+  if (fx < 1) fx = 1;
+  // the seeds count as appended by the phase before phase 0
+  auto prepare = [&](auto fill, auto seed) {
+    hipLaunchKernelGGL(fill, dim3(fx, ntasks), dim3(SS_BLOCK), 0, st, c, ntasks);
+    hipLaunchKernelGGL(seed, dim3((ntasks + 255) / 256), dim3(256), 0, st, c, ntasks,
+                       w.q[0].as<uint64_t>(), &loop->adds[2].near, gen);
+  };
+  if (single)
+    prepare(sssp_fill_kernel<Tr, true>, sssp_seed_kernel<Tr, true>);
+  else
+    prepare(sssp_fill_kernel<Tr, false>, sssp_seed_kernel<Tr, false>);
+  GB_HIP(hipGetLastError());
   Queues qs{{w.q[0].as<uint64_t>(), w.q[1].as<uint64_t>(), w.q[2].as<uint64_t>(),
              w.q[3].as<uint64_t>(), w.q[4].as<uint64_t>()}};
   const uint32_t cus = (uint32_t)gb_num_cus();
-  auto one_phase = [&]() {
-    hipLaunchKernelGGL(sssp_ctrl_kernel, dim3(1), dim3(64), 0, st, cnt, ctl, cus);
-    if (single)
-      hipLaunchKernelGGL((sssp_step_kernel<Tr, true>), dim3(grid), dim3(SS_BLOCK), 0, st, c, qs,
-                         (const SsspCtl *)ctl);
-    else
-      hipLaunchKernelGGL((sssp_step_kernel<Tr, false>), dim3(grid), dim3(SS_BLOCK), 0, st, c, qs,
-                         (const SsspCtl *)ctl);
+  auto step = [&](auto kernel) {
+    return gb_drive_phases(prog, SSSP_AHEAD, st, [&](uint32_t k) {
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(SS_BLOCK), 0, st, c, qs, loop, k, cus, prog);
+      return hipGetLastError();
+    });
   };
-  // Chunks of PH phases are captured once per call and replayed until the
-  // state is done; a replay past the end costs two near-empty launches per
-  // phase.  The null stream cannot be captured: a blocking stream, ordered
-  // with it, is used for the replays instead.
-  constexpr int PH = 16;
-  hipStream_t cs = st;
-  hipStream_t own = nullptr;
-  if (!st) {
-    GB_HIP(hipStreamCreate(&own));
-    cs = own;
-    hipEvent_t ready;
-    GB_HIP(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
-    GB_HIP(hipEventRecord(ready, st));
-    GB_HIP(hipStreamWaitEvent(cs, ready, 0));
-    (void)hipEventDestroy(ready);
-  }
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  gb_status gst = GB_OK;
-  {
-    hipStream_t keep = st;
-    st = cs;
-    hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
-    if (e == hipSuccess) {
-      for (int k = 0; k < PH; k++) one_phase();
-      e = hipStreamEndCapture(cs, &graph);
-    }
-    if (e == hipSuccess) e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    st = keep;
-    if (e != hipSuccess) gst = gb_fail(GB_ERR_HIP, "sssp: graph capture failed: %s", hipGetErrorString(e));
-  }
-  SsspCtl hs{};
-  int64_t last_phases = -1;
-  while (gst == GB_OK) {
-    if (hipGraphLaunch(exec, cs) != hipSuccess ||
-        hipMemcpyAsync(&hs, ctl, sizeof(hs), hipMemcpyDeviceToHost, cs) != hipSuccess ||
-        hipStreamSynchronize(cs) != hipSuccess) {
-      gst = gb_fail(GB_ERR_HIP, "sssp: phase replay failed");
-      break;
-    }
-    if (hs.done) break;
-    // every replay that is not done issues PH actions; guard the host loop
-    if (hs.phases == last_phases) {
-      gst = gb_fail(GB_ERR_HIP, "sssp: bucket loop made no progress");
-      break;
-    }
-    last_phases = hs.phases;
-  }
-  if (exec) (void)hipGraphExecDestroy(exec);
-  if (graph) (void)hipGraphDestroy(graph);
-  if (own) {
-    (void)hipStreamSynchronize(own);
-    (void)hipStreamDestroy(own);
-  }
-  if (gst == GB_OK && hs.capped) gst = gb_fail(GB_ERR_NOT_CONVERGED, "sssp: phase cap reached");
+  const gb_status gst =
+      single ? step(sssp_step_kernel<Tr, true>) : step(sssp_step_kernel<Tr, false>);
   if (gst != GB_OK) {
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
+    (void)hipStreamSynchronize(st);  // launches before an error end first
     return gst;
   }
-  GB_HIP(hipGetLastError());
-  gb_status status = GB_OK;
-  const int64_t phases = hs.phases, buckets = hs.buckets;
+  if (prog->capped) return gb_fail(GB_ERR_NOT_CONVERGED, "sssp: phase cap reached");
   GB_TRY(gb_wstat_fold(nwaves, wstat, cnt, C_RELAX, C_IMP_NEAR, C_IMP_FAR, st));
-  GB_HIP(hipEventRecord(e1, st));
-  unsigned long long h[C_N];
+  if (stats) {
+    int gx = (int)std::min<int64_t>((maxV + SS_BLOCK - 1) / SS_BLOCK,
+                                    std::max<int64_t>(1, (int64_t)gb_num_cus() * 4 / ntasks));
+    if (gx < 1) gx = 1;
+    GB_HIP(hipEventRecord(ev.e[1], st));
+    hipLaunchKernelGGL(sssp_count_kernel<Tr>, dim3(gx, ntasks), dim3(SS_BLOCK), 0, st, c, ntasks,
+                       cnt + C_N);
+    GB_HIP(hipGetLastError());
+  }
+  unsigned long long h[C_N + 2];
   GB_HIP(hipMemcpyAsync(h, cnt, sizeof(h), hipMemcpyDeviceToHost, st));
   GB_HIP(hipStreamSynchronize(st));
-  if (h[C_OVF]) status = gb_fail(GB_ERR_OVERFLOW, "sssp: uint32 distance overflow");
-  float ms = 0.0f;
-  GB_HIP(hipEventSynchronize(e1));
-  GB_HIP(hipEventElapsedTime(&ms, e0, e1));
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
+  *ovf = h[C_OVF] != 0;
   if (stats) {
-    stats->buckets = buckets;
-    stats->phases = phases;
+    float ms = 0.0f;
+    GB_HIP(hipEventElapsedTime(&ms, ev.e[0], ev.e[1]));
+    stats->buckets = prog->buckets;
+    stats->phases = prog->phases;
     stats->relax_edges = (int64_t)h[C_RELAX];
     stats->improved_near = (int64_t)h[C_IMP_NEAR];
     stats->improved_far = (int64_t)h[C_IMP_FAR];
     stats->expanded_edges = (int64_t)h[C_RELAX];  // one source per expansion
     stats->ms = ms;
-    GB_TRY(w.counts.ensure(2 * sizeof(unsigned long long)));
-    GB_HIP(hipMemsetAsync(w.counts.p, 0, 2 * sizeof(unsigned long long), st));
-    int gx = (int)std::min<int64_t>((maxV + SS_BLOCK - 1) / SS_BLOCK,
-                                    std::max<int64_t>(1, (int64_t)gb_num_cus() * 4 / ntasks));
-    if (gx < 1) gx = 1;
-    hipLaunchKernelGGL(sssp_count_kernel<Tr>, dim3(gx, ntasks), dim3(SS_BLOCK), 0, st, c, ntasks,
-                       w.counts.as<unsigned long long>());
-    unsigned long long hc[2];
-    GB_HIP(hipMemcpyAsync(hc, w.counts.p, sizeof(hc), hipMemcpyDeviceToHost, st));
-    GB_HIP(hipStreamSynchronize(st));
-    stats->reached = (int64_t)hc[0];
-    stats->traversed = (int64_t)hc[1];
+    stats->reached = (int64_t)h[C_N];
+    stats->traversed = (int64_t)h[C_N + 1];
   }
-  return status;
+  return GB_OK;
+}
+
+// One solve of all tasks.  Buckets are merged into ranges unless the caller
+// caps the phases (a count of its own width's) or GB_SSSP_SPANS=0.  A wider
+// range may add a weight to a distance that is not final yet: when a sum
+// overflows in a solve with ranges, the solve with single buckets decides.
+template <class Tr>
+gb_status sssp_engine(const std::vector<SGraph<typename Tr::W>> &hg, std::vector<STask<Tr>> &ht,
+                      int max_phases, gb_sssp_stats *stats, hipStream_t st) {
+  const char *e = getenv("GB_SSSP_SPANS");
+  const bool spans = max_phases <= 0 && !(e && e[0] == '0');
+  bool ovf = false;
+  GB_TRY(sssp_engine_run<Tr>(hg, ht, max_phases, spans, stats, &ovf, st));
+  if (ovf && spans) GB_TRY(sssp_engine_run<Tr>(hg, ht, max_phases, false, stats, &ovf, st));
+  if (ovf) return gb_fail(GB_ERR_OVERFLOW, "sssp: uint32 distance overflow");
+  return GB_OK;
 }
 
 // ---- graphs whose distances fit one workgroup's LDS ------------------------
