@@ -171,6 +171,7 @@ struct GbProgress {
   uint32_t started, done;
   int64_t phases, buckets;
   int32_t capped, pad;
+  double residual, dangling;  // PageRank
 };
 __device__ __forceinline__ void gb_progress(GbProgress *p, uint32_t k, bool done, int64_t phases,
                                             int64_t buckets, int32_t capped) {

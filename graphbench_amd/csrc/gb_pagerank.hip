@@ -82,6 +82,24 @@ __device__ __forceinline__ double block_sum_f64(double v, double *s_red) {
   return t;
 }
 
+// Two block sums with the barriers of one.
+__device__ __forceinline__ void block_sum2_f64(double &a, double &b, double (*s_red)[2]) {
+  a = gb_wave_sum_f64(a);
+  b = gb_wave_sum_f64(b);
+  __syncthreads();
+  if (gb_lane() == 0) {
+    s_red[threadIdx.x >> 6][0] = a;
+    s_red[threadIdx.x >> 6][1] = b;
+  }
+  __syncthreads();
+  a = b = 0.0;
+  const int nw = blockDim.x >> 6;
+  for (int k = 0; k < nw; k++) {
+    a += s_red[k][0];
+    b += s_red[k][1];
+  }
+}
+
 // perm (optional): gather numbering -> caller's numbering, for x0
 __global__ __launch_bounds__(PR_BLOCK) void pr_init_kernel(
     int32_t V, const float *__restrict__ x0, const int32_t *__restrict__ perm,
@@ -419,6 +437,189 @@ __global__ __launch_bounds__(PR_BLOCK) void pr_fixup_kernel(
 }
 
 // ---- reference-semantics form (FP64, bit-identical to the C loop) ---------
+
+// ---- small graphs: one launch per iteration --------------------------------
+// Up to PS_MAX_ITEMS rows and edges an iteration is a few microseconds of work,
+// and a second launch for the fix-up, a hipGraph instantiated whenever another
+// handle's was the last, a stream of its own and the copies of state and ranks
+// around the loop were most of a solve (uniform graph, 20011 vertices, 320 K
+// edges: 370 us for 12 iterations, 130 us now; R-MAT with 60000 vertices, 960 K
+// edges: 468 and 346 us).  Here
+//   * a block owns whole rows (those that end in its merge-path tile), so no
+//     row is left to a fix-up;
+//   * every block starts by summing the residual and dangling partials that the
+//     iteration before left, one pair per block, in the same order: it knows the
+//     next base and whether to stop, so the end of an iteration needs no launch;
+//   * a rank is read and written by its row's owner alone, so the ranks stay in
+//     the caller's array; contributions and partials alternate;
+//   * launches run ahead of the device (gb_drive_phases).
+// A block stages up to PS_CHUNK gathered contributions at a time in LDS, all
+// reads of a chunk in flight together, and sums each row with a power-of-two
+// group of lanes, a row of many edges per lane with a wave (compensated FP32,
+// fixed order); a row that goes past the chunk carries its sum on.
+constexpr int PS_BLOCK = 256;
+constexpr int PS_CHUNK = 4096;
+constexpr int PS_LONG = 16;  // edges per lane of a group from which a wave takes the row
+constexpr int PS_MAX_TILE = 2048;    // rows + edges per tile
+constexpr int PS_MAX_BLOCKS = 1024;  // partials summed by every block
+constexpr int64_t PS_MAX_ITEMS = (int64_t)PS_MAX_TILE * PS_MAX_BLOCKS;
+constexpr int PS_AHEAD = 6, PS_REPORT = 3;  // launches ahead, iterations per report
+
+__global__ __launch_bounds__(PS_BLOCK) void ps_init_kernel(
+    int32_t V, const float *__restrict__ x0, const float *__restrict__ inv_od,
+    const int32_t *__restrict__ tile_row, float *__restrict__ x, float *__restrict__ contrib,
+    double *__restrict__ part, int32_t *__restrict__ done) {
+  __shared__ double s_red[PS_BLOCK / 64];
+  const int32_t r0 = tile_row[blockIdx.x], r1 = tile_row[blockIdx.x + 1];
+  double dang = 0.0;
+  for (int32_t v = r0 + (int32_t)threadIdx.x; v < r1; v += PS_BLOCK) {
+    const float xv = x0 ? x0[v] : (float)(1.0 / (double)V);
+    const float io = inv_od[v];
+    x[v] = xv;
+    contrib[v] = xv * io;
+    if (io == 0.0f) dang += (double)xv;
+  }
+  const double t = block_sum_f64(dang, s_red);
+  if (threadIdx.x == 0) {
+    part[blockIdx.x] = 0.0;
+    part[PS_MAX_BLOCKS + blockIdx.x] = t;
+    if (blockIdx.x == 0) *done = 0;
+  }
+}
+
+// Launch k: the sums of iteration k (k = 0: of the start) decide; if they do
+// not stop the loop, iteration k + 1 runs.  part[parity][2][PS_MAX_BLOCKS]:
+// residual and dangling partials.
+// s_val[0 .. n) = c_old[ic[0 .. n)], n <= PER * PS_BLOCK
+template <int PER>
+__device__ __forceinline__ void ps_stage(const int32_t *__restrict__ ic, int n,
+                                         const float *__restrict__ c_old, float *s_val) {
+  const int tid = threadIdx.x;
+  int32_t u[PER];
+  float g[PER];
+#pragma unroll
+  for (int m = 0; m < PER; m++) u[m] = ic[min(tid + m * PS_BLOCK, n - 1)];
+#pragma unroll
+  for (int m = 0; m < PER; m++) g[m] = c_old[u[m]];
+#pragma unroll
+  for (int m = 0; m < PER; m++)
+    if (tid + m * PS_BLOCK < n) s_val[tid + m * PS_BLOCK] = g[m];
+}
+
+// Compensated sum of val[b .. e) by the G lanes of a group (lane `sub` of it),
+// the same in every lane: strided partial sums, then a butterfly that merges
+// the lower lane's sum first on both sides.
+__device__ __forceinline__ F2 ps_sum(const float *val, int b, int e, int sub, int G) {
+  F2 acc = {0.0f, 0.0f};
+  for (int j = b + sub; j < e; j += G) f2_add(acc, val[j]);
+  for (int m = G >> 1; m >= 1; m >>= 1) {
+    F2 o;
+    o.s = __shfl_xor(acc.s, m, GB_WAVE);
+    o.c = __shfl_xor(acc.c, m, GB_WAVE);
+    acc = (sub & m) ? f2_merge(o, acc) : f2_merge(acc, o);
+  }
+  return acc;
+}
+
+__global__ __launch_bounds__(PS_BLOCK) void ps_iter_kernel(
+    int32_t V, const int32_t *__restrict__ irp, const int32_t *__restrict__ icol,
+    const int32_t *__restrict__ tile_row, const float *__restrict__ inv_od, float *__restrict__ x,
+    const float *__restrict__ c_old, float *__restrict__ c_new, double *__restrict__ part,
+    int32_t *__restrict__ done, int32_t k, int32_t max_iter, double tol, float damping,
+    GbProgress *prog) {
+  __shared__ double s_red[PS_BLOCK / 64][2];
+  __shared__ float s_val[PS_CHUNK];
+  __shared__ int32_t s_rp[PS_MAX_TILE + 1];
+  __shared__ F2 s_carry;
+  if (*done) return;  // by an earlier launch
+  const int tid = threadIdx.x, lane = gb_lane();
+  const int32_t nb = (int32_t)gridDim.x;
+  const double *pin = part + (size_t)(k & 1) * 2 * PS_MAX_BLOCKS;
+  double *pout = part + (size_t)((k + 1) & 1) * 2 * PS_MAX_BLOCKS;
+  const int32_t r0 = tile_row[blockIdx.x], nrows = tile_row[blockIdx.x + 1] - r0;
+  double ra = 0.0, da = 0.0;
+#pragma unroll
+  for (int i = 0; i < PS_MAX_BLOCKS / PS_BLOCK; i++) {
+    const int j = tid + i * PS_BLOCK;
+    const double a = pin[j < nb ? j : 0], b = pin[PS_MAX_BLOCKS + (j < nb ? j : 0)];
+    ra += j < nb ? a : 0.0;
+    da += j < nb ? b : 0.0;
+  }
+  for (int i = tid; i <= nrows; i += PS_BLOCK) s_rp[i] = irp[r0 + i];
+  block_sum2_f64(ra, da, s_red);
+  const double residual = k == 0 ? (double)INFINITY : ra, dangling = da;
+  const bool stop = residual < tol || k >= max_iter;
+  if (blockIdx.x == 0 && tid == 0) {
+    if (stop) {
+      *done = 1;
+      __hip_atomic_store(&prog->residual, residual, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(&prog->dangling, dangling, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    // every store to host memory holds up the launch's end
+    if (stop || k % PS_REPORT == PS_REPORT - 1) gb_progress(prog, (uint32_t)k, stop, k, 0, 0);
+  }
+  if (stop) return;
+  const double N = (double)V, d = (double)damping;
+  const float base = (float)((1.0 - d) / N + d * dangling / N);
+  double res = 0.0, dang = 0.0;
+  if (nrows > 0) {
+    // (the barriers of the block sum came after the writes of s_rp)
+    const int32_t e0 = s_rp[0], e1 = s_rp[nrows];
+    // lanes per row: as many as keep every row in one pass, at most a wave
+    int glog = 0;
+    while (glog < 6 && (nrows << (glog + 1)) <= PS_BLOCK) glog++;
+    const int G = 1 << glog, sub = lane & (G - 1), step = PS_BLOCK >> glog;
+    for (int32_t c0 = e0; c0 == e0 || c0 < e1; c0 += PS_CHUNK) {  // block-uniform
+      const int32_t c1 = min(c0 + PS_CHUNK, e1);
+      const int n = c1 - c0;
+      if (n > 8 * PS_BLOCK)
+        ps_stage<16>(icol + c0, n, c_old, s_val);
+      else if (n > 4 * PS_BLOCK)
+        ps_stage<8>(icol + c0, n, c_old, s_val);
+      else if (n > 0)
+        ps_stage<4>(icol + c0, n, c_old, s_val);
+      const F2 carry = c0 > e0 ? s_carry : F2{0.0f, 0.0f};
+      __syncthreads();
+      // row i, whose part in this chunk is [b, e) and sums to acc
+      auto finish = [&](int i, int32_t rs, int32_t re, int32_t b, int32_t e, F2 acc) {
+        if (rs < c0 && e > b) acc = f2_merge(carry, acc);
+        const bool here = rs < re ? (re > c0 && re <= c1) : c0 == e0;
+        if (here) {
+          const int32_t v = r0 + i;
+          const float xn = base + damping * f2_value(acc), io = inv_od[v];
+          res += fabs((double)xn - (double)x[v]);
+          x[v] = xn;
+          c_new[v] = xn * io;
+          if (io == 0.0f) dang += (double)xn;
+        } else if (e > b && re > c1) {
+          s_carry = acc;  // the one row that goes past this chunk
+        }
+      };
+      for (int i0 = 0; i0 < nrows; i0 += step) {  // block-uniform
+        const int i = i0 + (tid >> glog);
+        const int32_t rs = i < nrows ? s_rp[i] : e1, re = i < nrows ? s_rp[i + 1] : e1;
+        const int32_t b = max(rs, c0), e = min(re, c1);
+        const bool is_long = G < GB_WAVE && e - b > PS_LONG * G;
+        const F2 acc = ps_sum(s_val, b - c0, is_long ? b - c0 : e - c0, sub, G);
+        if (sub == 0 && i < nrows && !is_long) finish(i, rs, re, b, e, acc);
+        uint64_t longs = __ballot(is_long && sub == 0);
+        while (longs) {  // wave-uniform
+          const int l = __ffsll((unsigned long long)longs) - 1;
+          longs &= longs - 1;
+          const int32_t lb = __shfl(b, l, GB_WAVE), le = __shfl(e, l, GB_WAVE);
+          const F2 la = ps_sum(s_val, lb - c0, le - c0, lane, GB_WAVE);
+          if (lane == l) finish(i, rs, re, b, e, la);
+        }
+      }
+      __syncthreads();
+    }
+  }
+  block_sum2_f64(res, dang, s_red);
+  if (tid == 0) {
+    pout[blockIdx.x] = res;
+    pout[PS_MAX_BLOCKS + blockIdx.x] = dang;
+  }
+}
 
 __global__ void pr_ref_init_kernel(int32_t V, const double *__restrict__ recip,
                                    double *__restrict__ x, double *__restrict__ diff,
@@ -1221,7 +1422,7 @@ void build_row_blocks(const std::vector<int32_t> &rp, int nb, std::vector<RowBlo
 }
 
 struct PrWork {
-  DevBuf xa, xb, ca, cb, tail, head, pres, pdang, fres, fdang, state, counter;
+  DevBuf xa, xb, ca, cb, tail, head, pres, pdang, fres, fdang, state, counter, ps_done;
   // the instantiated hipGraph of CH iterations and what its kernels were
   // captured with (graph id, form, sizes, every device pointer): replayed by
   // later calls with the same key instead of captured again
@@ -1241,7 +1442,8 @@ struct PrWork {
   }
   void release() {
     for (DevBuf *b :
-         {&xa, &xb, &ca, &cb, &tail, &head, &pres, &pdang, &fres, &fdang, &state, &counter})
+         {&xa, &xb, &ca, &cb, &tail, &head, &pres, &pdang, &fres, &fdang, &state, &counter,
+          &ps_done})
       b->release();
     for (hipEvent_t e : events) (void)hipEventDestroy(e);
     events.clear();
@@ -1608,6 +1810,73 @@ static bool use_relabel(gb_graph g, const gb_pr_params *p) {
   return p->relabel > 0 || (p->relabel == 0 && g->E >= ((int64_t)1 << 20));
 }
 
+// The one-launch form serves a call that leaves the form open, on graphs that
+// are not relabelled, unless the gather is to be timed or the environment fixes
+// a shape (GB_PR_IPT, GB_PR_HOT, GB_PR_RB, GB_PR_PB) or GB_PR_SMALL=0.
+static bool small_fits(gb_graph g, const gb_pr_params *p) {
+  if (p->items_per_thread || p->row_block || p->binned || p->time_kernels || use_relabel(g, p) ||
+      (int64_t)g->V + g->E > PS_MAX_ITEMS)
+    return false;
+  for (const char *k : {"GB_PR_IPT", "GB_PR_HOT", "GB_PR_RB", "GB_PR_PB"}) {
+    const char *e = getenv(k);
+    if (e && e[0]) return false;
+  }
+  const char *e = getenv("GB_PR_SMALL");
+  return !(e && e[0] == '0');
+}
+
+static gb_status pagerank_small(gb_graph g, const gb_pr_params *p, float *d_x, gb_pr_result *res,
+                                hipStream_t st) {
+  const int32_t V = g->V;
+  const int64_t items = (int64_t)V + g->E;
+  // 1024 items per block (four edges in flight per lane), more past 1024 blocks
+  const int64_t tile = std::max<int64_t>(1024, (items + PS_MAX_BLOCKS - 1) / PS_MAX_BLOCKS);
+  const int64_t nb = (items + tile - 1) / tile;
+  if (g->pr_tile_items != tile || g->pr_tile_relabeled) {
+    GB_TRY(g->pr_tile_row.ensure(sizeof(int32_t) * (nb + 1)));
+    GB_TRY(g->pr_tile_edge.ensure(sizeof(int32_t) * (nb + 1)));
+    GB_TRY(gb_merge_path_split(V, g->rrp, tile, nb, g->pr_tile_row.as<int32_t>(),
+                               g->pr_tile_edge.as<int32_t>(), st));
+    g->pr_tile_items = (int32_t)tile;
+    g->pr_tile_relabeled = false;
+    g->pr_ntiles = nb;
+  }
+  PrWork &w = g_prw;
+  GB_TRY(w.ca.ensure(sizeof(float) * V));
+  GB_TRY(w.cb.ensure(sizeof(float) * V));
+  GB_TRY(w.pres.ensure(sizeof(double) * 4 * PS_MAX_BLOCKS));
+  GB_TRY(w.ps_done.ensure(sizeof(int32_t)));
+  GbProgress *prog = nullptr;
+  GB_TRY(gb_progress_begin(&prog));
+  const int32_t *rows = g->pr_tile_row.as<int32_t>();
+  const float *inv = g->inv_outdeg.as<float>();
+  float *c[2] = {w.ca.as<float>(), w.cb.as<float>()};
+  double *part = w.pres.as<double>();
+  int32_t *done = w.ps_done.as<int32_t>();
+  hipLaunchKernelGGL(ps_init_kernel, dim3((unsigned)nb), dim3(PS_BLOCK), 0, st, V, p->d_x0, inv,
+                     rows, d_x, c[0], part, done);
+  GB_HIP(hipGetLastError());
+  const gb_status gst = gb_drive_phases(prog, PS_AHEAD, st, [&](uint32_t k) {
+    hipLaunchKernelGGL(ps_iter_kernel, dim3((unsigned)nb), dim3(PS_BLOCK), 0, st, V, g->rrp,
+                       g->rcol, rows, inv, d_x, (const float *)c[k & 1], c[(k + 1) & 1], part,
+                       done, (int32_t)k, p->max_iter, p->tol, (float)p->damping, prog);
+    return hipGetLastError();
+  });
+  if (gst != GB_OK) {
+    (void)hipStreamSynchronize(st);  // launches before an error end first
+    return gst;
+  }
+  if (res) {
+    *res = gb_pr_result{};
+    res->iterations = (int32_t)prog->phases;
+    res->residual = prog->residual;
+    res->dangling = prog->dangling;
+    res->converged = prog->residual < p->tol ? 1 : 0;
+    res->tiles = (int32_t)nb;
+  }
+  return GB_OK;
+}
+
 // Gather form and shape for a graph.  gb_pr_params.row_block > 0 or GB_PR_RB
 // fix the row-block form; items_per_thread (or GB_PR_IPT) and GB_PR_HOT fix
 // merge-path shapes.  Otherwise the autotuner runs once per graph handle and
@@ -1719,6 +1988,7 @@ extern "C" gb_status gb_pagerank(gb_graph g, const gb_pr_params *p, float *d_x,
     return gb_fail(GB_ERR_INVALID, "gb_pagerank: binned set with row_block or items_per_thread");
   PrShape sh{8, 0, 0, 0};
   GB_TRY(ensure_inv_outdeg(g, gb_stream(stream)));
+  if (small_fits(g, p)) return pagerank_small(g, p, d_x, res, gb_stream(stream));
   GB_TRY(pick_shape(g, p, d_x, stream, &sh));
   return pagerank_run(g, p, d_x, res, stream, sh);
 }

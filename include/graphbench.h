@@ -220,7 +220,9 @@ typedef struct gb_pr_result {
   double gather_ms;      /* summed gather-kernel time (time_kernels=1) */
   int32_t gather_launches;
   int32_t tiles;
-  int32_t items_per_thread; /* merge-path shape used: tile = 256 x items_per_thread */
+  int32_t items_per_thread; /* merge-path shape used: tile = 256 x items_per_thread;
+                               0 with row_block and binned 0: the form of small
+                               graphs, one launch per iteration */
   int32_t hot;              /* sources served from LDS (0 = none) */
   int32_t relabeled;        /* 1 if the gather ran in out-degree order */
   int32_t row_block;        /* row-block form used: edges per block (0 = merge path) */
