@@ -119,9 +119,9 @@ struct gb_graph_s {
     bool valid = false, relabeled = false;
     int32_t hub = 0, csl = 0, bsl = 0;  // hub chunk width, log2 chunk / bin widths
     int32_t piece = 0;                  // entries per accumulation piece at most
-    int64_t padded = 0;                   // stream entries (segments padded to 4)
-    int64_t ntasks = 0, nunits = 0, npieces = 0, nmulti = 0;
-    DevBuf src16, dst16, vals, tasks, units, pieces, multi, sum64;
+    int64_t padded = 0;                 // edge places (with padding)
+    int64_t nunits = 0, npieces = 0, nmulti = 0;
+    DevBuf src16, out4, dst16, before, vals, units, pieces, multi, sum64;
   } pr_pb;
   // PageRank relabelling: vertices renumbered by out-degree (descending), the
   // in-CSR and 1/outdeg in the new numbering (gb_graph_pr_relabel)

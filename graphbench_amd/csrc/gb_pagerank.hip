@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 
 #include <hipcub/device/device_radix_sort.hpp>
+#include <hipcub/device/device_scan.hpp>
 
 #include <algorithm>
 #include <cmath>
@@ -999,43 +1000,59 @@ __global__ __launch_bounds__(PR_BLOCK) void pr_rb_fixup_kernel(
 // (propagation blocking) streams instead.  Sources are cut into a hub chunk
 // (chunk 0: the first HUB ids, the highest out-degrees once relabelled)
 // and chunks of 2^CSL ids after it, destinations into bins of 2^BSL ids; the
-// edges of each (chunk, bin) pair form a segment, padded to a multiple of 4
-// entries.
-//   pb_scatter  one block per unit (a run of one chunk's segments): the
-//               chunk's contributions are copied into LDS, then each wave
-//               task (<= 256 entries of one segment) reads 4 u16 local source
-//               ids per lane and writes the 4 contributions to the value
+// edges of each (chunk, bin) pair form a segment, sorted by (source,
+// destination).  A source's contribution goes to a bin once, however many of
+// its edges end there: on R-MAT 22 the 67 M edges need 14.9 M values (58% of
+// the edges leave the hub chunk's 16384 sources, and those share a value by
+// 2.6 on average).
+//   pb_scatter  one block per unit (a run of one chunk's values): the chunk's
+//               contributions are copied into LDS, then a lane reads 4 u16
+//               local source ids and the place of their 4 values in the value
 //               stream, where segments lie in (bin, chunk) order.
-//   pb_accum    one block per piece (a run of one bin's stream): 4 values and
-//               4 u16 local destination ids per lane, added into 2^BSL int64
-//               LDS accumulators.  A bin held by one piece finishes its rows
-//               in the block; a bin split over several pieces adds its sums
-//               to sum64 with integer atomics and
-//   pb_fixup    finishes those rows, sums the per-wave residual and dangling
-//               partials and sets the next base and stop flag (as the other
-//               forms' fix-ups do).
+//   pb_accum    one block per piece (a run of one bin's edges): 4 u16 local
+//               destination ids per lane, added into 2^BSL int64 LDS
+//               accumulators.  Bit 15 of an id says that its edge starts the
+//               next value: a wave's 256 edges count those bits with ballots
+//               from the number before them (one per 256 edges), which gives
+//               every edge the index of its value.  A bin held by one piece
+//               finishes its rows in the block; a bin split over several
+//               pieces adds its sums to sum64 with integer atomics and
+//   pb_rows     finishes those rows.
+//   pb_fix      sums the residual and dangling partials and sets the next base
+//               and stop flag.
 // Sums are fixed point (value * 2^fx_shift, rounded to nearest, int64), so
 // the order of the LDS and global atomics changes nothing: results are
 // run-to-run identical, and each row sum is exact up to one rounding per
 // edge of 2^-51 of the mass bound (2^-51 for ranks summing to 1) and the
 // final rounding to FP32.
-constexpr int PB_TASK = 256;  // stream entries per wave task, 4 per lane
+// What bounds it (R-MAT 22, hub 16384, bins of 8192; per iteration): the
+// scatter moves 10 bytes a value and takes 26.7 us; it took 64 us when every
+// edge had a value of its own (8 bytes an edge).  The accumulation takes 73 us
+// (91 us with a value per edge): 22 us are its fixed part (hub copy, clear and
+// row ends by 2.5 rounds of one 131 KB block per CU), the rest is the 2-byte
+// ids, the values and one LDS add per edge in about equal parts, behind the
+// latency of 16 waves per CU.  A solve of 20 iterations: 3.49 -> 2.36 ms; R-MAT
+// 24 warm: 12.8 -> 8.6 ms.  With few shared values (uniform graph, 2 M
+// vertices, 32 M edges: 1.02 edges a value) 1341 -> 1250 us.  Pieces of 192 K
+// edges 2386 us, 256 K 2316, 384 K 2508; units of 8 K to 64 K values are level.
+constexpr int PB_BATCH = 256;  // edges per wave batch, 4 per lane
 constexpr int PB_SCATTER_BLOCK = 512;
 constexpr int PB_ACCUM_BLOCK = 1024;
 constexpr int PB_ACCUM_WAVES = PB_ACCUM_BLOCK / GB_WAVE;
-constexpr uint16_t PB_PAD = 0xFFFF;  // padding entry of the source stream
-constexpr int PB_ALIGN = 4;          // segments padded to a multiple of this many entries
+constexpr int PB_SCATTER_QUADS = 4;  // quads of values in flight per thread
+constexpr int64_t PB_UNIT = 32768;    // values per scatter unit at most
+// Destination ids: bit 15, the edge starts the next value; id 2^BSL, one past
+// the bin, is padding (which may start a value too: segments take a multiple of
+// 4 values) and is added into a place of its own, so that no edge needs a test.
+constexpr uint32_t PB_FIRST = 0x8000;
 
-struct PbTask {
-  int32_t in0, out0, n;  // n entries (multiple of 4) at src16[in0..], vals[out0..]
-};
 struct PbUnit {
-  int32_t src0, t0, t1;  // chunk's first source, tasks [t0, t1)
+  int32_t src0, q0, q1;  // chunk's first source, quads (4 values) [q0, q1)
 };
-// Stream entries [e0, e1) of bin; multi: the bin is split over pieces.  The
-// bin's first segment (the hub chunk's edges) ends at hub_e1 and is read from
-// src16 at e + hub_off: its contributions come from an LDS copy, the scatter
-// skips the hub chunk.
+// Edges [e0, e1) (multiples of PB_BATCH) of bin; multi: the bin is split over
+// pieces.  The bin's first segment (the hub chunk's edges) ends at hub_e1: its
+// value i is the contribution of hub source src16[i + hub_off], from an LDS
+// copy; the scatter skips the hub chunk.
 struct PbPiece {
   int32_t bin, e0, e1, multi, hub_e1, hub_off;
 };
@@ -1044,15 +1061,11 @@ typedef float pb_f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ pb_u32x2 pb_ids4(const uint16_t *p) {
   return __builtin_nontemporal_load(reinterpret_cast<const pb_u32x2 *>(p));
 }
-__device__ __forceinline__ pb_f32x4 pb_vals4(const float *p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const pb_f32x4 *>(p));
-}
-
 // round(v * scale) as int64 (nearest, ties to even), scale a power of two
 // with |v| * scale < 2^51: the product is exact in FP64, and adding 1.5 * 2^52
 // leaves the rounded integer in the low mantissa bits.
 __device__ __forceinline__ long long pb_fixed(float v, double scale) {
-  const double y = (double)v * scale + 6755399441055744.0;
+  const double y = fma((double)v, scale, 6755399441055744.0);  // as exact as mul and add
   return __double_as_longlong(y) - 0x4338000000000000LL;
 }
 
@@ -1060,15 +1073,14 @@ __device__ __forceinline__ float pb_value(unsigned long long a, int S) {
   return (float)ldexp((double)(long long)a, -S);
 }
 
-// contributions of 4 local source ids (padding ids, >= CS, give 0)
-template <int CS>
+// contributions of 4 local source ids (padding holds id 0: its value is not
+// added to any row)
 __device__ __forceinline__ pb_f32x4 pb_lookup4(const float *s_c, pb_u32x2 s) {
-  const uint32_t i0 = s.x & 0xFFFFu, i1 = s.x >> 16, i2 = s.y & 0xFFFFu, i3 = s.y >> 16;
   pb_f32x4 o;
-  o.x = i0 < (uint32_t)CS ? s_c[i0] : 0.0f;
-  o.y = i1 < (uint32_t)CS ? s_c[i1] : 0.0f;
-  o.z = i2 < (uint32_t)CS ? s_c[i2] : 0.0f;
-  o.w = i3 < (uint32_t)CS ? s_c[i3] : 0.0f;
+  o.x = s_c[s.x & 0xFFFFu];
+  o.y = s_c[s.x >> 16];
+  o.z = s_c[s.y & 0xFFFFu];
+  o.w = s_c[s.y >> 16];
   return o;
 }
 
@@ -1121,36 +1133,25 @@ __global__ __launch_bounds__(PB_SCATTER_BLOCK) void pb_fix_kernel(
 // done after the last iteration is only wasted work, and at most one is.
 template <int CSL>
 __global__ __launch_bounds__(PB_SCATTER_BLOCK) void pb_scatter_kernel(
-    const PbUnit *__restrict__ units, const PbTask *__restrict__ tasks,
-    const uint16_t *__restrict__ src16, const float *__restrict__ contrib,
+    const PbUnit *__restrict__ units, const uint16_t *__restrict__ src16,
+    const uint32_t *__restrict__ out4, const float *__restrict__ contrib,
     float *__restrict__ vals, int fold, int64_t nparts, const double *__restrict__ p_res,
     const double *__restrict__ p_dang, PrState *st) {
   constexpr int CS = 1 << CSL;
   constexpr int PER = CS / PB_SCATTER_BLOCK;
-  constexpr int WAVES = PB_SCATTER_BLOCK / GB_WAVE;
   __shared__ float s_c[CS];
   if (fold && blockIdx.x == 0) {
-    __shared__ double s_red[WAVES];
+    __shared__ double s_red[PB_SCATTER_BLOCK / GB_WAVE];
     if (st->done) return;
     pb_fix_block<2>(nparts, p_res, p_dang, st, s_red);  // few registers: the scatter's occupancy
     return;
   }
   if (__hip_atomic_load(&st->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
   const PbUnit u = units[blockIdx.x - fold];
-  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / GB_WAVE);
-  const int lane = gb_lane(), l4 = lane * 4;
-  // waves take R consecutive tasks in turn (wave w: tasks t0 + w * R + k *
-  // WAVES * R), so a unit's tasks spread over all its waves; a round's R
-  // descriptors come one per lane, loaded during the round before, and its R
-  // id loads are in flight together.  The first round's descriptors and ids
-  // load together with the chunk's contributions.
-  constexpr int R = 16;
-  constexpr int32_t STRIDE = WAVES * R;
-  int32_t base = u.t0 + wave * R;
-  PbTask my = {0, 0, 0};
-  if (lane < R && base + lane < u.t1) my = tasks[base + lane];
+  // a round's R quads per thread are in flight together, the first round's with
   // the chunk's contributions (the last chunk may be short: clamped reads,
   // entries past it are never indexed)
+  constexpr int R = PB_SCATTER_QUADS;
   const int32_t nsrc = min(CS, st->V - u.src0);
   float c[PER];
 #pragma unroll
@@ -1158,67 +1159,97 @@ __global__ __launch_bounds__(PB_SCATTER_BLOCK) void pb_scatter_kernel(
     const int k = (int)threadIdx.x + j * PB_SCATTER_BLOCK;
     c[j] = contrib[u.src0 + (k < nsrc ? k : nsrc - 1)];
   }
-  int32_t in0[R], out0[R], n[R];
   pb_u32x2 ids[R];
-  auto decode_and_load = [&](int nt) {
+  uint32_t to[R];
+  auto load = [&](int32_t q) {
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-      n[k] = k < nt ? __builtin_amdgcn_readlane(my.n, k) : 0;
-      in0[k] = __builtin_amdgcn_readlane(my.in0, k);
-      out0[k] = __builtin_amdgcn_readlane(my.out0, k);
+      const int32_t i = min(q + k * PB_SCATTER_BLOCK, u.q1 - 1);
+      ids[k] = pb_ids4(src16 + 4 * (int64_t)i);
+      to[k] = __builtin_nontemporal_load(out4 + i);
     }
-#pragma unroll
-    for (int k = 0; k < R; ++k)
-      if (l4 < n[k]) ids[k] = pb_ids4(src16 + in0[k] + l4);
   };
-  if (base < u.t1) decode_and_load(min(R, u.t1 - base));
+  int32_t q = u.q0 + (int32_t)threadIdx.x;
+  load(q);  // u.q0 < u.q1
 #pragma unroll
   for (int j = 0; j < PER; ++j) s_c[threadIdx.x + j * PB_SCATTER_BLOCK] = c[j];
   __syncthreads();
-  for (bool first = true; base < u.t1; base += STRIDE, first = false) {
-    PbTask nx = {0, 0, 0};
-    if (lane < R && base + STRIDE + lane < u.t1) nx = tasks[base + STRIDE + lane];
-    if (!first) decode_and_load(min(R, u.t1 - base));
+  while (q < u.q1) {
 #pragma unroll
     for (int k = 0; k < R; ++k)
-      if (l4 < n[k])
-        *reinterpret_cast<pb_f32x4 *>(vals + out0[k] + l4) = pb_lookup4<CS>(s_c, ids[k]);
-    my = nx;
+      if (q + k * PB_SCATTER_BLOCK < u.q1)
+        *reinterpret_cast<pb_f32x4 *>(vals + 4 * (int64_t)to[k]) = pb_lookup4(s_c, ids[k]);
+    q += R * PB_SCATTER_BLOCK;
+    if (q < u.q1) load(q);
   }
 }
 
+// Whether this lane's 4 edges start a value, and the first one's value counted
+// from 1 (0: the last one before): n, the values started before the wave's 256
+// edges.
+__device__ __forceinline__ uint32_t pb_index4(pb_u32x2 d, uint32_t n, bool (&f)[4]) {
+  f[0] = (d.x & PB_FIRST) != 0u;
+  f[1] = (int32_t)d.x < 0;
+  f[2] = (d.y & PB_FIRST) != 0u;
+  f[3] = (int32_t)d.y < 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {  // started by lower lanes
+    const uint64_t b = __ballot(f[k]);
+    n = __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32),
+                                  __builtin_amdgcn_mbcnt_lo((uint32_t)b, n));
+  }
+  return n + (f[0] ? 1u : 0u);
+}
+
+// The 4 edges' values out of the 4 consecutive ones from the first edge's on:
+// an edge that starts a value moves on by one.
+__device__ __forceinline__ void pb_pick4(const bool (&f)[4], float (&v)[4]) {
+  float w0 = v[0], w1 = v[1], w2 = v[2], w3 = v[3];
+#pragma unroll
+  for (int k = 1; k < 4; ++k) {
+    w0 = f[k] ? w1 : w0;
+    w1 = f[k] ? w2 : w1;
+    w2 = f[k] ? w3 : w2;
+    v[k] = w0;
+  }
+}
+// 4 consecutive values or ids at any place: one load
+struct __attribute__((packed, aligned(4))) PbVals4 {
+  float v[4];
+};
+struct __attribute__((packed, aligned(2))) PbIds4 {
+  uint16_t v[4];
+};
+
 template <int BSL>
-__device__ __forceinline__ void pb_add4(unsigned long long *s_acc, pb_f32x4 v, pb_u32x2 d,
+__device__ __forceinline__ void pb_add4(unsigned long long *s_acc, const float (&v)[4], pb_u32x2 d,
                                         double scale) {
-  constexpr uint32_t M = (1u << BSL) - 1;
-  const long long f0 = pb_fixed(v.x, scale), f1 = pb_fixed(v.y, scale);
-  const long long f2 = pb_fixed(v.z, scale), f3 = pb_fixed(v.w, scale);
-  if (f0) atomicAdd(&s_acc[d.x & M], (unsigned long long)f0);
-  if (f1) atomicAdd(&s_acc[(d.x >> 16) & M], (unsigned long long)f1);
-  if (f2) atomicAdd(&s_acc[d.y & M], (unsigned long long)f2);
-  if (f3) atomicAdd(&s_acc[(d.y >> 16) & M], (unsigned long long)f3);
+  constexpr uint32_t M = (2u << BSL) - 1;  // the padding place included
+  const uint32_t id[4] = {d.x & M, (d.x >> 16) & M, d.y & M, (d.y >> 16) & M};
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    atomicAdd(&s_acc[id[k]], (unsigned long long)pb_fixed(v[k], scale));
 }
 
 template <int HUB, int BSL>
 __global__ __launch_bounds__(PB_ACCUM_BLOCK) void pb_accum_kernel(
     const PbPiece *__restrict__ pieces, const float *__restrict__ vals,
     const uint16_t *__restrict__ src16, const uint16_t *__restrict__ dst16,
-    const float *__restrict__ contrib, RowOut out, unsigned long long *__restrict__ sum64,
-    double *__restrict__ part_res, double *__restrict__ part_dang,
-    const PrState *__restrict__ st) {
+    const uint32_t *__restrict__ before, const float *__restrict__ contrib, RowOut out,
+    unsigned long long *__restrict__ sum64, double *__restrict__ part_res,
+    double *__restrict__ part_dang, const PrState *__restrict__ st) {
   constexpr int BS = 1 << BSL;
   constexpr int CS = HUB;  // hub chunk width (a multiple of the block size)
   static_assert(HUB % PB_ACCUM_BLOCK == 0, "hub chunk width");
-  constexpr int STEP = PB_ACCUM_BLOCK * 4;
-  constexpr int U = 4;  // batches of loads in flight per thread
-  __shared__ unsigned long long s_acc[BS];
+  constexpr int U = 4;  // batches in flight per wave
+  __shared__ unsigned long long s_acc[BS + 1];
   __shared__ float s_hot[CS];
   if (st->done) return;
   out.base = st->base;
   const int S = st->fx_shift;
   const double scale = ldexp(1.0, S);
   const PbPiece pc = pieces[blockIdx.x];
-  const int32_t he = min(pc.e1, pc.hub_e1);  // chunk-0 entries of the piece: [e0, he)
+  const int32_t he = min(pc.e1, pc.hub_e1);  // hub edges of the piece: [e0, he)
   // the hub copy's loads go out first, the accumulators are cleared while
   // they are in flight
   constexpr int PER = CS / PB_ACCUM_BLOCK;
@@ -1238,35 +1269,78 @@ __global__ __launch_bounds__(PB_ACCUM_BLOCK) void pb_accum_kernel(
     for (int j = 0; j < PER; ++j) s_hot[threadIdx.x + j * PB_ACCUM_BLOCK] = c[j];
   }
   __syncthreads();
-  // e0, e1, hub_e1 and every e are multiples of 4
-  int32_t e = pc.e0 + (int32_t)threadIdx.x * 4;
-  for (; e + (U - 1) * STEP < he; e += U * STEP) {
-    pb_u32x2 q[U], d[U];
+  // batches of 256 edges, dealt to the waves in turn; before[b]: the values
+  // started before batch b.  Bases one before the piece's first value, so that
+  // a value is an unsigned 32-bit offset away.
+  const uint32_t pv = before[pc.e0 / PB_BATCH];
+  const uint16_t *hub_src = src16 + ((int64_t)pc.hub_off + pv - 1);
+  const float *pvals = vals + ((int64_t)pv - 1);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / GB_WAVE);
+  const int l4 = gb_lane() * 4;
+  auto batches = [&](int32_t b0, int32_t b1, auto value) {
+    const int32_t bw = b0 + wave;
+    const int32_t all = bw < b1 ? (b1 - bw + PB_ACCUM_WAVES - 1) / PB_ACCUM_WAVES : 0;
+    for (int32_t j0 = 0; j0 < all; j0 += GB_WAVE) {
+      // the wave's next (at most) 64 batches; lane j holds the count of batch j:
+      // a scalar load per batch would wait for the LDS adds in flight
+      const int32_t n = min(GB_WAVE, all - j0);
+      const int32_t first = bw + j0 * PB_ACCUM_WAVES;
+      const uint32_t counts =
+          before[first + min(gb_lane(), n - 1) * PB_ACCUM_WAVES] - pv;
+      const uint16_t *ids = dst16 + (int64_t)first * PB_BATCH + l4;
+      auto load = [&](int32_t j) {
+        return pb_ids4(ids + (uint32_t)(min(j, n - 1) * (PB_ACCUM_WAVES * PB_BATCH)));
+      };
+      pb_u32x2 nx[U];
 #pragma unroll
-    for (int k = 0; k < U; ++k) {
-      q[k] = pb_ids4(src16 + pc.hub_off + e + k * STEP);
-      d[k] = pb_ids4(dst16 + e + k * STEP);
+      for (int k = 0; k < U; ++k) nx[k] = load(k);
+      for (int32_t j = 0; j < n; j += U) {
+        pb_u32x2 d[U];
+        float v[U][4];
+        bool f[U][4];
+        uint32_t i[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+          d[k] = nx[k];
+          i[k] = pb_index4(d[k], __builtin_amdgcn_readlane(counts, min(j + k, n - 1)), f[k]);
+        }
+        // the next batches' ids load while this one's values do
+        if (j + U < n) {
+#pragma unroll
+          for (int k = 0; k < U; ++k) nx[k] = load(j + U + k);
+        }
+        value(i, v);
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+          if (j + k < n) {
+            pb_pick4(f[k], v[k]);
+            pb_add4<BSL>(s_acc, v[k], d[k], scale);
+          }
+      }
     }
+  };
+  // One load per lane for its 4 edges' values: they lie within the 4 from the
+  // first one's on (a load per edge had kept the address units busy for 20 us of
+  // an R-MAT 22 iteration).  32-bit byte offsets from a uniform base.
+  batches(pc.e0 / PB_BATCH, he / PB_BATCH, [&](const uint32_t (&i)[U], float (&v)[U][4]) {
+    PbIds4 q[U];
 #pragma unroll
-    for (int k = 0; k < U; ++k) pb_add4<BSL>(s_acc, pb_lookup4<CS>(s_hot, q[k]), d[k], scale);
-  }
-  for (; e < he; e += STEP)
-    pb_add4<BSL>(s_acc, pb_lookup4<CS>(s_hot, pb_ids4(src16 + pc.hub_off + e)),
-                 pb_ids4(dst16 + e), scale);
-  e = max(pc.e0, pc.hub_e1) + (int32_t)threadIdx.x * 4;
-  for (; e + (U - 1) * STEP < pc.e1; e += U * STEP) {
-    pb_f32x4 v[U];
-    pb_u32x2 d[U];
+    for (int k = 0; k < U; ++k) q[k] = *(const PbIds4 *)((const char *)hub_src + i[k] * 2u);
+    // ids past the hub's list are another list's, below the chunk width <= HUB
 #pragma unroll
-    for (int k = 0; k < U; ++k) {
-      v[k] = pb_vals4(vals + e + k * STEP);
-      d[k] = pb_ids4(dst16 + e + k * STEP);
-    }
+    for (int k = 0; k < U; ++k)
 #pragma unroll
-    for (int k = 0; k < U; ++k) pb_add4<BSL>(s_acc, v[k], d[k], scale);
-  }
-  for (; e < pc.e1; e += STEP)
-    pb_add4<BSL>(s_acc, pb_vals4(vals + e), pb_ids4(dst16 + e), scale);
+      for (int m = 0; m < 4; ++m) v[k][m] = s_hot[q[k].v[m]];
+  });
+  batches(max(pc.e0, pc.hub_e1) / PB_BATCH, pc.e1 / PB_BATCH,
+          [&](const uint32_t (&i)[U], float (&v)[U][4]) {
+#pragma unroll
+            for (int k = 0; k < U; ++k) {
+              const PbVals4 q = *(const PbVals4 *)((const char *)pvals + i[k] * 4u);
+#pragma unroll
+              for (int m = 0; m < 4; ++m) v[k][m] = q.v[m];
+            }
+          });
   __syncthreads();
   const int32_t v0 = pc.bin << BSL;
   const int32_t nv = min(BS, st->V - v0);
@@ -1378,23 +1452,78 @@ __global__ void pb_first_kernel(int64_t E, const uint64_t *__restrict__ keys, in
   if (head) first[seg] = (int32_t)k;
 }
 
-// Sorted edge k of segment (b, c) goes to src16[k + d1[seg]] (chunk-major
-// order) and dst16[k + d2[seg]] (bin-major order) as local ids.
+// start[k] = 1 where sorted edge k has another (bin, source) than the one
+// before: it starts a value.
+__global__ void pb_start_kernel(int64_t E, const uint64_t *__restrict__ keys,
+                                int32_t *__restrict__ start) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < E) start[k] = k == 0 || keys[k] != keys[k - 1] ? 1 : 0;
+}
+
+// rank of every segment's first value (rank: inclusive sums of start)
+__global__ void pb_first_rank_kernel(int64_t nseg, const int32_t *__restrict__ first,
+                                     const int32_t *__restrict__ rank,
+                                     int32_t *__restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < nseg) out[i] = first[i] >= 0 ? rank[first[i]] - 1 : -1;
+}
+
+// Per segment: where its edges and values go relative to their sorted index
+// and rank, and its padding.
+struct PbSeg {
+  int32_t edge;      // dst16 place minus sorted index
+  int32_t vsrc;      // src16 place (chunk-major) minus value rank
+  int32_t vout;      // value place (bin-major) minus value rank
+  int32_t pad0;      // dst16 place of the padding that starts values
+  int32_t npad;      // how many
+};
+
 __global__ void pb_place_kernel(int64_t E, const uint64_t *__restrict__ keys,
-                                const int32_t *__restrict__ vs, int vbits, int hub, int csl,
-                                int bsl,
-                                int64_t nchunks, const int32_t *__restrict__ d1,
-                                const int32_t *__restrict__ d2, uint16_t *__restrict__ src16,
-                                uint16_t *__restrict__ dst16) {
+                                const int32_t *__restrict__ vs, const int32_t *__restrict__ rank,
+                                int vbits, int hub, int csl, int bsl, int64_t nchunks,
+                                const PbSeg *__restrict__ segs, uint16_t *__restrict__ src16,
+                                uint32_t *__restrict__ out4, uint16_t *__restrict__ dst16) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= E) return;
   const uint64_t key = keys[k];
   const int32_t b = (int32_t)(key >> vbits);
   const int32_t u = (int32_t)(key & ((1ull << vbits) - 1));
   const int32_t c = pb_chunk(u, hub, csl);
-  const int64_t seg = (int64_t)b * nchunks + c;
-  src16[k + d1[seg]] = (uint16_t)(u - pb_chunk_base(c, hub, csl));
-  dst16[k + d2[seg]] = (uint16_t)(vs[k] - (b << bsl));
+  const PbSeg g = segs[(int64_t)b * nchunks + c];
+  const int32_t r = rank[k] - 1;
+  const bool first = k == 0 || rank[k - 1] - 1 != r;
+  dst16[k + g.edge] = (uint16_t)((vs[k] - (b << bsl)) | (first ? PB_FIRST : 0u));
+  if (first) {
+    const int32_t at = r + g.vsrc;
+    src16[at] = (uint16_t)(u - pb_chunk_base(c, hub, csl));
+    if (at % 4 == 0) out4[at / 4] = (uint32_t)(r + g.vout) / 4u;
+  }
+}
+
+// All ids to n copies of v (8 per thread)
+__global__ void pb_fill16_kernel(int64_t n, uint16_t v, uint16_t *__restrict__ a) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    a[i] = v;
+}
+
+__global__ void pb_pad_kernel(int64_t nseg, int bsl, const PbSeg *__restrict__ segs,
+                              uint16_t *__restrict__ dst16) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nseg) return;
+  const PbSeg g = segs[i];
+  for (int32_t k = 0; k < g.npad; k++) dst16[g.pad0 + k] = (uint16_t)(PB_FIRST | 1u << bsl);
+}
+
+// values started in each batch, one wave per batch
+__global__ void pb_count_kernel(int64_t nbatches, const uint16_t *__restrict__ dst16,
+                                uint32_t *__restrict__ count) {
+  const int64_t b = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / GB_WAVE;
+  if (b >= nbatches) return;
+  uint32_t n = 0;
+  for (int k = 0; k < PB_BATCH / GB_WAVE; k++)
+    n += (uint32_t)__popcll(__ballot(dst16[b * PB_BATCH + k * GB_WAVE + gb_lane()] & PB_FIRST));
+  if (gb_lane() == 0) count[b] = n;
 }
 
 // Row blocks of an in-CSR (host side; irp copied from the device).
@@ -1596,14 +1725,15 @@ static gb_status ensure_inv_outdeg(gb_graph g, hipStream_t st) {
 
 // Binned layout of the gather's in-CSR (irp, icol) for a hub chunk of hub
 // sources, chunks of 2^csl sources after it and bins of 2^bsl destinations,
-// cached on the handle.  Edges are
-// sorted by (bin, source) with a stable radix sort (in-CSR order, so by
-// destination, among equal keys); each (bin, chunk) segment is padded to a
-// multiple of 4 entries.  Host side: segment offsets in both orders, wave
-// tasks (<= 256 entries of one segment), units (runs of one chunk's tasks of
-// about `unit` entries: one scatter block each) and pieces (runs of a bin's
-// stream of at most `piece` entries: one accumulation block each; largest
-// first, so that the block scheduler hands out the long ones first).
+// cached on the handle.  Edges are sorted by (bin, source) with a stable radix
+// sort (in-CSR order, so by destination, among equal keys); equal keys share a
+// value.  Host side: the segments' places in both orders, units (runs of one
+// chunk's values of at most `unit`: one scatter block each) and pieces (runs
+// of a bin's edges of at most `piece`: one accumulation block each; largest
+// first, so that the block scheduler hands out the long ones first).  A
+// segment's values take a multiple of 4 places in both orders, padding edges
+// that start a value stand for the rest, and its edges take a multiple of 4; a
+// hub segment and a bin take whole batches.
 static gb_status pb_build(gb_graph g, bool relabel, const int32_t *irp, const int32_t *icol,
                           int hub, int csl, int bsl, int piece, hipStream_t st) {
   gb_graph_s::PrBinned &L = g->pr_pb;
@@ -1617,16 +1747,16 @@ static gb_status pb_build(gb_graph g, bool relabel, const int32_t *irp, const in
       1 + (V > hub ? (((int64_t)V - hub + (1 << csl) - 1) >> csl) : 0);
   const int64_t nbins = ((int64_t)V + (1 << bsl) - 1) >> bsl;
   const int64_t nseg = nchunks * nbins;
-  if (nseg > ((int64_t)1 << 26) ||
-      E + (PB_ALIGN - 1) * std::min<int64_t>(nseg, E) > INT32_MAX - PB_ALIGN)
+  if (nseg > ((int64_t)1 << 26))
     return gb_fail(GB_ERR_UNSUPPORTED, "gb_pagerank: graph too large for the binned form");
   int vbits = 1;
   while (((int64_t)1 << vbits) < V) vbits++;
   int bbits = 1;
   while (((int64_t)1 << bbits) < nbins) bbits++;
   // sorted (bin, source) keys and destinations
-  std::vector<int32_t> first((size_t)nseg, -1);
-  DevBuf keys, keys2, vs, vs2, dfirst, tmp;
+  std::vector<int32_t> first((size_t)nseg, -1), frank((size_t)nseg, -1);
+  int32_t values = 0;  // of all segments
+  DevBuf keys, keys2, vs, vs2, dfirst, dfrank, rank, tmp;
   if (E > 0) {
     GB_TRY(keys.ensure(sizeof(uint64_t) * E));
     GB_TRY(keys2.ensure(sizeof(uint64_t) * E));
@@ -1651,112 +1781,137 @@ static gb_status pb_build(gb_graph g, bool relabel, const int32_t *irp, const in
     GB_HIP(hipMemsetAsync(dfirst.p, 0xFF, sizeof(int32_t) * nseg, st));
     hipLaunchKernelGGL(pb_first_kernel, dim3(eb), dim3(256), 0, st, E, keys2.as<uint64_t>(),
                        vbits, hub, csl, nchunks, dfirst.as<int32_t>());
+    // value ranks: inclusive sums of the value starts
+    DevBuf start;
+    GB_TRY(start.ensure(sizeof(int32_t) * E));
+    GB_TRY(rank.ensure(sizeof(int32_t) * E));
+    GB_TRY(dfrank.ensure(sizeof(int32_t) * nseg));
+    hipLaunchKernelGGL(pb_start_kernel, dim3(eb), dim3(256), 0, st, E, keys2.as<uint64_t>(),
+                       start.as<int32_t>());
+    size_t ts = 0;
+    GB_HIP(hipcub::DeviceScan::InclusiveSum(nullptr, ts, start.as<int32_t>(), rank.as<int32_t>(),
+                                            (int)E, st));
+    GB_TRY(tmp.ensure(ts));
+    GB_HIP(hipcub::DeviceScan::InclusiveSum(tmp.p, ts, start.as<int32_t>(), rank.as<int32_t>(),
+                                            (int)E, st));
+    hipLaunchKernelGGL(pb_first_rank_kernel, dim3((unsigned)((nseg + 255) / 256)), dim3(256), 0,
+                       st, nseg, dfirst.as<int32_t>(), rank.as<int32_t>(), dfrank.as<int32_t>());
     GB_HIP(hipMemcpyAsync(first.data(), dfirst.p, sizeof(int32_t) * nseg, hipMemcpyDeviceToHost,
                           st));
+    GB_HIP(hipMemcpyAsync(frank.data(), dfrank.p, sizeof(int32_t) * nseg, hipMemcpyDeviceToHost,
+                          st));
+    GB_HIP(hipMemcpyAsync(&values, rank.as<int32_t>() + (E - 1), sizeof(int32_t),
+                          hipMemcpyDeviceToHost, st));
     GB_HIP(hipStreamSynchronize(st));
   }
-  // segment sizes (bin-major = sorted order), padded sizes and offsets
-  std::vector<int32_t> cnt((size_t)nseg, 0);
+  // segment sizes in edges and values (bin-major = sorted order)
+  std::vector<int32_t> cnt((size_t)nseg, 0), vcnt((size_t)nseg, 0);
   {
     int64_t next = E;
+    int32_t vnext = values;
     for (int64_t i = nseg - 1; i >= 0; --i)
       if (first[i] >= 0) {
         cnt[i] = (int32_t)(next - first[i]);
+        vcnt[i] = vnext - frank[i];
         next = first[i];
+        vnext = frank[i];
       }
   }
-  auto pad4 = [](int64_t n) { return (n + 3) & ~(int64_t)3; };
-  auto padseg = [](int64_t n) { return (n + PB_ALIGN - 1) & ~(int64_t)(PB_ALIGN - 1); };
-  std::vector<int32_t> d1((size_t)nseg), d2((size_t)nseg);
-  std::vector<int32_t> out_start((size_t)nseg);
-  std::vector<int32_t> bin_start((size_t)nbins + 1);
-  int64_t P = 0;
+  auto up = [](int64_t n, int64_t m) { return (n + m - 1) / m * m; };
+  std::vector<PbSeg> segs((size_t)nseg);
+  std::vector<int32_t> bin_start((size_t)nbins + 1), hub_end((size_t)nbins);
+  std::vector<int64_t> hub_v((size_t)nbins);  // first value place of a bin's hub segment
+  int64_t P = 0, PV = 0;                      // edge and value places
   for (int64_t b = 0; b < nbins; ++b) {
     bin_start[b] = (int32_t)P;
+    hub_v[b] = PV;
     for (int64_t c = 0; c < nchunks; ++c) {
       const int64_t i = b * nchunks + c;
-      out_start[i] = (int32_t)P;
-      d2[i] = (int32_t)(P - (first[i] >= 0 ? first[i] : 0));
-      P += padseg(cnt[i]);
+      const int64_t mv = up(vcnt[i], 4);
+      segs[i].edge = first[i] >= 0 ? (int32_t)(P - first[i]) : 0;
+      segs[i].vout = first[i] >= 0 ? (int32_t)(PV - frank[i]) : 0;
+      segs[i].pad0 = (int32_t)(P + cnt[i]);
+      segs[i].npad = (int32_t)(mv - vcnt[i]);
+      PV += mv;
+      P = up(P + cnt[i] + segs[i].npad, c == 0 || c + 1 == nchunks ? PB_BATCH : 4);
+      if (c == 0) hub_end[b] = (int32_t)P;
+      if (P > INT32_MAX - PB_BATCH)
+        return gb_fail(GB_ERR_UNSUPPORTED, "gb_pagerank: graph too large for the binned form");
     }
   }
   bin_start[nbins] = (int32_t)P;
-  std::vector<PbTask> tasks;
   std::vector<PbUnit> units;
-  const int64_t unit = 65536;
-  std::vector<int32_t> hub_in((size_t)nbins);  // chunk-major offset of segment (0, b)
+  std::vector<int32_t> hub_off((size_t)nbins);
   {
+    const int64_t unit = PB_UNIT / 4;  // quads
     int64_t in = 0;
     for (int64_t c = 0; c < nchunks; ++c) {
-      int32_t ut0 = (int32_t)tasks.size();
-      int64_t ue = 0;
+      const int64_t q0 = in / 4;
       for (int64_t b = 0; b < nbins; ++b) {
         const int64_t i = b * nchunks + c;
-        d1[i] = (int32_t)(in - (first[i] >= 0 ? first[i] : 0));
-        const int64_t n = padseg(cnt[i]);
-        if (c == 0) {  // read by pb_accum from src16, no scatter
-          hub_in[b] = (int32_t)in;
-          in += n;
-          continue;
-        }
-        for (int64_t j = 0; j < n; j += PB_TASK) {
-          tasks.push_back(PbTask{(int32_t)(in + j), (int32_t)(out_start[i] + j),
-                                 (int32_t)std::min<int64_t>(PB_TASK, n - j)});
-          ue += std::min<int64_t>(PB_TASK, n - j);
-          if (ue >= unit) {
-            units.push_back(PbUnit{pb_chunk_base((int32_t)c, hub, csl), ut0, (int32_t)tasks.size()});
-            ut0 = (int32_t)tasks.size();
-            ue = 0;
-          }
-        }
-        in += n;
+        segs[i].vsrc = first[i] >= 0 ? (int32_t)(in - frank[i]) : 0;
+        if (c == 0) hub_off[b] = (int32_t)(in - hub_v[b]);
+        in += up(vcnt[i], 4);
       }
-      if ((int32_t)tasks.size() > ut0)
-        units.push_back(PbUnit{pb_chunk_base((int32_t)c, hub, csl), ut0, (int32_t)tasks.size()});
+      if (c == 0) continue;  // read by pb_accum from src16, no scatter
+      const int64_t q1 = in / 4, k = (q1 - q0 + unit - 1) / unit;
+      for (int64_t j = 0; j < k; ++j)
+        units.push_back(PbUnit{pb_chunk_base((int32_t)c, hub, csl),
+                               (int32_t)(q0 + (q1 - q0) * j / k),
+                               (int32_t)(q0 + (q1 - q0) * (j + 1) / k)});
     }
   }
   std::vector<PbPiece> pieces;
   std::vector<int32_t> multi;
   for (int64_t b = 0; b < nbins; ++b) {
-    const int64_t s = bin_start[b], n = bin_start[b + 1] - s;
-    const int64_t k = std::max<int64_t>(1, (n + piece - 1) / piece);
+    const int64_t s = bin_start[b] / PB_BATCH, n = bin_start[b + 1] / PB_BATCH - s;
+    const int64_t most = std::max(1, piece / PB_BATCH);
+    const int64_t k = std::max<int64_t>(1, (n + most - 1) / most);
     if (k > 1) multi.push_back((int32_t)b);
-    const int32_t hub_e1 = (int32_t)(s + padseg(cnt[b * nchunks]));
     for (int64_t j = 0; j < k; ++j)
-      pieces.push_back(PbPiece{(int32_t)b, (int32_t)(s + pad4(n * j / k)),
-                               (int32_t)(j + 1 == k ? s + n : s + pad4(n * (j + 1) / k)),
-                               k > 1 ? 1 : 0, hub_e1, (int32_t)(hub_in[b] - s)});
+      pieces.push_back(PbPiece{(int32_t)b, (int32_t)((s + n * j / k) * PB_BATCH),
+                               (int32_t)((s + n * (j + 1) / k) * PB_BATCH), k > 1 ? 1 : 0,
+                               hub_end[b], hub_off[b]});
   }
   std::stable_sort(pieces.begin(), pieces.end(), [](const PbPiece &x, const PbPiece &y) {
     return x.e1 - x.e0 > y.e1 - y.e0;
   });
   // device copies
-  GB_TRY(L.src16.ensure(sizeof(uint16_t) * (P + 4)));
+  const int64_t nbatches = P / PB_BATCH;
+  GB_TRY(L.src16.ensure(sizeof(uint16_t) * (PV + 4)));
+  GB_TRY(L.out4.ensure(sizeof(uint32_t) * (PV / 4 + 1)));
   GB_TRY(L.dst16.ensure(sizeof(uint16_t) * (P + 4)));
-  GB_TRY(L.vals.ensure(sizeof(float) * (P + 4)));
-  GB_TRY(L.tasks.ensure(sizeof(PbTask) * (tasks.size() + 1)));
+  GB_TRY(L.before.ensure(sizeof(uint32_t) * (nbatches + 1)));
+  GB_TRY(L.vals.ensure(sizeof(float) * (PV + 4)));
   GB_TRY(L.units.ensure(sizeof(PbUnit) * (units.size() + 1)));
   GB_TRY(L.pieces.ensure(sizeof(PbPiece) * (pieces.size() + 1)));
   GB_TRY(L.multi.ensure(sizeof(int32_t) * (multi.size() + 1)));
   GB_TRY(L.sum64.ensure(sizeof(unsigned long long) * V));
-  GB_HIP(hipMemsetAsync(L.src16.p, 0xFF, sizeof(uint16_t) * (P + 4), st));
-  GB_HIP(hipMemsetAsync(L.dst16.p, 0, sizeof(uint16_t) * (P + 4), st));
+  GB_HIP(hipMemsetAsync(L.src16.p, 0, sizeof(uint16_t) * (PV + 4), st));
+  hipLaunchKernelGGL(pb_fill16_kernel, dim3((unsigned)(gb_num_cus() * 16)), dim3(256), 0, st,
+                     P + 4, (uint16_t)(1u << bsl), L.dst16.as<uint16_t>());
   GB_HIP(hipMemsetAsync(L.sum64.p, 0, sizeof(unsigned long long) * V, st));
   if (E > 0) {
-    DevBuf dd1, dd2;
-    GB_TRY(dd1.ensure(sizeof(int32_t) * nseg));
-    GB_TRY(dd2.ensure(sizeof(int32_t) * nseg));
-    GB_HIP(hipMemcpyAsync(dd1.p, d1.data(), sizeof(int32_t) * nseg, hipMemcpyHostToDevice, st));
-    GB_HIP(hipMemcpyAsync(dd2.p, d2.data(), sizeof(int32_t) * nseg, hipMemcpyHostToDevice, st));
+    DevBuf dsegs, count;
+    GB_TRY(dsegs.ensure(sizeof(PbSeg) * nseg));
+    GB_HIP(hipMemcpyAsync(dsegs.p, segs.data(), sizeof(PbSeg) * nseg, hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(pb_place_kernel, dim3((unsigned)((E + 255) / 256)), dim3(256), 0, st, E,
-                       keys2.as<uint64_t>(), vs2.as<int32_t>(), vbits, hub, csl, bsl, nchunks,
-                       dd1.as<int32_t>(), dd2.as<int32_t>(), L.src16.as<uint16_t>(),
-                       L.dst16.as<uint16_t>());
-    GB_HIP(hipStreamSynchronize(st));  // dd1 / dd2 go out of scope
+                       keys2.as<uint64_t>(), vs2.as<int32_t>(), rank.as<int32_t>(), vbits, hub,
+                       csl, bsl, nchunks, dsegs.as<PbSeg>(), L.src16.as<uint16_t>(),
+                       L.out4.as<uint32_t>(), L.dst16.as<uint16_t>());
+    hipLaunchKernelGGL(pb_pad_kernel, dim3((unsigned)((nseg + 255) / 256)), dim3(256), 0, st, nseg,
+                       bsl, dsegs.as<PbSeg>(), L.dst16.as<uint16_t>());
+    GB_TRY(count.ensure(sizeof(uint32_t) * (nbatches + 1)));
+    hipLaunchKernelGGL(pb_count_kernel, dim3((unsigned)((nbatches + 3) / 4)), dim3(256), 0, st,
+                       nbatches, L.dst16.as<uint16_t>(), count.as<uint32_t>());
+    size_t ts = 0;
+    GB_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, ts, count.as<uint32_t>(),
+                                            L.before.as<uint32_t>(), (int)nbatches, st));
+    GB_TRY(tmp.ensure(ts));
+    GB_HIP(hipcub::DeviceScan::ExclusiveSum(tmp.p, ts, count.as<uint32_t>(),
+                                            L.before.as<uint32_t>(), (int)nbatches, st));
+    GB_HIP(hipStreamSynchronize(st));  // dsegs and count go out of scope
   }
-  if (!tasks.empty())
-    GB_HIP(hipMemcpyAsync(L.tasks.p, tasks.data(), sizeof(PbTask) * tasks.size(),
-                          hipMemcpyHostToDevice, st));
   if (!units.empty())
     GB_HIP(hipMemcpyAsync(L.units.p, units.data(), sizeof(PbUnit) * units.size(),
                           hipMemcpyHostToDevice, st));
@@ -1774,7 +1929,6 @@ static gb_status pb_build(gb_graph g, bool relabel, const int32_t *irp, const in
   L.bsl = bsl;
   L.piece = piece;
   L.padded = P;
-  L.ntasks = (int64_t)tasks.size();
   L.nunits = (int64_t)units.size();
   L.npieces = (int64_t)pieces.size();
   L.nmulti = (int64_t)multi.size();
@@ -2117,8 +2271,8 @@ static gb_status pagerank_run(gb_graph g, const gb_pr_params *p, float *d_x, gb_
                                       : pb_scatter_kernel<13>;
         const int f = fold ? 1 : 0;
         hipLaunchKernelGGL(scatter, dim3((unsigned)PB.nunits + f), dim3(PB_SCATTER_BLOCK), 0,
-                           st, PB.units.as<PbUnit>(), PB.tasks.as<PbTask>(),
-                           PB.src16.as<uint16_t>(), c_old, PB.vals.as<float>(), f, nparts,
+                           st, PB.units.as<PbUnit>(), (const uint16_t *)PB.src16.as<uint16_t>(),
+                           (const uint32_t *)PB.out4.as<uint32_t>(), c_old, PB.vals.as<float>(), f, nparts,
                            (const double *)w.pres.as<double>(),
                            (const double *)w.pdang.as<double>(), state);
       }
@@ -2128,8 +2282,9 @@ static gb_status pagerank_run(gb_graph g, const gb_pr_params *p, float *d_x, gb_
                                      : pb_accum_kernel<8192, 13>;
       hipLaunchKernelGGL(accum, dim3((unsigned)PB.npieces), dim3(PB_ACCUM_BLOCK), 0, st,
                          PB.pieces.as<PbPiece>(), (const float *)PB.vals.as<float>(),
-                         (const uint16_t *)PB.src16.as<uint16_t>(), PB.dst16.as<uint16_t>(),
-                         c_old, out, PB.sum64.as<unsigned long long>(), w.pres.as<double>(),
+                         (const uint16_t *)PB.src16.as<uint16_t>(),
+                         (const uint16_t *)PB.dst16.as<uint16_t>(),
+                         (const uint32_t *)PB.before.as<uint32_t>(), c_old, out, PB.sum64.as<unsigned long long>(), w.pres.as<double>(),
                          w.pdang.as<double>(), state);
       if (ev1) (void)hipEventRecord(ev1, st);
       if (pb_rows > 0)
@@ -2208,7 +2363,7 @@ static gb_status pagerank_run(gb_graph g, const gb_pr_params *p, float *d_x, gb_
         u(irp), u(icol), u(inv), u(trow), u(tedge), u(g->pr_rb.p), u(g->pr_rb_long.p), u(xa),
         u(xb), u(ca), u(cb), u(w.tail.p), u(w.head.p), u(w.pres.p), u(w.pdang.p), u(w.fres.p),
         u(w.fdang.p), u(w.counter.p), u(state), u(L.src16.p), u(L.dst16.p), u(L.vals.p),
-        u(L.tasks.p), u(L.units.p), u(L.pieces.p), u(L.multi.p), u(L.sum64.p),
+        u(L.out4.p), u(L.before.p), u(L.units.p), u(L.pieces.p), u(L.multi.p), u(L.sum64.p),
         (uint64_t)L.nunits, (uint64_t)L.npieces, (uint64_t)L.nmulti, (uint64_t)L.hub,
         (uint64_t)L.csl, (uint64_t)L.bsl};
     if (!w.exec || w.exec_key != key) {
