@@ -43,9 +43,13 @@ def test_hub_chunks(gpu, kind, directed):
     g = gb.Graph.from_host(h, reverse=r) if directed else gb.Graph.from_host(h, need_reverse=False)
     srcs = np.concatenate([np.arange(0, 9), rng.integers(0, V, 80), [V - 1, 0]]).astype(np.int32)
     ref = oracle.brandes_bfs(h.row_ptr, h.col, srcs, r.row_ptr, r.col)
-    for batch in (0, 64):
-        bc = gb.bc(g, srcs, batch=batch).cpu().numpy()
+    both = [gb.bc(g, srcs, batch=batch).cpu().numpy() for batch in (0, 64)]
+    for bc in both:
         np.testing.assert_allclose(bc, ref, rtol=1e-12, atol=1e-12)
+    # sources are grouped by their reach over the whole call, not by batch
+    assert np.array_equal(*both)
+    mixed = gb.bc(g, rng.permutation(srcs)).cpu().numpy()
+    np.testing.assert_allclose(mixed, ref, rtol=1e-12, atol=1e-12)
     lv = gb.bfs(g, srcs[:12]).cpu().numpy()
     for i, s in enumerate(srcs[:12]):
         assert np.array_equal(lv[i], oracle.bfs_levels(h.row_ptr, h.col, int(s)))
