@@ -32,23 +32,26 @@
 //   * finalize: each L_{d+1} entry takes its final mask, sets visited, writes
 //     BFS levels, and queues its out-edges as push items; the L_d masks are
 //     cleared for reuse as level d+2.
-// Backward (comp_delta, csr_bc.c:98-123, pull form), levels depth-2 .. 0: one
+// Backward (comp_delta, csr_bc.c:98-123, pull form), levels depth-1 .. 0: one
 // wave per L_d vertex; lane s sums ((1+delta[w][s])*sigma[v][s])/sigma[w][s]
 // over out-edges (v,w) with w at level d+1 for s, in CSR order (the operand
 // order of csr_bc.c:116).  The level masks are looked up in the two dense
 // mask arrays of the forward pass (zero when it ends): level l's entries are
 // written from the pool into array l & 1 before level l - 1 is processed,
-// and the entries of level l + 2 are cleared from it first.  Vertices above
+// and cleared once level l - 1 is done.  Vertices above
 // hub out-edges are summed in chunks whose partials are added in chunk order.
 // Accumulation (csr_bc.c:57-61): bc[v] += delta[v][s] for v != source(s), in the
 // order of the launch, which is by the sources' two-hop degrees (bc_order) and the
 // same however the sources are split into batches.
-// Both level loops are state machines on the device, replayed from captured
-// hipGraphs LPR levels at a time; the host reads one small state per replay.
+// The forward loop is a state machine on the device: the host launches levels
+// ahead of it (control; push or scan; pull; finalize) until it reports the end.
+// The backward loop's depth is known: masks, sums, combine per level.  (Two
+// hipGraphs of 16 levels with 6 launches each, captured per call, ran 9 idle
+// levels at 27 us a level on R-MAT graphs: R-MAT 20, 256 sources, 21.1 -> 19.9
+// ms; R-MAT 17, 64 sources, 1.9 -> 1.25; R-MAT 15, 8 sources, 1.3 -> 0.68.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <chrono>
 #include <cstring>
 #include <vector>
 
@@ -60,7 +63,7 @@ namespace {
 constexpr int MB = 256;            // threads per block (4 waves)
 constexpr int MBQ = 256;           // staged appends per wave
 constexpr int32_t PUSH_CH = 256;   // out-edges per push item at most
-constexpr int LPR = 16;            // levels per replay
+constexpr uint32_t AHEAD = 2;      // levels launched ahead of the device
 
 enum { MODE_NONE = 0, MODE_PUSH = 1, MODE_PULL = 2 };
 // per-group counters (u64), CN per group
@@ -96,13 +99,11 @@ struct BcLoop {
   int32_t done;   // forward finished
   int32_t stall;  // the pool or the level table needs room: the host grows it
   int32_t depth;  // forward: number of non-empty levels once done
-  int32_t bd;     // backward: the level last processed
-  int32_t bdone;  // backward finished
-  int32_t pad[2];
 };
 
 struct BcCtx {
   int32_t V, G, hub, lvl_cap;
+  int32_t lists;  // blocks per group that append to a list by vertex
   int64_t E;  // edges of the CSR (both directions have E)
   const int32_t *rp, *col, *rrp, *rcol;
   const unsigned long long *act;  // [G] sources of the group
@@ -196,7 +197,7 @@ __global__ void mbc_seed_kernel(BcCtx c, const int32_t *__restrict__ src, int32_
 }
 
 // Forward control, one wave: advances to level d = st->d + 1 (see the header).
-__global__ void mbc_fwd_ctl_kernel(BcCtx c) {
+__global__ void mbc_fwd_ctl_kernel(BcCtx c, GbProgress *prog, uint32_t k0) {
   BcLoop *st = c.st;
   if (st->done || st->stall) return;
   const int lane = threadIdx.x;
@@ -216,13 +217,17 @@ __global__ void mbc_fwd_ctl_kernel(BcCtx c) {
   const bool all_ok = __ballot(!ok) == 0ull;
   __builtin_amdgcn_wave_barrier();
   if (!all_ok) {
-    if (lane == 0) st->stall = 1;
+    if (lane == 0) {
+      st->stall = 1;
+      gb_progress(prog, k0, true, 0, 0, 1);
+    }
     return;
   }
   if (total == 0) {
     if (lane == 0) {
       st->done = 1;
       st->depth = d;
+      gb_progress(prog, k0, true, d, 0, 0);
     }
     return;
   }
@@ -240,7 +245,10 @@ __global__ void mbc_fwd_ctl_kernel(BcCtx c) {
     cg[C_PQ0 + ((d + 1) & 1)] = 0;
   }
   __builtin_amdgcn_wave_barrier();
-  if (lane == 0) st->d = d;
+  if (lane == 0) {
+    st->d = d;
+    gb_progress(prog, k0, false, 0, 0, 0);
+  }
 }
 
 // The next level's queue of group g
@@ -255,9 +263,7 @@ __device__ __forceinline__ NextList next_list(const BcCtx &c, int32_t g, int d) 
 
 // Pull candidates: vertices with 1..hub in-edges that some source of the
 // group has not reached.
-__global__ __launch_bounds__(MB) void mbc_scan_kernel(BcCtx c) {
-  const int32_t g = blockIdx.y;
-  if (c.st->done || c.st->stall || c.mode[g] != MODE_PULL) return;
+__device__ __forceinline__ void scan_level(const BcCtx &c, int32_t g) {
   const int64_t gV = (int64_t)g * c.V;
   const uint64_t act = c.act[g];
   const int lane = gb_lane();
@@ -265,7 +271,7 @@ __global__ __launch_bounds__(MB) void mbc_scan_kernel(BcCtx c) {
   gb_wave_queue<int32_t, MBQ> q(s_q[threadIdx.x / GB_WAVE], c.cand + gV,
                                 &c.cnt[(int64_t)g * CN + C_CAND]);
   for (int64_t b0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) & ~63ll; b0 < c.V;
-       b0 += (int64_t)gridDim.x * blockDim.x) {
+       b0 += (int64_t)c.lists * blockDim.x) {
     const int64_t v = b0 + lane;
     bool keep = false;
     if (v < c.V) {
@@ -277,11 +283,15 @@ __global__ __launch_bounds__(MB) void mbc_scan_kernel(BcCtx c) {
   gb_block_flush(q);
 }
 
-// Push over the level's items (see the header).
+// Push over the level's items (see the header), or the pull's candidates (from
+// the first c.lists blocks of the group).
 template <bool SIGMA>
-__global__ __launch_bounds__(MB) void mbc_push_kernel(BcCtx c) {
+__global__ __launch_bounds__(MB) void mbc_push_scan_kernel(BcCtx c) {
   const int32_t g = blockIdx.y;
-  if (c.st->done || c.st->stall || c.mode[g] != MODE_PUSH) return;
+  if (c.st->done || c.st->stall) return;
+  const int32_t mode = c.mode[g];
+  if (mode == MODE_PULL && (int32_t)blockIdx.x < c.lists) scan_level(c, g);
+  if (mode != MODE_PUSH) return;
   const int d = c.st->d;
   const int64_t gV = (int64_t)g * c.V;
   const int lane = gb_lane();
@@ -370,6 +380,8 @@ __device__ __forceinline__ void pull_in(int lane, int32_t beg, int32_t end,
   }
 }
 
+// Pull of one level: the hubs' chunks first, a wave each (their sums of sigma are
+// integers, so atomicAdd keeps them exact), then the candidates.
 template <bool SIGMA>
 __global__ __launch_bounds__(MB) void mbc_pull_kernel(BcCtx c) {
   const int32_t g = blockIdx.y;
@@ -378,38 +390,6 @@ __global__ __launch_bounds__(MB) void mbc_pull_kernel(BcCtx c) {
   const int64_t gV = (int64_t)g * c.V;
   const int lane = gb_lane();
   const uint64_t n = c.cnt[(int64_t)g * CN + C_CAND];
-  const unsigned long long *fmc = c.fm[d & 1] + gV;
-  unsigned long long *fmn = c.fm[(d + 1) & 1] + gV;
-  const uint64_t act = c.act[g];
-  const NextList nl = next_list(c, g, d);
-  __shared__ int32_t s_list[MB / GB_WAVE][MBQ];
-  gb_wave_queue<int32_t, MBQ> lq(s_list[threadIdx.x / GB_WAVE], nl.base, nl.count);
-  const uint64_t nwaves = wave_count();
-  for (uint64_t i = wave_id(); i < n; i += nwaves) {
-    const int32_t x = c.cand[gV + i];
-    const uint64_t need = ~c.visited[gV + x] & act;
-    double acc = 0.0;
-    uint64_t any = 0;
-    pull_in<SIGMA>(lane, c.rrp[x], c.rrp[x + 1], c.rcol, fmc, need, c.sigma, gV, acc, any);
-    const uint64_t found = SIGMA ? (__ballot(acc > 0.0) & need) : (any & need);
-    if (found) {
-      if (SIGMA && ((found >> lane) & 1ull)) c.sigma[(gV + x) * 64 + lane] = acc;
-      if (lane == 0) fmn[x] = found;  // one wave per candidate: a plain store
-    }
-    lq.push(lane == 0 && found ? 1u : 0u, [&](uint32_t) { return x; });
-  }
-  gb_block_flush(lq);
-}
-
-// Pull for in-degree hubs: one wave per (hub, chunk of `hub` edges).  Chunk
-// sums of sigma are integers, so atomicAdd keeps them exact.
-template <bool SIGMA>
-__global__ __launch_bounds__(MB) void mbc_pull_hub_kernel(BcCtx c) {
-  const int32_t g = blockIdx.y;
-  if (c.st->done || c.st->stall || c.mode[g] != MODE_PULL || c.n_in == 0) return;
-  const int d = c.st->d;
-  const int64_t gV = (int64_t)g * c.V;
-  const int lane = gb_lane();
   const unsigned long long *fmc = c.fm[d & 1] + gV;
   unsigned long long *fmn = c.fm[(d + 1) & 1] + gV;
   const uint64_t act = c.act[g];
@@ -432,6 +412,19 @@ __global__ __launch_bounds__(MB) void mbc_pull_hub_kernel(BcCtx c) {
     unsigned long long old = 1ull;
     if (found && lane == 0) old = atomicOr(&fmn[x], (unsigned long long)found);
     lq.push(lane == 0 && old == 0ull ? 1u : 0u, [&](uint32_t) { return x; });
+  }
+  for (uint64_t i = wave_id(); i < n; i += nwaves) {
+    const int32_t x = c.cand[gV + i];
+    const uint64_t need = ~c.visited[gV + x] & act;
+    double acc = 0.0;
+    uint64_t any = 0;
+    pull_in<SIGMA>(lane, c.rrp[x], c.rrp[x + 1], c.rcol, fmc, need, c.sigma, gV, acc, any);
+    const uint64_t found = SIGMA ? (__ballot(acc > 0.0) & need) : (any & need);
+    if (found) {
+      if (SIGMA && ((found >> lane) & 1ull)) c.sigma[(gV + x) * 64 + lane] = acc;
+      if (lane == 0) fmn[x] = found;  // one wave per candidate: a plain store
+    }
+    lq.push(lane == 0 && found ? 1u : 0u, [&](uint32_t) { return x; });
   }
   gb_block_flush(lq);
 }
@@ -514,33 +507,17 @@ __global__ __launch_bounds__(MB) void mbc_fin_kernel(BcCtx c) {
 
 // ---- backward -------------------------------------------------------------
 
-// Backward control (one thread): level st->bd - 1, done below 0.
-__global__ void mbc_bwd_ctl_kernel(BcCtx c) {
-  BcLoop *st = c.st;
-  if (st->bdone) return;
-  const int bd = st->bd - 1;
-  if (bd < 0)
-    st->bdone = 1;
-  else
-    st->bd = bd;
-}
-
-// Level l's entries into mask array l & 1 (write) or their masks cleared
-// (!write), for l = st->bd + off.
-template <bool WRITE>
-__global__ void mbc_bwd_masks_kernel(BcCtx c, int off) {
+// Level bd's entries into mask array bd & 1 (zero before).
+__global__ void mbc_bwd_masks_kernel(BcCtx c, int bd) {
   const int32_t g = blockIdx.y;
-  if (c.st->bdone) return;
-  const int l = c.st->bd + off;
-  if (l < 0 || l >= c.st->depth) return;
   const int64_t gV = (int64_t)g * c.V;
   const int64_t *lo = c.loff + (int64_t)g * c.lvl_cap;
-  const int64_t base = (int64_t)g * c.pool_cap + lo[l];
-  const int64_t n = lo[l + 1] - lo[l];
-  unsigned long long *m = c.fm[l & 1] + gV;
+  const int64_t base = (int64_t)g * c.pool_cap + lo[bd];
+  const int64_t n = lo[bd + 1] - lo[bd];
+  unsigned long long *m = c.fm[bd & 1] + gV;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
-    m[c.pool_v[base + i]] = WRITE ? c.pool_m[base + i] : 0ull;
+    m[c.pool_v[base + i]] = c.pool_m[base + i];
 }
 
 // The backward pass sums, per vertex v and source s, psi[w][s] over the
@@ -589,25 +566,33 @@ __device__ __forceinline__ double pull_out(int lane, int32_t beg, int32_t end,
   return acc;
 }
 
-__global__ __launch_bounds__(MB) void mbc_bwd_kernel(BcCtx c) {
+// One level: the partial sums of the hubs' chunks, a wave each, then the other
+// vertices (the deepest level has no successors).
+__global__ __launch_bounds__(MB) void mbc_bwd_kernel(BcCtx c, int bd, bool deepest) {
   const int32_t g = blockIdx.y;
-  if (c.st->bdone) return;
-  const int bd = c.st->bd;
   const int64_t gV = (int64_t)g * c.V;
   const int lane = gb_lane();
   const int64_t *lo = c.loff + (int64_t)g * c.lvl_cap;
   const int64_t base = (int64_t)g * c.pool_cap + lo[bd];
   const uint64_t n = (uint64_t)(lo[bd + 1] - lo[bd]);
   const unsigned long long *fm1 = c.fm[(bd + 1) & 1] + gV;
-  const bool deepest = bd == c.st->depth - 1;
+  const unsigned long long *fm0 = c.fm[bd & 1] + gV;
   const uint64_t nwaves = wave_count();
+  if (!deepest) {
+    for (uint64_t it = wave_id(); it < (uint64_t)c.n_out; it += nwaves) {
+      const HubChunk h = c.out_chunks[it];
+      const uint64_t mine = fm0[h.v];
+      if (mine == 0) continue;
+      const double acc = pull_out(lane, h.beg, h.end, c.col, fm1, mine, c.sigma, gV);
+      c.part[((int64_t)g * c.n_out + it) * 64 + lane] = acc;
+    }
+  }
   for (uint64_t i = wave_id(); i < n; i += nwaves) {
     const int32_t v = c.pool_v[base + i];
     const int32_t beg = c.rp[v], end = c.rp[v + 1];
     if (end - beg > c.bch) continue;  // split over several waves by the hub kernels
     const uint64_t mine = c.pool_m[base + i];
     const bool me = (mine >> lane) & 1ull;
-    // the deepest level has no successors
     const double acc = deepest ? 0.0 : pull_out(lane, beg, end, c.col, fm1, mine, c.sigma, gV);
     if (me) {
       const int64_t r = (gV + v) * 64 + lane;
@@ -619,32 +604,20 @@ __global__ __launch_bounds__(MB) void mbc_bwd_kernel(BcCtx c) {
   }
 }
 
-// Backward for out-degree hubs: per-chunk partials ...
-__global__ __launch_bounds__(MB) void mbc_bwd_hub_kernel(BcCtx c) {
+// The hubs' partials summed in chunk order (deterministic), one wave per hub, and
+// the masks of level bd + 1 cleared: its array takes level bd - 1 next.
+__global__ __launch_bounds__(MB) void mbc_bwd_combine_kernel(BcCtx c, int bd, bool deepest) {
   const int32_t g = blockIdx.y;
-  if (c.st->bdone || c.nhub_out == 0) return;
-  const int bd = c.st->bd;
-  if (bd == c.st->depth - 1) return;  // no successors: the combine writes 0
   const int64_t gV = (int64_t)g * c.V;
-  const int lane = gb_lane();
-  const unsigned long long *fm0 = c.fm[bd & 1] + gV;
-  const unsigned long long *fm1 = c.fm[(bd + 1) & 1] + gV;
-  const uint64_t nwaves = wave_count();
-  for (uint64_t it = wave_id(); it < (uint64_t)c.n_out; it += nwaves) {
-    const HubChunk h = c.out_chunks[it];
-    const uint64_t mine = fm0[h.v];
-    if (mine == 0) continue;
-    const double acc = pull_out(lane, h.beg, h.end, c.col, fm1, mine, c.sigma, gV);
-    c.part[((int64_t)g * c.n_out + it) * 64 + lane] = acc;
+  if (!deepest) {
+    const int64_t *lo = c.loff + (int64_t)g * c.lvl_cap;
+    const int64_t base = (int64_t)g * c.pool_cap + lo[bd + 1];
+    const int64_t n = lo[bd + 2] - lo[bd + 1];
+    unsigned long long *m = c.fm[(bd + 1) & 1] + gV;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * blockDim.x)
+      m[c.pool_v[base + i]] = 0ull;
   }
-}
-
-// ... summed in chunk order (deterministic), one wave per hub.
-__global__ __launch_bounds__(MB) void mbc_bwd_combine_kernel(BcCtx c) {
-  const int32_t g = blockIdx.y;
-  if (c.st->bdone || c.nhub_out == 0) return;
-  const int bd = c.st->bd;
-  const int64_t gV = (int64_t)g * c.V;
   const int lane = gb_lane();
   const unsigned long long *fm0 = c.fm[bd & 1] + gV;
   const uint64_t nwaves = wave_count();
@@ -653,7 +626,7 @@ __global__ __launch_bounds__(MB) void mbc_bwd_combine_kernel(BcCtx c) {
     const int32_t x = h.v;
     const uint64_t mine = fm0[x];
     if (!((mine >> lane) & 1ull)) continue;
-    const int32_t nch = bd == c.st->depth - 1 ? 0 : h.n;
+    const int32_t nch = deepest ? 0 : h.n;
     double acc = 0.0;
     const double *p = c.part + ((int64_t)g * c.n_out + h.first) * 64 + lane;
     for (int32_t k = 0; k < nch; k += 8) {  // 8 loads in flight
@@ -769,45 +742,17 @@ gb_status grow_rows(DevBuf &buf, size_t elem, int32_t G, int64_t old, int64_t wa
   return GB_OK;  // nb frees the old buffer
 }
 
-// One replayable chunk of LPR levels: forward or backward.
-struct LevelGraph {
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  void reset() {
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (graph) (void)hipGraphDestroy(graph);
-    exec = nullptr;
-    graph = nullptr;
-  }
-  ~LevelGraph() { reset(); }
-};
-
-template <class F>
-gb_status capture(LevelGraph &lg, hipStream_t cs, F launches) {
-  lg.reset();
-  hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
-  if (e == hipSuccess) {
-    launches();
-    e = hipStreamEndCapture(cs, &lg.graph);
-  }
-  if (e == hipSuccess) e = hipGraphInstantiate(&lg.exec, lg.graph, nullptr, nullptr, 0);
-  if (e != hipSuccess) return gb_fail(GB_ERR_HIP, "bc: graph capture failed: %s", hipGetErrorString(e));
-  return GB_OK;
-}
-
 // A launch shape: grid blocks per group (x) as blocks per CU, and the
 // push/pull ratio alpha.
 struct BcShape {
   int per_cu, alpha;
 };
 
-// The rules when the autotuner does not run: 8 blocks per CU per group, at
-// least 16 and at most 32768 blocks over all groups; push while 16 times the
-// frontier's out-edges stay below the unvisited vertices' in-edges.
+// Blocks per group: at least 16, and at most 32768 over all groups; push while
+// alpha times the frontier's out-edges stay below the unvisited vertices' in-edges.
 int bc_grid(const BcShape &sh, int32_t G) {
   return std::max(16, std::min(gb_num_cus() * sh.per_cu, 32768 / G));
 }
-constexpr BcShape BC_RULES{8, 16};
 
 // Runs one batch of up to 64*G sources.  with_sigma: Brandes (sigma, delta,
 // accumulate into d_bc); otherwise BFS levels into d_level [nsrc][V].
@@ -933,57 +878,35 @@ gb_status ms_run(gb_graph g, const int32_t *h_src, int32_t nsrc, bool with_sigma
   // 25 ns of that counter's time, so few blocks (two per CU over all groups;
   // symmetric R-MAT 20, 4 groups, 8 per CU and group: scan 760 -> 350 us,
   // finalize 900 -> 570 us)
-  const dim3 lists(std::min(gx, std::max(16, 2 * gb_num_cus() / G)), G);
+  c.lists = std::min(gx, std::max(16, 2 * gb_num_cus() / G));
+  const dim3 lists(c.lists, G);
   hipLaunchKernelGGL(mbc_seed_kernel, dim3(G), dim3(64), 0, st, c, w.src.as<int32_t>(), nsrc);
   hipLaunchKernelGGL(mbc_fin_kernel, lists, block, 0, st, c);
   GB_HIP(hipGetLastError());
-  hipStream_t cs = st, own = nullptr;
-  if (!st) {  // the null stream cannot be captured
-    GB_HIP(hipStreamCreate(&own));
-    cs = own;
-  }
-  struct OwnStream {
-    hipStream_t s;
-    ~OwnStream() {
-      if (s) {
-        (void)hipStreamSynchronize(s);
-        (void)hipStreamDestroy(s);
-      }
-    }
-  } own_guard{own};
-  if (own) {
-    hipEvent_t ready;
-    GB_HIP(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
-    GB_HIP(hipEventRecord(ready, st));
-    GB_HIP(hipStreamWaitEvent(cs, ready, 0));
-    (void)hipEventDestroy(ready);
-  }
-  auto fwd_launches = [&]() {
-    for (int k = 0; k < LPR; k++) {
-      hipLaunchKernelGGL(mbc_fwd_ctl_kernel, dim3(1), dim3(64), 0, cs, c);
-      hipLaunchKernelGGL(mbc_scan_kernel, lists, block, 0, cs, c);
-      if (with_sigma) {
-        hipLaunchKernelGGL(mbc_push_kernel<true>, grid, block, 0, cs, c);
-        hipLaunchKernelGGL(mbc_pull_kernel<true>, grid, block, 0, cs, c);
-        hipLaunchKernelGGL(mbc_pull_hub_kernel<true>, grid, block, 0, cs, c);
-      } else {
-        hipLaunchKernelGGL(mbc_push_kernel<false>, grid, block, 0, cs, c);
-        hipLaunchKernelGGL(mbc_pull_kernel<false>, grid, block, 0, cs, c);
-        hipLaunchKernelGGL(mbc_pull_hub_kernel<false>, grid, block, 0, cs, c);
-      }
-      hipLaunchKernelGGL(mbc_fin_kernel, lists, block, 0, cs, c);
-    }
-  };
-  LevelGraph fg;
-  GB_TRY(capture(fg, cs, fwd_launches));
-  BcLoop hl{};
-  int32_t last_d = -2;
+  GbProgress *prog = nullptr;
   for (;;) {
-    GB_HIP(hipGraphLaunch(fg.exec, cs));
-    GB_HIP(hipMemcpyAsync(&hl, c.st, sizeof(hl), hipMemcpyDeviceToHost, cs));
-    GB_HIP(hipStreamSynchronize(cs));
-    if (hl.done) break;
-    if (hl.stall) {
+    GB_TRY(gb_progress_begin(&prog));
+    const gb_status lst = gb_drive_phases(prog, AHEAD, st, [&](uint32_t k) {
+      hipLaunchKernelGGL(mbc_fwd_ctl_kernel, dim3(1), dim3(64), 0, st, c, prog, k);
+      if (with_sigma) {
+        hipLaunchKernelGGL(mbc_push_scan_kernel<true>, grid, block, 0, st, c);
+        hipLaunchKernelGGL(mbc_pull_kernel<true>, grid, block, 0, st, c);
+      } else {
+        hipLaunchKernelGGL(mbc_push_scan_kernel<false>, grid, block, 0, st, c);
+        hipLaunchKernelGGL(mbc_pull_kernel<false>, grid, block, 0, st, c);
+      }
+      hipLaunchKernelGGL(mbc_fin_kernel, lists, block, 0, st, c);
+      return hipGetLastError();
+    });
+    if (lst != GB_OK) {
+      (void)hipStreamSynchronize(st);  // launches before an error end first
+      return lst;
+    }
+    if (!prog->capped) break;
+    {
+      // stalled at level d + 1
+      BcLoop hl{};
+      GB_HIP(hipMemcpy(&hl, c.st, sizeof(hl), hipMemcpyDeviceToHost));
       // room for one more level of V entries per group, and for the level table
       int64_t used = 0;
       std::vector<int64_t> lo((size_t)G * lvl_cap);
@@ -997,59 +920,36 @@ gb_status ms_run(gb_graph g, const int32_t *h_src, int32_t nsrc, bool with_sigma
                                            (int64_t)cn[(size_t)k * CN + C_NEXT]);
       if (used + V > pool_cap) {
         const int64_t ncap = std::max<int64_t>(2 * pool_cap, used + 2 * (int64_t)V);
-        GB_TRY(grow_rows(w.pool_v, sizeof(int32_t), G, pool_cap, ncap, cs));
-        GB_TRY(grow_rows(w.pool_m, sizeof(uint64_t), G, pool_cap, ncap, cs));
+        GB_TRY(grow_rows(w.pool_v, sizeof(int32_t), G, pool_cap, ncap, st));
+        GB_TRY(grow_rows(w.pool_m, sizeof(uint64_t), G, pool_cap, ncap, st));
         pool_cap = ncap;
       }
       if (dn + 1 >= lvl_cap) {
-        GB_TRY(grow_rows(w.loff, sizeof(int64_t), G, lvl_cap, 2 * lvl_cap, cs));
+        GB_TRY(grow_rows(w.loff, sizeof(int64_t), G, lvl_cap, 2 * lvl_cap, st));
         lvl_cap *= 2;
       }
       set_pool();
       hl.stall = 0;
-      GB_HIP(hipMemcpyAsync(c.st, &hl, sizeof(hl), hipMemcpyHostToDevice, cs));
-      GB_HIP(hipStreamSynchronize(cs));
-      GB_TRY(capture(fg, cs, fwd_launches));
-      continue;
+      GB_HIP(hipMemcpyAsync(c.st, &hl, sizeof(hl), hipMemcpyHostToDevice, st));
+      GB_HIP(hipStreamSynchronize(st));
     }
-    if (hl.d == last_d) return gb_fail(GB_ERR_HIP, "bc: level loop made no progress");
-    last_d = hl.d;
   }
-  const int depth = hl.depth;  // levels 0..depth-1 are non-empty
+  const int depth = (int)prog->phases;  // levels 0..depth-1 are non-empty
   if (depth_out) *depth_out = depth;
   if (!with_sigma) return GB_OK;
-  if (depth >= 2) {
-    // levels depth-1 .. 0 (the forward pass left both mask arrays zero): clear
-    // level bd + 2, write level bd, process; the deepest level only turns
-    // sigma into psi
-    hl.bd = depth;
-    hl.bdone = 0;
-    GB_HIP(hipMemcpyAsync(c.st, &hl, sizeof(hl), hipMemcpyHostToDevice, cs));
-    GB_HIP(hipStreamSynchronize(cs));
-    LevelGraph bg;
-    GB_TRY(capture(bg, cs, [&]() {
-      for (int k = 0; k < LPR; k++) {
-        hipLaunchKernelGGL(mbc_bwd_ctl_kernel, dim3(1), dim3(1), 0, cs, c);
-        hipLaunchKernelGGL(mbc_bwd_masks_kernel<false>, grid, block, 0, cs, c, 2);
-        hipLaunchKernelGGL(mbc_bwd_masks_kernel<true>, grid, block, 0, cs, c, 0);
-        hipLaunchKernelGGL(mbc_bwd_kernel, grid, block, 0, cs, c);
-        hipLaunchKernelGGL(mbc_bwd_hub_kernel, grid, block, 0, cs, c);
-        hipLaunchKernelGGL(mbc_bwd_combine_kernel, grid, block, 0, cs, c);
-      }
-    }));
-    for (;;) {
-      GB_HIP(hipGraphLaunch(bg.exec, cs));
-      GB_HIP(hipMemcpyAsync(&hl, c.st, sizeof(hl), hipMemcpyDeviceToHost, cs));
-      GB_HIP(hipStreamSynchronize(cs));
-      if (hl.bdone) break;
-    }
+  // the forward pass left both mask arrays zero; the deepest level only turns
+  // sigma into psi
+  for (int bd = depth - 1; bd >= 0 && depth >= 2; bd--) {
+    const bool deepest = bd == depth - 1;
+    hipLaunchKernelGGL(mbc_bwd_masks_kernel, grid, block, 0, st, c, bd);
+    hipLaunchKernelGGL(mbc_bwd_kernel, grid, block, 0, st, c, bd, deepest);
+    hipLaunchKernelGGL(mbc_bwd_combine_kernel, grid, block, 0, st, c, bd, deepest);
   }
   hipLaunchKernelGGL(mbc_accum_kernel,
                      dim3((V + ACC_V * (ACC_BLOCK / GB_WAVE) - 1) / (ACC_V * (ACC_BLOCK / GB_WAVE))),
-                     dim3(ACC_BLOCK), 0, cs, V, G, nsrc,
+                     dim3(ACC_BLOCK), 0, st, V, G, nsrc,
                      w.src.as<int32_t>(), c.visited, c.delta, d_bc);
   GB_HIP(hipGetLastError());
-  if (own) GB_HIP(hipStreamSynchronize(cs));
   return GB_OK;
 }
 
@@ -1112,80 +1012,18 @@ gb_status bc_order(gb_graph g, const int32_t *h_src, int32_t nsrc, std::vector<i
   return GB_OK;
 }
 
-// The shape for a launch of G groups on graph g: GB_BC_GRID (4, 8 or 16
-// blocks per CU) and GB_BC_ALPHA (4 .. 64) fix parts; else the shape cached
-// in the handle for G groups, else the rules.
-const gb_graph_s::BcTuned *bc_cached(gb_graph g, int32_t G) {
-  for (const auto &t : g->bc_tuned)
-    if (t.groups == G) return &t;
-  return nullptr;
-}
-BcShape bc_shape(gb_graph g, int32_t G, int *fixed_parts) {
-  BcShape sh = BC_RULES;
-  if (const auto *t = bc_cached(g, G)) sh = BcShape{t->per_cu, t->alpha};
-  int fixed = 0;
+// The shape for a launch of G groups on graph g; GB_BC_GRID (4, 8 or 16 blocks per
+// CU) and GB_BC_ALPHA (4 .. 64) fix parts.  Timing each graph's first batch in six
+// shapes cost six solves and found at most 2%: alpha 4 .. 64 is level, 4 blocks
+// per CU 1.15 times slower, 16 against 8 take 19.9 and 20.3 ms on R-MAT 20 with
+// 4 groups, 1.26 and 1.26 on R-MAT 17, 0.75 and 0.71 on R-MAT 15 with one.
+BcShape bc_shape(gb_graph g, int32_t G) {
+  BcShape sh{(int64_t)g->V * G >= ((int64_t)1 << 20) ? 16 : 8, 16};
   const char *e = getenv("GB_BC_GRID");
-  if (e && (atoi(e) == 4 || atoi(e) == 8 || atoi(e) == 16)) {
-    sh.per_cu = atoi(e);
-    fixed |= 1;
-  }
+  if (e && (atoi(e) == 4 || atoi(e) == 8 || atoi(e) == 16)) sh.per_cu = atoi(e);
   e = getenv("GB_BC_ALPHA");
-  if (e && atoi(e) >= 4 && atoi(e) <= 64) {
-    sh.alpha = atoi(e);
-    fixed |= 2;
-  }
-  if (fixed_parts) *fixed_parts = fixed;
+  if (e && atoi(e) >= 4 && atoi(e) <= 64) sh.alpha = atoi(e);
   return sh;
-}
-
-// Autotuner for the Brandes engine, run on a graph's first batch of G groups
-// when the handle has no shape for G yet (GB_BC_TUNE=0: rules only): the
-// batch is solved in the rules' shape, then with one change at a time (the
-// other blocks-per-CU counts, then alpha halved and doubled), into a scratch
-// score array; the fastest shape is kept in the handle.  Every shape gives
-// the same scores.
-gb_status bc_tune(gb_graph g, const int32_t *h_src, int32_t nsrc, hipStream_t st) {
-  const int32_t G = (nsrc + 63) / 64;
-  int fixed = 0;
-  const BcShape base = bc_shape(g, G, &fixed);
-  const char *e = getenv("GB_BC_TUNE");
-  if ((e && e[0] == '0') || bc_cached(g, G) || fixed == 3) return GB_OK;
-  DevBuf scratch;
-  GB_TRY(scratch.ensure(sizeof(double) * (g->V + 1)));
-  auto timed = [&](const BcShape &s, double &ms) -> gb_status {
-    GB_HIP(hipMemsetAsync(scratch.p, 0, sizeof(double) * g->V, st));
-    GB_HIP(hipStreamSynchronize(st));
-    const auto t0 = std::chrono::steady_clock::now();
-    int32_t depth = 0;
-    GB_TRY(ms_run(g, h_src, nsrc, true, scratch.as<double>(), nullptr, st, &depth, s));
-    GB_HIP(hipStreamSynchronize(st));
-    ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-    return GB_OK;
-  };
-  BcShape best = base;
-  double best_ms = 0;
-  GB_TRY(timed(best, best_ms));
-  auto consider = [&](BcShape s) -> gb_status {
-    double ms = 0;
-    GB_TRY(timed(s, ms));
-    if (ms < best_ms) {
-      best = s;
-      best_ms = ms;
-    }
-    return GB_OK;
-  };
-  if (!(fixed & 1)) {
-    const int pc0 = best.per_cu;
-    for (int pc : {4, 8, 16})
-      if (pc != pc0) GB_TRY(consider(BcShape{pc, best.alpha}));
-  }
-  if (!(fixed & 2)) {
-    const int a0 = best.alpha;
-    for (int a : {a0 / 2, a0 * 2})
-      if (a >= 4 && a <= 64) GB_TRY(consider(BcShape{best.per_cu, a}));
-  }
-  g->bc_tuned.push_back(gb_graph_s::BcTuned{G, best.per_cu, best.alpha});
-  return GB_OK;
 }
 
 }  // namespace
@@ -1210,7 +1048,7 @@ extern "C" gb_status gb_bfs(gb_graph g, const int32_t *h_sources, int32_t nsrc, 
   for (int32_t b0 = 0; b0 < nsrc; b0 += per) {
     const int32_t ns = std::min(per, nsrc - b0);
     GB_TRY(ms_run(g, h_sources + b0, ns, false, nullptr, d_level + (int64_t)b0 * V, st, nullptr,
-                  bc_shape(g, (ns + 63) / 64, nullptr)));
+                  bc_shape(g, (ns + 63) / 64)));
   }
   GB_HIP(hipStreamSynchronize(st));
   return GB_OK;
@@ -1249,9 +1087,8 @@ extern "C" gb_status gb_bc(gb_graph g, const int32_t *h_sources, int32_t nsrc, i
       batches++;
       continue;
     }
-    GB_TRY(bc_tune(g, h_sources + b0, ns, st));
     GB_TRY(ms_run(g, h_sources + b0, ns, true, d_bc, nullptr, st, &depth,
-                  bc_shape(g, (ns + 63) / 64, nullptr)));
+                  bc_shape(g, (ns + 63) / 64)));
     max_depth = std::max(max_depth, depth - 1);
     batches++;
   }
