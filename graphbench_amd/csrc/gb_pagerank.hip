@@ -1863,10 +1863,26 @@ static gb_status pb_build(gb_graph g, bool relabel, const int32_t *irp, const in
   }
   std::vector<PbPiece> pieces;
   std::vector<int32_t> multi;
+  // Edges per piece: 5/4 of a CU's share, or 256 K.  A piece costs about 8 us
+  // besides its edges, and a split bin's pieces meet in global atomics and pb_rows,
+  // so a bin is split only from half a piece over, and where all bins are about as
+  // large not at all.  (R-MAT, 2 M vertices, 17 M edges: 3/4 of the share 1.65 ms,
+  // 1 1.47, 5/4 1.39, 2 1.40, bins of up to 256 K whole 1.76; 1 M, 25 M edges:
+  // 1.10, 1.02, 1.09, 1.29, 1.47; 4 M, 67 M: 2.31, 2.28, 2.27, 2.28, 2.28.  Uniform,
+  // 0.5 M vertices, 6 M edges: pieces of 32 K 0.72, whole bins 0.66.)
+  int64_t per = piece;
+  if (per == 0) {
+    int64_t largest = 0;
+    for (int64_t b = 0; b < nbins; ++b)
+      largest = std::max<int64_t>(largest, bin_start[b + 1] - bin_start[b]);
+    const bool even = nbins >= 32 && 2 * nbins * largest <= 3 * P;
+    per = even ? (int64_t)1 << 18
+               : std::min<int64_t>(1 << 18, std::max<int64_t>(1 << 14, P * 5 / (4 * gb_num_cus())));
+  }
+  const int64_t most = std::max<int64_t>(1, per / PB_BATCH);
   for (int64_t b = 0; b < nbins; ++b) {
     const int64_t s = bin_start[b] / PB_BATCH, n = bin_start[b + 1] / PB_BATCH - s;
-    const int64_t most = std::max(1, piece / PB_BATCH);
-    const int64_t k = std::max<int64_t>(1, (n + most - 1) / most);
+    const int64_t k = std::max<int64_t>(1, piece ? (n + most - 1) / most : (n + most / 2) / most);
     if (k > 1) multi.push_back((int32_t)b);
     for (int64_t j = 0; j < k; ++j)
       pieces.push_back(PbPiece{(int32_t)b, (int32_t)((s + n * j / k) * PB_BATCH),
@@ -1949,11 +1965,11 @@ constexpr PbShape PB_SHAPES[] = {{0, 0, 0},         {8192, 13, 13},  {16384, 14,
                                  {8192, 13, 12},    {16384, 13, 13}, {20480, 13, 13},
                                  {16384, 12, 13}};
 constexpr int PB_NSHAPES = 7;
-// stream entries per accumulation block at most (GB_PR_PB_PIECE, multiple of 4)
+// edges per accumulation block at most (GB_PR_PB_PIECE), 0: pb_build's rule
 static int pb_piece() {
   const char *e = getenv("GB_PR_PB_PIECE");
   const int v = e ? atoi(e) : 0;
-  return v >= 4096 && v <= (1 << 26) ? v & ~3 : 262144;
+  return v >= 4096 && v <= (1 << 26) ? v & ~3 : 0;
 }
 static bool valid_rb(int rb) { return rb == 1024 || rb == 2048 || rb == 4096; }
 
@@ -2040,9 +2056,13 @@ static gb_status pagerank_small(gb_graph g, const gb_pr_params *p, float *d_x, g
 // graphs only) takes the most-read sources off the L2 but its LDS lowers
 // occupancy.  Row-block candidates (unless row_block is -1) skip the merge-path
 // search and scan but leave lanes idle in blocks of uneven rows.  The binned
-// candidate (with the row-block ones, unless binned is -1) streams every edge
-// twice but issues no random reads.  Candidates are compared by the mean time
-// of a whole iteration (gather and fix-up).
+// candidate (with the row-block ones, unless binned is -1) streams instead of
+// reading at random.  Its shape: bins of 4096 for up to 1 M vertices (uniform
+// graph of 1 M, 25 M edges: 855 us a solve, shape 4 928), chunks of 16384 from 4 M
+// on (uniform, 8 M, 200 M edges: 6.5 ms, shape 4 7.0).  Candidates are compared by
+// the mean time of a whole iteration (gather and fix-up); if the binned one takes
+// under 0.8 of the first row-block one, the rest (within 1.2 of each other there)
+// is not timed: R-MAT 22, first call 56 -> 25 ms.
 static gb_status pick_shape(gb_graph g, const gb_pr_params *p, float *d_x, void *stream,
                             PrShape *out) {
   const bool rl = use_relabel(g, p);
@@ -2086,16 +2106,18 @@ static gb_status pick_shape(gb_graph g, const gb_pr_params *p, float *d_x, void 
     return GB_OK;
   }
   std::vector<PrShape> cands;
+  if (try_pb)
+    cands = {PrShape{0, rl ? 4096 : 0, 2048, 0},
+             PrShape{0, 0, 0, g->V <= (1 << 20) ? 3 : g->V < (1 << 22) ? 4 : 2}};
   for (int ci : fixed_ipt ? std::vector<int>{fixed_ipt} : std::vector<int>{4, 8, 12, 16})
     for (int ch : fixed_hot >= 0 ? std::vector<int>{fixed_hot} : std::vector<int>{0, 4096, 8192})
       cands.push_back(PrShape{ci, ch, 0, 0});
   if (try_rb)
     for (int rb : {1024, 2048, 4096})
       for (int ch : rl ? std::vector<int>{0, 4096, 8192} : std::vector<int>{0})
-        cands.push_back(PrShape{0, ch, rb, 0});
-  if (try_pb) cands.push_back(PrShape{0, 0, 0, 4});
+        if (!try_pb || rb != 2048 || ch != cands[0].hot) cands.push_back(PrShape{0, ch, rb, 0});
   PrShape best = cands[0];
-  double best_ms = 1e300;
+  double best_ms = 1e300, first_ms = 0.0;
   for (const PrShape &c : cands) {
     gb_pr_params q = *p;
     q.max_iter = 3;
@@ -2109,10 +2131,12 @@ static gb_status pick_shape(gb_graph g, const gb_pr_params *p, float *d_x, void 
     if (s == GB_ERR_UNSUPPORTED && c.pb) continue;  // graph too large for the binned layout
     GB_TRY(s);
     const double ms = r.gather_launches ? it_ms / r.gather_launches : 1e300;
+    if (&c == &cands[0]) first_ms = ms;
     if (ms < best_ms) {
       best_ms = ms;
       best = c;
     }
+    if (c.pb && ms < 0.8 * first_ms) break;
   }
   g->pr_tuned[key][0] = best.ipt;
   g->pr_tuned[key][1] = best.hot;

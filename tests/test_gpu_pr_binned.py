@@ -24,13 +24,17 @@ def _edges(kind, rng):
         return V, rng.integers(0, 8192, 60000), rng.integers(0, V, 60000)
     if kind == "nohub":  # no hub source, bins without edges
         return V, rng.integers(20480, V, 60000), rng.integers(0, V, 60000) // 8192 * 8192 % 24576
+    if kind == "even":  # bins of one size, left whole
+        return 150001, rng.integers(0, 150001, 700000), rng.integers(0, 150001, 700000)
+    if kind == "skew":  # a few bins with most edges
+        return 150001, rng.integers(0, 150001, 400000), rng.integers(0, 387, 400000) ** 2
     if kind == "sparse":  # segments of 0 to 5 values
         return V, rng.integers(0, V, 70), rng.integers(0, V, 70)
     src = rng.integers(0, V, 65536)  # "batch": bins near whole batches of 256
     return V, src, src * 13 % V
 
 
-@pytest.mark.parametrize("kind", ["runs", "long", "hub", "nohub", "sparse", "batch"])
+@pytest.mark.parametrize("kind", ["runs", "long", "hub", "nohub", "even", "skew", "sparse", "batch"])
 @pytest.mark.parametrize("piece", ["4096", None])
 def test_shared_values(gpu, monkeypatch, kind, piece):
     gb = gpu
