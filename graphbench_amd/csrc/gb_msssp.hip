@@ -185,7 +185,19 @@ __device__ __forceinline__ MsIn ms_load(const MsCtx &c, const unsigned long long
 // Light phase: expand the entries of near queue a_in.  Entries are software
 // pipelined: entry i is expanded while entry i + nwaves's loads and entry
 // i + 2 nwaves's descriptor are in flight.
-template <int W, bool SCAN>
+// WIDE: the distance array is 4 GiB or more.  Below, its byte offsets are 32 bits.
+// What bounds the step beside its lines is instructions per (edge, source): with
+// a 64-bit multiply for the bucket of every new distance, 64-bit offsets and
+// counters per lane, R-MAT 24 with 32 sources took 48.9 ms; a compare with the
+// bucket's end 42.6; saturating adds, counts of ballots and 32-bit offsets 40.3.
+template <int W, bool WIDE>
+__device__ __forceinline__ uint32_t *ms_dist(uint32_t *dist, int32_t x, int t) {
+  if (WIDE) return dist + ((int64_t)x * W + t);
+  return (uint32_t *)((char *)dist + ((uint32_t)x * (W * 4u) + (uint32_t)t * 4u));
+}
+
+// The counters are the wave's (uniform).
+template <int W, bool SCAN, bool WIDE>
 __device__ __forceinline__ void ms_light(const MsCtx &c, const MsIo &io, uint64_t b, bool all,
                                          MsEnt *lds_near, uint64_t *lds_far, uint32_t &relax, uint32_t &imp_near,
                                          uint32_t &imp_far, uint32_t &expanded, bool &ovf) {
@@ -196,12 +208,16 @@ __device__ __forceinline__ void ms_light(const MsCtx &c, const MsIo &io, uint64_
   // the lane that issues the mask update of (step lane / ES, slot lane % ES)
   const int kj = lane / ES, ej = lane % ES;
   const uint64_t wmask = W == 64 ? ~0ull : ((1ull << W) - 1);
+  const uint64_t tasks = c.ntask >= 64 ? ~0ull : ((1ull << c.ntask) - 1);
   const MsEnt *in = io.in;
   const unsigned long long *min_ = io.min_;
   unsigned long long *mout = io.mout;
   gb_wave_queue<MsEnt, MS_NCAP> nq(lds_near, io.near_out, io.n_near);
   gb_wave_queue<uint64_t, MS_FCAP> fq(lds_far, io.far_out, io.n_far);
   const uint64_t n = io.n;
+  // the largest distance of bucket b: a compare per edge instead of a division
+  const uint64_t top = b >= 0xFFFFFFFFull ? ~0ull : (b + 1) * c.delta - 1;
+  const uint32_t lim = top < 0xFFFFFFFFull ? (uint32_t)top : 0xFFFFFFFFu;
   // wave-uniform indices (readfirstlane): the entries are read with scalar
   // loads and live in scalar registers
   const uint64_t wave = __builtin_amdgcn_readfirstlane(
@@ -223,7 +239,8 @@ __device__ __forceinline__ void ms_light(const MsCtx &c, const MsIo &io, uint64_
     if (i2 < n) enn = in[i2];
     const bool act = t < c.ntask && ((cur.m >> t) & 1ull);
     const int cnt = ecur.end - ecur.beg;
-    expanded += lane == 0 ? (uint32_t)cnt : 0u;
+    expanded += (uint32_t)cnt;
+    relax += (uint32_t)__popcll((unsigned long long)gb_uniform((uint64_t)cur.m) & tasks) * (uint32_t)cnt;
     for (int g0 = 0; g0 < cnt; g0 += G) {
       int32_t x[UNROLL];
       uint32_t nd[UNROLL], old[UNROLL];
@@ -235,36 +252,33 @@ __device__ __forceinline__ void ms_light(const MsCtx &c, const MsIo &io, uint64_
         const uint32_t wk = __shfl(cur.w, r, GB_WAVE);
         // branch-free, so that the reads below stay one batch
         ok[k] = act & (r < cnt);
-        const uint64_t s = (uint64_t)cur.du + wk;
-        const bool big = s >= 0xFFFFFFFFull;
-        ovf |= ok[k] & big;
-        nd[k] = big ? 0xFFFFFFFEu : (uint32_t)s;
-        relax += ok[k];
+        const uint32_t s = __builtin_elementwise_add_sat(cur.du, wk);
+        ovf |= ok[k] & (s == 0xFFFFFFFFu);
+        nd[k] = min(s, 0xFFFFFFFEu);
       }
       // unconditional: x[k] is a vertex for every lane (0 past the chunk's
       // end) and t < W, so the read is in bounds; a conditional read would be
       // compiled to a branch per step that waits for its own load
 #pragma unroll
-      for (int k = 0; k < UNROLL; k++) old[k] = c.dist[(int64_t)x[k] * W + t];
-      // lane j < G updates the masks of edge g0 + j = (step j / ES, slot j % ES)
-      uint64_t nm = 0, fm = 0;
+      for (int k = 0; k < UNROLL; k++) old[k] = *ms_dist<W, WIDE>(c.dist, x[k], t);
+      uint64_t nb[UNROLL], fb[UNROLL], anyn = 0, anyf = 0;
 #pragma unroll
       for (int k = 0; k < UNROLL; k++) {
         ok[k] = ok[k] & (nd[k] < old[k]);
-        const bool isnear = ms_bucket(nd[k], c.magic) <= b;
-        const bool near = ok[k] & isnear;
-        const bool far = ok[k] & !isnear;
-        imp_near += near;
-        imp_far += far;
-        const uint64_t nbk = __ballot(near), fbk = __ballot(far);
-        nm = kj == k ? nbk : nm;
-        fm = kj == k ? fbk : fm;
+        const bool isnear = nd[k] <= lim;
+        nb[k] = __ballot(ok[k] & isnear);
+        fb[k] = __ballot(ok[k] & !isnear);
+        anyn |= nb[k];
+        anyf |= fb[k];
+        imp_near += (uint32_t)__popcll(nb[k]);
+        imp_far += (uint32_t)__popcll(fb[k]);
       }
+      if ((anyn | anyf) == 0ull) continue;  // no pair improved
       // the atomics go after every read of the group: a wait for a later read
       // would otherwise also wait for the atomics issued before it
 #pragma unroll
       for (int k = 0; k < UNROLL; k++)
-        if (ok[k]) atomicMin(&c.dist[(int64_t)x[k] * W + t], nd[k]);
+        if (ok[k]) atomicMin(ms_dist<W, WIDE>(c.dist, x[k], t), nd[k]);
       // the counters tell the buckets of the caller's width apart, also within
       // a range of several
       if (all) {
@@ -272,20 +286,30 @@ __device__ __forceinline__ void ms_light(const MsCtx &c, const MsIo &io, uint64_
 #pragma unroll
         for (int k = 0; k < UNROLL; k++) {
           const uint64_t bk = ms_bucket(nd[k], c.magic);
-          const uint32_t moved = ok[k] & (bk <= b) & (bk > bu);
+          const uint32_t moved = (uint32_t)__popcll(__ballot(ok[k] & (bk <= b) & (bk > bu)));
           imp_near -= moved;
           imp_far += moved;
         }
       }
-      nm = (nm >> (ej * W)) & wmask;
-      fm = (fm >> (ej * W)) & wmask;
+      // lane j < G updates the masks of edge g0 + j = (step j / ES, slot j % ES)
+      uint64_t nm = 0, fm = 0;
+      if (anyn) {
+#pragma unroll
+        for (int k = 0; k < UNROLL; k++) nm = kj == k ? nb[k] : nm;
+        nm = (nm >> (ej * W)) & wmask;
+      }
+      if (anyf) {
+#pragma unroll
+        for (int k = 0; k < UNROLL; k++) fm = kj == k ? fb[k] : fm;
+        fm = (fm >> (ej * W)) & wmask;
+      }
       const uint32_t xj = (uint32_t)__shfl(cur.x, (g0 + lane) & (GB_WAVE - 1), GB_WAVE);
       if (SCAN) {
         // no return value: the compaction pass after the phase queues the
         // marked targets
         if (lane < G && nm) atomicOr(&mout[xj], (unsigned long long)nm);
         // far marks are rarer: the lane that starts a far mask queues the target
-        if (__ballot(lane < G && fm) != 0ull) {
+        if (anyf) {
           unsigned long long of = 1ull;
           if (lane < G && fm) of = atomicOr(&c.far[xj], (unsigned long long)fm);
           fq.push(of == 0ull ? 1u : 0u, [&](uint32_t) { return (uint64_t)xj; });
@@ -384,7 +408,7 @@ __device__ __forceinline__ void ms_far(const MsCtx &c, const MsIo &io, uint64_t 
 }
 
 // The action (ACT_LIGHT or ACT_FAR) of one phase.
-template <int W, bool SCAN>
+template <int W, bool SCAN, bool WIDE>
 __device__ __forceinline__ void ms_phase(const MsCtx &c, const MsIo &io, int act, uint64_t first,
                                          uint64_t last, bool all) {
   __shared__ uint64_t s_far[MS_BLOCK / GB_WAVE][MS_FCAP];
@@ -394,17 +418,12 @@ __device__ __forceinline__ void ms_phase(const MsCtx &c, const MsIo &io, int act
   if (act == ACT_LIGHT) {
     uint32_t relax = 0, imp_near = 0, imp_far = 0, expanded = 0;
     bool ovf = false;
-    ms_light<W, SCAN>(c, io, last, all, ln, lf, relax, imp_near, imp_far, expanded, ovf);
-    uint32_t tot, tn, tf, te;
-    (void)gb_wave_excl_sum(relax, &tot);
-    (void)gb_wave_excl_sum(imp_near, &tn);
-    (void)gb_wave_excl_sum(imp_far, &tf);
-    (void)gb_wave_excl_sum(expanded, &te);
+    ms_light<W, SCAN, WIDE>(c, io, last, all, ln, lf, relax, imp_near, imp_far, expanded, ovf);
     if (gb_lane() == 0) {
-      gb_wstat_add(c.wstat, 0, tot);
-      gb_wstat_add(c.wstat, 1, tn);
-      gb_wstat_add(c.wstat, 2, tf);
-      gb_wstat_add(c.wstat, 3, te);
+      gb_wstat_add(c.wstat, 0, relax);
+      gb_wstat_add(c.wstat, 1, imp_near);
+      gb_wstat_add(c.wstat, 2, imp_far);
+      gb_wstat_add(c.wstat, 3, expanded);
     }
     if (__ballot(ovf) && gb_lane() == 0) atomicOr(&c.cnt[MS_OVF], 1ull);
   } else {
@@ -413,7 +432,7 @@ __device__ __forceinline__ void ms_phase(const MsCtx &c, const MsIo &io, int act
 }
 
 // Scan form: the step; the state machine advances in a launch of its own.
-template <int W>
+template <int W, bool WIDE>
 __global__ __launch_bounds__(MS_BLOCK)
 __attribute__((amdgpu_waves_per_eu(MsShape<W>::MIN_WAVES))) void ms_step_kernel(MsCtx c,
                                                            const MsCtl *__restrict__ ctl) {
@@ -432,7 +451,7 @@ __attribute__((amdgpu_waves_per_eu(MsShape<W>::MIN_WAVES))) void ms_step_kernel(
   io.n_near = &c.cnt[ctl->a_near];
   io.n_far = &c.cnt[ctl->a_far];
   io.minb = &c.cnt[MS_MINB];
-  ms_phase<W, true>(c, io, act, ctl->a_first, ctl->a_bucket, ctl->a_all != 0);
+  ms_phase<W, true, WIDE>(c, io, act, ctl->a_first, ctl->a_bucket, ctl->a_all != 0);
 }
 
 // Scan form, between two phases: one thread.
@@ -463,7 +482,7 @@ struct MsLoop {
   MsAdds adds[3];
 };
 
-template <int W>
+template <int W, bool WIDE>
 __global__ __launch_bounds__(MS_BLOCK)
 __attribute__((amdgpu_waves_per_eu(MsShape<W>::MIN_WAVES))) void ms_append_kernel(
     MsCtx c, MsLoop *__restrict__ L, uint32_t k, GbProgress *prog) {
@@ -524,7 +543,7 @@ __attribute__((amdgpu_waves_per_eu(MsShape<W>::MIN_WAVES))) void ms_append_kerne
   io.n_near = &add->near;
   io.n_far = &add->far;
   io.minb = &add->minb;
-  ms_phase<W, false>(c, io, act, gb_uniform(s_dev.ctl.a_first), gb_uniform(s_dev.ctl.a_bucket),
+  ms_phase<W, false, WIDE>(c, io, act, gb_uniform(s_dev.ctl.a_first), gb_uniform(s_dev.ctl.a_bucket),
                      gb_uniform((uint32_t)s_dev.ctl.a_all) != 0);
 }
 
@@ -857,15 +876,18 @@ gb_status ms_group(MsCtx c, const int32_t *d_src, int max_phases, bool spans, in
   const int cgrid = ms_compact_grid(c.V);
   // vertices per compaction block: a multiple of MS_CSPAN, cgrid blocks cover V
   const int64_t crange = ((c.V + cgrid - 1) / cgrid + MS_CSPAN - 1) / MS_CSPAN * MS_CSPAN;
+  const bool wide = (uint64_t)V * W * sizeof(uint32_t) > 0xFFFFFFFFull;
+  auto step = wide ? ms_step_kernel<W, true> : ms_step_kernel<W, false>;
+  auto append = wide ? ms_append_kernel<W, true> : ms_append_kernel<W, false>;
   const gb_status gst = gb_drive_phases(prog, MS_AHEAD, st, [&](uint32_t k) {
     if (SCAN) {
-      hipLaunchKernelGGL(ms_step_kernel<W>, dim3(grid), dim3(MS_BLOCK), 0, st, c,
+      hipLaunchKernelGGL(step, dim3(grid), dim3(MS_BLOCK), 0, st, c,
                          (const MsCtl *)ctl);
       hipLaunchKernelGGL(ms_compact_kernel<W>, dim3(cgrid), dim3(MS_BLOCK), 0, st, c,
                          (const MsCtl *)ctl, crange);
       hipLaunchKernelGGL(ms_ctrl_kernel, dim3(1), dim3(1), 0, st, c, ctl, k, prog);
     } else {
-      hipLaunchKernelGGL(ms_append_kernel<W>, dim3(grid), dim3(MS_BLOCK), 0, st, c, loop, k, prog);
+      hipLaunchKernelGGL(append, dim3(grid), dim3(MS_BLOCK), 0, st, c, loop, k, prog);
     }
     return hipGetLastError();
   });
