@@ -67,8 +67,10 @@ struct MsShape {
   static constexpr int STEPS = CHUNK / ES;              // steps per full chunk
   static constexpr int UNROLL = STEPS < 4 ? STEPS : 4;  // steps per group
   static constexpr int G = ES * UNROLL;                 // edges per group (<= 64)
-  // waves per SIMD the step kernel's registers must allow (1: no bound)
-  static constexpr int MIN_WAVES = W >= 16 ? 6 : 1;
+  // waves per SIMD the step kernel's registers must allow (1: no bound).  8 (62
+  // VGPRs, no spills) against 6: R-MAT 24 with 32 sources 33.7 and 40.3 ms, R-MAT
+  // 22 with 16 6.6 and 7.2, with 64 17.7 and 18.7; with 8 sources level.
+  static constexpr int MIN_WAVES = W >= 16 ? 8 : 1;
 };
 constexpr int32_t MS_MIN_CHUNK = 32;  // for queue capacities
 constexpr int MS_NCAP = 128, MS_FCAP = 128;  // LDS append buffers per wave (entries)
