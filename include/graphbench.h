@@ -143,7 +143,8 @@ gb_status gb_separate(gb_graph g, uint32_t light_max, int32_t *d_col_out,
 
 /* ---- SSSP (delta-stepping) --------------------------------------------------*/
 typedef struct gb_sssp_params {
-  uint32_t delta;     /* bucket width (0 = plain rule max_w / avg_degree) */
+  uint32_t delta;     /* bucket width (0 = plain rule max_w / avg_degree); small
+                       * buckets may be solved several at a time */
   uint32_t light_max; /* light/heavy threshold (0 = delta) */
   int32_t max_phases; /* safety cap on phases (0 = none) */
   int32_t reserved;
