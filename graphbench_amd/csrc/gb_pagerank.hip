@@ -532,8 +532,13 @@ __global__ __launch_bounds__(PS_BLOCK) void ps_iter_kernel(
   __shared__ float s_val[PS_CHUNK];
   __shared__ int32_t s_rp[PS_MAX_TILE + 1];
   __shared__ F2 s_carry;
-  if (*done) return;  // by an earlier launch
+  __shared__ int32_t s_done;
   const int tid = threadIdx.x, lane = gb_lane();
+  // One thread reads the flag for its block: block 0 of this launch may be
+  // setting it, and a block whose waves read it themselves could go on with some
+  // of them, over partial sums and row bounds that the others had not left in
+  // LDS.  The barriers of the block sum below publish it.
+  if (tid == 0) s_done = *done;
   const int32_t nb = (int32_t)gridDim.x;
   const double *pin = part + (size_t)(k & 1) * 2 * PS_MAX_BLOCKS;
   double *pout = part + (size_t)((k + 1) & 1) * 2 * PS_MAX_BLOCKS;
@@ -548,6 +553,7 @@ __global__ __launch_bounds__(PS_BLOCK) void ps_iter_kernel(
   }
   for (int i = tid; i <= nrows; i += PS_BLOCK) s_rp[i] = irp[r0 + i];
   block_sum2_f64(ra, da, s_red);
+  if (s_done) return;  // the loop has ended: by an earlier launch, or below by block 0
   const double residual = k == 0 ? (double)INFINITY : ra, dangling = da;
   const bool stop = residual < tol || k >= max_iter;
   if (blockIdx.x == 0 && tid == 0) {
