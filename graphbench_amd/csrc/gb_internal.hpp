@@ -211,27 +211,40 @@ void gb_learned_release();
 // Gives back the scratch kept for CSR builds unless one is running.
 bool gb_csr_trim();
 
-template <class Launch>
-gb_status gb_drive_phases(GbProgress *p, uint32_t ahead, hipStream_t st, Launch launch) {
+// The loop of gb_drive_phases without its stream: query() is hipSuccess once
+// everything launched has run, hipErrorNotReady before.  The difference of the
+// two phase numbers is signed: a record ahead of the host admits a launch.
+template <class Launch, class Query>
+gb_status gb_drive_loop(GbProgress *p, uint32_t ahead, Launch launch, Query query) {
   uint32_t k = 0, spins = 0;
-  while (!__atomic_load_n(&p->done, __ATOMIC_ACQUIRE)) {
-    if (k - __atomic_load_n(&p->started, __ATOMIC_RELAXED) < ahead) {
+  auto done = [&]() { return __atomic_load_n(&p->done, __ATOMIC_ACQUIRE) != 0; };
+  auto room = [&]() {
+    return (int32_t)(k - __atomic_load_n(&p->started, __ATOMIC_RELAXED)) < (int32_t)ahead;
+  };
+  while (!done()) {
+    if (room()) {
       GB_HIP(launch(k));
       k++;
       spins = 0;
     } else if (++spins % 65536 == 0) {
-      // a stream that has run dry, or failed, makes no more progress
-      const hipError_t e = hipStreamQuery(st);
-      if (e == hipErrorNotReady) {
-        (void)hipGetLastError();
-      } else {
-        GB_HIP(e);
-        if (!__atomic_load_n(&p->done, __ATOMIC_ACQUIRE) &&
-            __atomic_load_n(&p->started, __ATOMIC_RELAXED) != k)
-          return gb_fail(GB_ERR_HIP, "phase loop made no progress");
-      }
+      // a stream that has run dry, or failed, makes no more progress: if it has
+      // left no room for a launch by then, it never will
+      const hipError_t e = query();
+      if (e == hipErrorNotReady) continue;
+      GB_HIP(e);
+      if (!done() && !room()) return gb_fail(GB_ERR_HIP, "phase loop made no progress");
     }
   }
+  return GB_OK;
+}
+
+template <class Launch>
+gb_status gb_drive_phases(GbProgress *p, uint32_t ahead, hipStream_t st, Launch launch) {
+  GB_TRY(gb_drive_loop(p, ahead, launch, [st]() {
+    const hipError_t e = hipStreamQuery(st);
+    if (e == hipErrorNotReady) (void)hipGetLastError();
+    return e;
+  }));
   GB_HIP(hipStreamSynchronize(st));
   return GB_OK;
 }

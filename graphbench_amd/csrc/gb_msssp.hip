@@ -456,7 +456,7 @@ __attribute__((amdgpu_waves_per_eu(MsShape<W>::MIN_WAVES))) void ms_step_kernel(
   ms_phase<W, true, WIDE>(c, io, act, ctl->a_first, ctl->a_bucket, ctl->a_all != 0);
 }
 
-// Scan form, between two phases: one thread.
+// Scan form, between two phases: one thread.  k: the phase before (~0: none).
 __global__ void ms_ctrl_kernel(MsCtx c, MsCtl *__restrict__ ctl, uint32_t k, GbProgress *prog) {
   MsCtl s = *ctl;
   ms_ctl_advance(s, c.cnt);
@@ -873,7 +873,8 @@ gb_status ms_group(MsCtx c, const int32_t *d_src, int max_phases, bool spans, in
   // the append form's seeds count as appended by the phase before phase 0
   hipLaunchKernelGGL((ms_seed_kernel<W, SCAN>), dim3(1), dim3(64), 0, st, c, d_src,
                      SCAN ? &c.cnt[MS_NEAR0] : &loop->adds[2].near);
-  if (SCAN) hipLaunchKernelGGL(ms_ctrl_kernel, dim3(1), dim3(1), 0, st, c, ctl, 0u, prog);
+  // the first advance comes before phase 0: it reports no phase begun
+  if (SCAN) hipLaunchKernelGGL(ms_ctrl_kernel, dim3(1), dim3(1), 0, st, c, ctl, ~0u, prog);
   GB_HIP(hipGetLastError());
   const int cgrid = ms_compact_grid(c.V);
   // vertices per compaction block: a multiple of MS_CSPAN, cgrid blocks cover V
