@@ -447,6 +447,12 @@ CsrWork &csr_work() {
   return *w;
 }
 
+// Whether [a, a + na) and [b, b + nb) share a byte.
+bool overlap(const void *a, size_t na, const void *b, size_t nb) {
+  const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+  return a && b && x < y + nb && y < x + na;
+}
+
 int grid_for(int64_t n) {
   return (int)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, (int64_t)gb_num_cus() * 16));
 }
@@ -579,12 +585,22 @@ gb_status csr_build(CsrWork &k, int32_t V, int64_t E, const int32_t *d_src, cons
   GB_TRY(k.hist.ensure(sizeof(uint32_t) * ntiles * D));
   GB_TRY(k.gsum.ensure(sizeof(uint32_t) * ngroups * D));
   GB_TRY(k.total.ensure(sizeof(uint32_t) * D));
+  // An output may take the place of the keys (d_src; a transpose in place:
+  // d_tcol == d_col).  Where the first pass writes the caller's arrays, tiles
+  // would write them while others read their keys: the keys move away first.
+  const bool aside = passes % 2 == 1 && (overlap(d_src, sizeof(int32_t) * E, d_col, sizeof(int32_t) * E) ||
+                                         overlap(d_src, sizeof(int32_t) * E, d_w_out, (size_t)WB * E));
+  if (aside) GB_TRY(k.k[1].ensure(sizeof(int32_t) * E));
   int *bad = k.flag.as<int>();
   uint32_t *hist = k.hist.as<uint32_t>(), *gsum = k.gsum.as<uint32_t>(),
            *total = k.total.as<uint32_t>();
   GB_HIP(hipMemsetAsync(bad, 0, sizeof(int), st));
   const int32_t *key = d_src, *val = d_dst;
   const void *w = d_w;
+  if (aside) {
+    GB_HIP(hipMemcpyAsync(k.k[1].p, d_src, sizeof(int32_t) * E, hipMemcpyDeviceToDevice, st));
+    key = k.k[1].as<int32_t>();  // pass 0 writes k[0], and pass 1, if any, reads that
+  }
   for (int p = 0; p < passes; p++) {
     const int shift = p * db;
     const bool to_caller = (passes - 1 - p) % 2 == 0;

@@ -116,7 +116,9 @@ gb_status gb_edge_parts(int64_t E, const int32_t *d_src, const int32_t *d_dst,
  * of w_bytes 4 (uint32) or 8 (double) carried along (w_bytes 0: none).
  * d_row_ptr has V+1 entries, d_col (and d_w_out) E.  Endpoints outside
  * [0, V) are rejected.  gb_csr_transpose: the reverse CSR of a CSR (rows of
- * the transpose keep the order of their source rows). */
+ * the transpose keep the order of their source rows).  An output may take the
+ * place of d_src (of d_col in a transpose, of d_row_ptr for d_trow_ptr), not
+ * that of another input. */
 gb_status gb_csr_from_edges(int32_t V, int64_t E, const int32_t *d_src,
                             const int32_t *d_dst, const void *d_w, int32_t w_bytes,
                             int32_t *d_row_ptr, int32_t *d_col, void *d_w_out,
