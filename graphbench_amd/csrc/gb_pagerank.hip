@@ -454,17 +454,51 @@ __global__ __launch_bounds__(PR_BLOCK) void pr_fixup_kernel(
 //   * a rank is read and written by its row's owner alone, so the ranks stay in
 //     the caller's array; contributions and partials alternate;
 //   * launches run ahead of the device (gb_drive_phases).
-// A block stages up to PS_CHUNK gathered contributions at a time in LDS, all
-// reads of a chunk in flight together, and sums each row with a power-of-two
-// group of lanes, a row of many edges per lane with a wave (compensated FP32,
-// fixed order); a row that goes past the chunk carries its sum on.
+// A block stages its rows' gathered contributions (up to PS_CHUNK) in LDS, all
+// reads in flight together, and sums each row with a power-of-two group of
+// lanes, a row of many edges per lane with a wave (compensated FP32, fixed order).
+// Rows of more than PS_ROW edges are summed in pieces by a launch of their own
+// ahead of each iteration, on graphs that have such rows: in one block a row
+// costs 4.7 us per 4096 edges, beside which the other blocks wait (20 iterations, a
+// row of 2^16 / 2^18 / 2^20 in-edges: 1.67 / 6.15 / 24.4 ms with the row in one block,
+// 0.25 / 0.26 / 0.29 ms in pieces; row blocks 0.41 / 0.47 / 0.57 ms).  A tile holds
+// fewer items than such a row, so at most its first row is one.
 constexpr int PS_BLOCK = 256;
 constexpr int PS_CHUNK = 4096;
 constexpr int PS_LONG = 16;  // edges per lane of a group from which a wave takes the row
 constexpr int PS_MAX_TILE = 2048;    // rows + edges per tile
+constexpr int PS_ROW = PS_CHUNK - PS_MAX_TILE;
+static_assert(PS_ROW >= PS_MAX_TILE, "a longer row ends in a tile as its first row");
+constexpr int PS_PIECE = 2048;       // edges per piece of a long row
 constexpr int PS_MAX_BLOCKS = 1024;  // partials summed by every block
 constexpr int64_t PS_MAX_ITEMS = (int64_t)PS_MAX_TILE * PS_MAX_BLOCKS;
 constexpr int PS_AHEAD = 6, PS_REPORT = 3;  // launches ahead, iterations per report
+
+// The pieces [first, first + n) of the long row that ends in a tile (n 0: none).
+struct PsLong {
+  int32_t first, n;
+};
+
+// One thread per tile; the pieces of a row one after another.
+__global__ void ps_long_list_kernel(int32_t ntiles, const int32_t *__restrict__ irp,
+                                    const int32_t *__restrict__ tile_row,
+                                    PsLong *__restrict__ longs, int2 *__restrict__ pieces,
+                                    int32_t *__restrict__ count) {
+  const int32_t t = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (t >= ntiles) return;
+  PsLong l = {0, 0};
+  const int32_t r0 = tile_row[t];
+  if (tile_row[t + 1] > r0) {
+    const int32_t e0 = irp[r0], e1 = irp[r0 + 1];
+    if (e1 - e0 > PS_ROW) {
+      l.n = (e1 - e0 + PS_PIECE - 1) / PS_PIECE;
+      l.first = atomicAdd(count, l.n);
+      for (int32_t k = 0; k < l.n; k++)
+        pieces[l.first + k] = make_int2(e0 + k * PS_PIECE, min(e0 + (k + 1) * PS_PIECE, e1));
+    }
+  }
+  longs[t] = l;
+}
 
 __global__ __launch_bounds__(PS_BLOCK) void ps_init_kernel(
     int32_t V, const float *__restrict__ x0, const float *__restrict__ inv_od,
@@ -507,12 +541,8 @@ __device__ __forceinline__ void ps_stage(const int32_t *__restrict__ ic, int n,
     if (tid + m * PS_BLOCK < n) s_val[tid + m * PS_BLOCK] = g[m];
 }
 
-// Compensated sum of val[b .. e) by the G lanes of a group (lane `sub` of it),
-// the same in every lane: strided partial sums, then a butterfly that merges
-// the lower lane's sum first on both sides.
-__device__ __forceinline__ F2 ps_sum(const float *val, int b, int e, int sub, int G) {
-  F2 acc = {0.0f, 0.0f};
-  for (int j = b + sub; j < e; j += G) f2_add(acc, val[j]);
+// Sum over the lanes of a group of G, in a fixed order, the same in every lane.
+__device__ __forceinline__ F2 ps_merge(F2 acc, int sub, int G) {
   for (int m = G >> 1; m >= 1; m >>= 1) {
     F2 o;
     o.s = __shfl_xor(acc.s, m, GB_WAVE);
@@ -522,16 +552,55 @@ __device__ __forceinline__ F2 ps_sum(const float *val, int b, int e, int sub, in
   return acc;
 }
 
+// Compensated sum of val[b .. e) by the G lanes of a group (lane `sub` of it),
+// the same in every lane: strided partial sums, then a butterfly that merges
+// the lower lane's sum first on both sides.
+__device__ __forceinline__ F2 ps_sum(const float *val, int b, int e, int sub, int G) {
+  F2 acc = {0.0f, 0.0f};
+  for (int j = b + sub; j < e; j += G) f2_add(acc, val[j]);
+  return ps_merge(acc, sub, G);
+}
+
+// One block per piece of a long row: its compensated sum, in a fixed order.
+__global__ __launch_bounds__(PS_BLOCK) void ps_long_kernel(const int2 *__restrict__ pieces,
+                                                           const int32_t *__restrict__ icol,
+                                                           const float *__restrict__ c_old,
+                                                           F2 *__restrict__ psum) {
+  constexpr int PER = PS_PIECE / PS_BLOCK;
+  __shared__ F2 s_w[PS_BLOCK / GB_WAVE];
+  const int2 p = pieces[blockIdx.x];
+  const int tid = threadIdx.x, n = p.y - p.x;  // n >= 1
+  int32_t u[PER];
+  float v[PER];
+#pragma unroll
+  for (int m = 0; m < PER; m++) u[m] = icol[p.x + min(tid + m * PS_BLOCK, n - 1)];
+#pragma unroll
+  for (int m = 0; m < PER; m++) v[m] = c_old[u[m]];
+  F2 acc = {0.0f, 0.0f};
+#pragma unroll
+  for (int m = 0; m < PER; m++)
+    if (tid + m * PS_BLOCK < n) f2_add(acc, v[m]);
+  acc = ps_merge(acc, gb_lane(), GB_WAVE);
+  if (gb_lane() == 0) s_w[tid / GB_WAVE] = acc;
+  __syncthreads();
+  if (tid == 0) {
+#pragma unroll
+    for (int k = 1; k < PS_BLOCK / GB_WAVE; k++) acc = f2_merge(acc, s_w[k]);
+    psum[blockIdx.x] = acc;
+  }
+}
+
+// longs, psum: null on graphs without long rows.
 __global__ __launch_bounds__(PS_BLOCK) void ps_iter_kernel(
     int32_t V, const int32_t *__restrict__ irp, const int32_t *__restrict__ icol,
-    const int32_t *__restrict__ tile_row, const float *__restrict__ inv_od, float *__restrict__ x,
+    const int32_t *__restrict__ tile_row, const PsLong *__restrict__ longs,
+    const F2 *__restrict__ psum, const float *__restrict__ inv_od, float *__restrict__ x,
     const float *__restrict__ c_old, float *__restrict__ c_new, double *__restrict__ part,
     int32_t *__restrict__ done, int32_t k, int32_t max_iter, double tol, float damping,
     GbProgress *prog) {
   __shared__ double s_red[PS_BLOCK / 64][2];
   __shared__ float s_val[PS_CHUNK];
   __shared__ int32_t s_rp[PS_MAX_TILE + 1];
-  __shared__ F2 s_carry;
   __shared__ int32_t s_done;
   const int tid = threadIdx.x, lane = gb_lane();
   // One thread reads the flag for its block: block 0 of this launch may be
@@ -543,6 +612,7 @@ __global__ __launch_bounds__(PS_BLOCK) void ps_iter_kernel(
   const double *pin = part + (size_t)(k & 1) * 2 * PS_MAX_BLOCKS;
   double *pout = part + (size_t)((k + 1) & 1) * 2 * PS_MAX_BLOCKS;
   const int32_t r0 = tile_row[blockIdx.x], nrows = tile_row[blockIdx.x + 1] - r0;
+  const PsLong lg = longs ? longs[blockIdx.x] : PsLong{0, 0};
   double ra = 0.0, da = 0.0;
 #pragma unroll
   for (int i = 0; i < PS_MAX_BLOCKS / PS_BLOCK; i++) {
@@ -552,6 +622,11 @@ __global__ __launch_bounds__(PS_BLOCK) void ps_iter_kernel(
     da += j < nb ? b : 0.0;
   }
   for (int i = tid; i <= nrows; i += PS_BLOCK) s_rp[i] = irp[r0 + i];
+  F2 lsum = {0.0f, 0.0f};  // of row 0, where it is long; the first wave's
+  if (lg.n > 0 && tid < GB_WAVE) {
+    for (int32_t j = lane; j < lg.n; j += GB_WAVE) lsum = f2_merge(lsum, psum[lg.first + j]);
+    lsum = ps_merge(lsum, lane, GB_WAVE);
+  }
   block_sum2_f64(ra, da, s_red);
   if (s_done) return;  // the loop has ended: by an earlier launch, or below by block 0
   const double residual = k == 0 ? (double)INFINITY : ra, dangling = da;
@@ -571,54 +646,44 @@ __global__ __launch_bounds__(PS_BLOCK) void ps_iter_kernel(
   double res = 0.0, dang = 0.0;
   if (nrows > 0) {
     // (the barriers of the block sum came after the writes of s_rp)
-    const int32_t e0 = s_rp[0], e1 = s_rp[nrows];
+    const int32_t first = lg.n > 0 ? 1 : 0;  // rows summed here: [first, nrows)
+    const int32_t e0 = s_rp[first], e1 = s_rp[nrows];
+    // row first has at most PS_ROW edges and the others lie in the tile
+    const int n = e1 - e0;
     // lanes per row: as many as keep every row in one pass, at most a wave
     int glog = 0;
     while (glog < 6 && (nrows << (glog + 1)) <= PS_BLOCK) glog++;
     const int G = 1 << glog, sub = lane & (G - 1), step = PS_BLOCK >> glog;
-    for (int32_t c0 = e0; c0 == e0 || c0 < e1; c0 += PS_CHUNK) {  // block-uniform
-      const int32_t c1 = min(c0 + PS_CHUNK, e1);
-      const int n = c1 - c0;
-      if (n > 8 * PS_BLOCK)
-        ps_stage<16>(icol + c0, n, c_old, s_val);
-      else if (n > 4 * PS_BLOCK)
-        ps_stage<8>(icol + c0, n, c_old, s_val);
-      else if (n > 0)
-        ps_stage<4>(icol + c0, n, c_old, s_val);
-      const F2 carry = c0 > e0 ? s_carry : F2{0.0f, 0.0f};
-      __syncthreads();
-      // row i, whose part in this chunk is [b, e) and sums to acc
-      auto finish = [&](int i, int32_t rs, int32_t re, int32_t b, int32_t e, F2 acc) {
-        if (rs < c0 && e > b) acc = f2_merge(carry, acc);
-        const bool here = rs < re ? (re > c0 && re <= c1) : c0 == e0;
-        if (here) {
-          const int32_t v = r0 + i;
-          const float xn = base + damping * f2_value(acc), io = inv_od[v];
-          res += fabs((double)xn - (double)x[v]);
-          x[v] = xn;
-          c_new[v] = xn * io;
-          if (io == 0.0f) dang += (double)xn;
-        } else if (e > b && re > c1) {
-          s_carry = acc;  // the one row that goes past this chunk
-        }
-      };
-      for (int i0 = 0; i0 < nrows; i0 += step) {  // block-uniform
-        const int i = i0 + (tid >> glog);
-        const int32_t rs = i < nrows ? s_rp[i] : e1, re = i < nrows ? s_rp[i + 1] : e1;
-        const int32_t b = max(rs, c0), e = min(re, c1);
-        const bool is_long = G < GB_WAVE && e - b > PS_LONG * G;
-        const F2 acc = ps_sum(s_val, b - c0, is_long ? b - c0 : e - c0, sub, G);
-        if (sub == 0 && i < nrows && !is_long) finish(i, rs, re, b, e, acc);
-        uint64_t longs = __ballot(is_long && sub == 0);
-        while (longs) {  // wave-uniform
-          const int l = __ffsll((unsigned long long)longs) - 1;
-          longs &= longs - 1;
-          const int32_t lb = __shfl(b, l, GB_WAVE), le = __shfl(e, l, GB_WAVE);
-          const F2 la = ps_sum(s_val, lb - c0, le - c0, lane, GB_WAVE);
-          if (lane == l) finish(i, rs, re, b, e, la);
-        }
+    if (n > 8 * PS_BLOCK)
+      ps_stage<16>(icol + e0, n, c_old, s_val);
+    else if (n > 4 * PS_BLOCK)
+      ps_stage<8>(icol + e0, n, c_old, s_val);
+    else if (n > 0)
+      ps_stage<4>(icol + e0, n, c_old, s_val);
+    auto finish = [&](int i, F2 acc) {
+      const int32_t v = r0 + i;
+      const float xn = base + damping * f2_value(acc), io = inv_od[v];
+      res += fabs((double)xn - (double)x[v]);
+      x[v] = xn;
+      c_new[v] = xn * io;
+      if (io == 0.0f) dang += (double)xn;
+    };
+    if (first && tid == 0) finish(0, lsum);
+    __syncthreads();
+    for (int i0 = first; i0 < nrows; i0 += step) {  // block-uniform
+      const int i = i0 + (tid >> glog);
+      const int b = i < nrows ? s_rp[i] - e0 : n, e = i < nrows ? s_rp[i + 1] - e0 : n;
+      const bool is_long = G < GB_WAVE && e - b > PS_LONG * G;
+      const F2 acc = ps_sum(s_val, b, is_long ? b : e, sub, G);
+      if (sub == 0 && i < nrows && !is_long) finish(i, acc);
+      uint64_t many = __ballot(is_long && sub == 0);
+      while (many) {  // wave-uniform
+        const int l = __ffsll((unsigned long long)many) - 1;
+        many &= many - 1;
+        const int32_t lb = __shfl(b, l, GB_WAVE), le = __shfl(e, l, GB_WAVE);
+        const F2 la = ps_sum(s_val, lb, le, lane, GB_WAVE);
+        if (lane == l) finish(i, la);
       }
-      __syncthreads();
     }
   }
   block_sum2_f64(res, dang, s_red);
@@ -1557,7 +1622,7 @@ void build_row_blocks(const std::vector<int32_t> &rp, int nb, std::vector<RowBlo
 }
 
 struct PrWork {
-  DevBuf xa, xb, ca, cb, tail, head, pres, pdang, fres, fdang, state, counter, ps_done;
+  DevBuf xa, xb, ca, cb, tail, head, pres, pdang, fres, fdang, state, counter, ps_done, ps_sum;
   // the instantiated hipGraph of CH iterations and what its kernels were
   // captured with (graph id, form, sizes, every device pointer): replayed by
   // later calls with the same key instead of captured again
@@ -1578,7 +1643,7 @@ struct PrWork {
   void release() {
     for (DevBuf *b :
          {&xa, &xb, &ca, &cb, &tail, &head, &pres, &pdang, &fres, &fdang, &state, &counter,
-          &ps_done})
+          &ps_done, &ps_sum})
       b->release();
     for (hipEvent_t e : events) (void)hipEventDestroy(e);
     events.clear();
@@ -2018,6 +2083,22 @@ static gb_status pagerank_small(gb_graph g, const gb_pr_params *p, float *d_x, g
     g->pr_ntiles = nb;
   }
   PrWork &w = g_prw;
+  if (g->ps_tile != tile) {  // the long rows' pieces, once per handle
+    DevBuf count;
+    GB_TRY(g->ps_long.ensure(sizeof(PsLong) * nb));
+    GB_TRY(g->ps_pieces.ensure(sizeof(int2) * (2 * (g->E / PS_PIECE) + 1)));
+    GB_TRY(count.ensure(sizeof(int32_t)));
+    GB_HIP(hipMemsetAsync(count.p, 0, sizeof(int32_t), st));
+    hipLaunchKernelGGL(ps_long_list_kernel, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, st,
+                       (int32_t)nb, g->rrp, g->pr_tile_row.as<int32_t>(),
+                       g->ps_long.as<PsLong>(), g->ps_pieces.as<int2>(), count.as<int32_t>());
+    GB_HIP(hipGetLastError());
+    GB_HIP(hipMemcpyAsync(&g->ps_npieces, count.p, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    GB_HIP(hipStreamSynchronize(st));
+    g->ps_tile = (int32_t)tile;
+  }
+  const int32_t np = g->ps_npieces;
+  if (np > 0) GB_TRY(w.ps_sum.ensure(sizeof(F2) * np));
   GB_TRY(w.ca.ensure(sizeof(float) * V));
   GB_TRY(w.cb.ensure(sizeof(float) * V));
   GB_TRY(w.pres.ensure(sizeof(double) * 4 * PS_MAX_BLOCKS));
@@ -2032,10 +2113,17 @@ static gb_status pagerank_small(gb_graph g, const gb_pr_params *p, float *d_x, g
   hipLaunchKernelGGL(ps_init_kernel, dim3((unsigned)nb), dim3(PS_BLOCK), 0, st, V, p->d_x0, inv,
                      rows, d_x, c[0], part, done);
   GB_HIP(hipGetLastError());
+  const PsLong *longs = np > 0 ? g->ps_long.as<PsLong>() : nullptr;
+  F2 *psum = np > 0 ? w.ps_sum.as<F2>() : nullptr;
   const gb_status gst = gb_drive_phases(prog, PS_AHEAD, st, [&](uint32_t k) {
+    if (np > 0)
+      hipLaunchKernelGGL(ps_long_kernel, dim3((unsigned)np), dim3(PS_BLOCK), 0, st,
+                         (const int2 *)g->ps_pieces.as<int2>(), g->rcol, (const float *)c[k & 1],
+                         psum);
     hipLaunchKernelGGL(ps_iter_kernel, dim3((unsigned)nb), dim3(PS_BLOCK), 0, st, V, g->rrp,
-                       g->rcol, rows, inv, d_x, (const float *)c[k & 1], c[(k + 1) & 1], part,
-                       done, (int32_t)k, p->max_iter, p->tol, (float)p->damping, prog);
+                       g->rcol, rows, longs, (const F2 *)psum, inv, d_x, (const float *)c[k & 1],
+                       c[(k + 1) & 1], part, done, (int32_t)k, p->max_iter, p->tol,
+                       (float)p->damping, prog);
     return hipGetLastError();
   });
   if (gst != GB_OK) {
