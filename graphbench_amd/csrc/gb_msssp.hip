@@ -865,6 +865,7 @@ gb_status ms_group(MsCtx c, const int32_t *d_src, int max_phases, bool spans, in
   hc.sp.few = ms_few(W);
   hc.sp.many = 16 * ms_few(W);
   hc.sp.leap = 8;
+  hc.sp.most = SPAN_MOST;
   MsLoop *loop = w.ctl.as<MsLoop>();
   MsCtl *ctl = (MsCtl *)(loop + 1);
   const int64_t fill = std::max<int64_t>(V * W / 4, GB_WSTAT * nwaves);

@@ -685,6 +685,7 @@ gb_status sssp_engine_run(const std::vector<SGraph<typename Tr::W>> &hg,
   hc.sp.few = SSSP_FEW;
   hc.sp.many = SSSP_MANY;
   hc.sp.leap = 2;
+  hc.sp.most = SPAN_MOST;
   const int64_t nstat = GB_WSTAT * nwaves;
   hipLaunchKernelGGL(sssp_begin_kernel, dim3((unsigned)((nstat + 255) / 256)), dim3(256), 0, st,
                      loop, hc, nstat, wstat, cnt);

@@ -20,20 +20,32 @@
 // grows after a range whose phases held few queue entries on average and
 // halves after one with many.  Distances are exact for any sequence of ranges.
 // One source of R-MAT 20, 16.8 M edges: 131 phases become 27; 8 sources of
-// R-MAT 16: 169 become 38; a 300 x 300 grid: 3061 become 655.
+// R-MAT 16: 169 become 38; a 300 x 300 grid: 3061 become 578.
+// A range of SPAN_MOST phases or more does not widen the next one: merging saves
+// the phases at a range's ends, few beside that many, while on graphs of high
+// diameter, whose phases stay small, a wider range only relaxes more edges again.
+// 64 sources, without the limit / 16 / 32 / 64 / 128: a 1000 x 1000 grid 344 / 172 /
+// 140 / 147 / 175 ms (single buckets 299), a 30 x 20000 strip 3057 / 798 / 734 / 711 /
+// 736 ms, a 300 x 300 grid 21.1 / 26.4 / 19.7 / 18.9 / 19.2 ms; R-MAT and uniform
+// graphs stay under it.  A leap may go to twice the limit: held to the limit itself,
+// 8 sources of R-MAT 16 take 48 phases instead of 38.
+constexpr uint32_t SPAN_MOST = 64;
 struct SpanCtl {
   uint64_t span;         // buckets per range (0 and 1: one)
   uint64_t work, steps;  // queue entries and phases of the current range
   uint32_t adapt;        // 0: single buckets
   uint32_t few, many;    // entries per phase below / above which the span moves
   uint32_t leap;         // the factor below few / 8
+  uint32_t most;         // phases from which a range does not widen the next (0: no limit)
 };
 __host__ __device__ inline void span_after_range(SpanCtl &c) {
   if (!c.adapt) return;
   if (c.span == 0) c.span = 1;
   if (c.work < (uint64_t)c.few * c.steps) {
-    if (c.span < ((uint64_t)1 << 40))
-      c.span *= c.work < (uint64_t)(c.few / 8) * c.steps ? c.leap : 2;
+    const bool leap = c.work < (uint64_t)(c.few / 8) * c.steps &&
+                      (!c.most || c.steps * c.leap <= 2 * (uint64_t)c.most);
+    if (c.span < ((uint64_t)1 << 40) && (!c.most || c.steps < c.most))
+      c.span *= leap ? c.leap : 2;
   } else if (c.work > (uint64_t)c.many * c.steps && c.span > 1) {
     c.span /= 2;
   }
