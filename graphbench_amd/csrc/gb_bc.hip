@@ -268,13 +268,18 @@ __global__ __launch_bounds__(SM_BLOCK) void bcw_small_kernel(SmGraph<double> G, 
   auto tight = [&](uint32_t u, uint32_t x, double w) {
     return SmF64::bits(__dadd_rn(SmF64::val(s.dist[u]), w)) == s.dist[x];
   };
+  // an infinite weight is tight to a vertex that is not reached, as in the
+  // kernels above, but counts for no order
+  auto leads = [&](uint32_t u, uint32_t x, double w) {
+    return tight(u, x, w) && s.dist[x] != SmF64::inf_bits();
+  };
   sm_expand(
       s, G, reached, sweep, [&](uint32_t i) { return order[i]; },
       [&](auto &in, auto &u, auto &x, auto &w) {
         constexpr int U = sizeof(in) / sizeof(in[0]);
 #pragma unroll
         for (int k = 0; k < U; k++)
-          if (in[k] && tight(u[k], x[k], w[k]))
+          if (in[k] && leads(u[k], x[k], w[k]))
             __hip_atomic_fetch_add(&indeg[x[k]], 1, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
       });
@@ -300,7 +305,7 @@ __global__ __launch_bounds__(SM_BLOCK) void bcw_small_kernel(SmGraph<double> G, 
 #pragma unroll
           for (int k = 0; k < U; k++) {
             left[k] = 0;
-            if (in[k] && x[k] != (uint32_t)s0 && tight(u[k], x[k], w[k])) {
+            if (in[k] && x[k] != (uint32_t)s0 && leads(u[k], x[k], w[k])) {
               __hip_atomic_fetch_add(&sigma[x[k]], su[k], __ATOMIC_RELAXED,
                                      __HIP_MEMORY_SCOPE_WORKGROUP);
               left[k] = __hip_atomic_fetch_add(&indeg[x[k]], -1, __ATOMIC_RELAXED,
