@@ -458,7 +458,7 @@ gb_status bcs_batch(gb_graph g, const int32_t *h_sources, int32_t ns, int32_t *m
   BcWork &w = g_bcw;
   const int32_t V = g->V;
   const double width = g->split64_valid ? g->split64_delta : 0.1;
-  GB_TRY(w.loff.ensure(sizeof(uint32_t) * (size_t)BCS_SOURCES * (V + 1)));
+  GB_TRY(w.loff.ensure(sizeof(uint32_t) * (size_t)std::min(ns, BCS_SOURCES) * (V + 1)));
   for (int32_t g0 = 0; g0 < ns; g0 += BCS_SOURCES) {
     const int n = std::min<int32_t>(BCS_SOURCES, ns - g0);
     BcsSources src{};
