@@ -2074,6 +2074,7 @@ static gb_status pagerank_small(gb_graph g, const gb_pr_params *p, float *d_x, g
   const int64_t tile = std::max<int64_t>(1024, (items + PS_MAX_BLOCKS - 1) / PS_MAX_BLOCKS);
   const int64_t nb = (items + tile - 1) / tile;
   if (g->pr_tile_items != tile || g->pr_tile_relabeled) {
+    g->pr_tile_items = 0;  // an allocation that fails below leaves no tiles
     GB_TRY(g->pr_tile_row.ensure(sizeof(int32_t) * (nb + 1)));
     GB_TRY(g->pr_tile_edge.ensure(sizeof(int32_t) * (nb + 1)));
     GB_TRY(gb_merge_path_split(V, g->rrp, tile, nb, g->pr_tile_row.as<int32_t>(),
@@ -2301,6 +2302,7 @@ static gb_status pagerank_run(gb_graph g, const gb_pr_params *p, float *d_x, gb_
                     PB_SHAPES[pb].bsl, pb_piece(), st));
   if (!rb && !pb && (g->pr_tile_items != tile || g->pr_tile_relabeled != relabel)) {
     const int64_t ntiles = ((int64_t)V + g->E + tile - 1) / tile;
+    g->pr_tile_items = 0;  // an allocation that fails below leaves no tiles
     GB_TRY(g->pr_tile_row.ensure(sizeof(int32_t) * (ntiles + 1)));
     GB_TRY(g->pr_tile_edge.ensure(sizeof(int32_t) * (ntiles + 1)));
     GB_TRY(gb_merge_path_split(V, irp, tile, ntiles, g->pr_tile_row.as<int32_t>(),
@@ -2316,6 +2318,7 @@ static gb_status pagerank_run(gb_graph g, const gb_pr_params *p, float *d_x, gb_
     std::vector<RowBlock> blocks;
     std::vector<LongRow> longs;
     build_row_blocks(hrp, rb, blocks, longs);
+    g->pr_rb_nb = 0;  // an allocation that fails below leaves no blocks
     GB_TRY(g->pr_rb.ensure(sizeof(RowBlock) * blocks.size()));
     GB_TRY(g->pr_rb_long.ensure(sizeof(LongRow) * (longs.size() + 1)));
     GB_HIP(hipMemcpyAsync(g->pr_rb.p, blocks.data(), sizeof(RowBlock) * blocks.size(),
