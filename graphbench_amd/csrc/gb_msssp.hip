@@ -925,9 +925,19 @@ gb_status ms_group_shape(MsCtx c, const int32_t *d_src, int max_phases, const Ms
                          hipStream_t st, uint32_t *out_rows, MsStats &sx) {
   c.cshift = sh.cshift;
   const int grid = gb_num_cus() * sh.per_cu;
-  auto run = [&](bool spans) {
-    return sh.scan ? ms_group<W, true>(c, d_src, max_phases, spans, grid, st, out_rows, sx)
-                   : ms_group<W, false>(c, d_src, max_phases, spans, grid, st, out_rows, sx);
+  auto run = [&](bool spans) -> gb_status {
+    if (!sh.scan) {
+      const gb_status s =
+          ms_group<W, false>(c, d_src, max_phases, spans, grid, st, out_rows, sx);
+      if (s != GB_ERR_NOMEM) return s;
+      // no room for the append form's third queue and masks: the scan form does
+      // with two queues and one mask
+      MsWork &w = g_msw;
+      w.mask[1].release();
+      w.mask[2].release();
+      w.q[2].release();
+    }
+    return ms_group<W, true>(c, d_src, max_phases, spans, grid, st, out_rows, sx);
   };
   // Buckets are merged unless the caller caps the phases (a count of its own
   // width's) or GB_SSSP_SPANS=0.  A wider range may add a weight to a distance
