@@ -838,14 +838,16 @@ gb_status ms_run(gb_graph g, const int32_t *h_src, int32_t nsrc, bool with_sigma
   const int64_t hmax = g->E / c.hub + 1, omax = g->E / c.bch + 1;
   GB_TRY(w.hub_in.ensure(sizeof(HubRow) * hmax));
   GB_TRY(w.in_chunks.ensure(sizeof(HubChunk) * 2 * hmax));
-  GB_TRY(w.hub_out.ensure(sizeof(HubRow) * omax));
-  GB_TRY(w.out_chunks.ensure(sizeof(HubChunk) * 2 * omax));
+  const bool same = c.rp == c.rrp && c.hub == c.bch;  // one list serves both
+  if (with_sigma && !same) {
+    GB_TRY(w.hub_out.ensure(sizeof(HubRow) * omax));
+    GB_TRY(w.out_chunks.ensure(sizeof(HubChunk) * 2 * omax));
+  }
   GB_TRY(w.hub_meta.ensure(sizeof(unsigned long long) * 4));
   GB_HIP(hipMemsetAsync(w.hub_meta.p, 0, sizeof(unsigned long long) * 4, st));
   unsigned long long *hm = w.hub_meta.as<unsigned long long>();
   hipLaunchKernelGGL(mbc_hub_list_kernel, dim3(vgrid), dim3(256), 0, st, V, c.rrp, c.hub,
                      w.hub_in.as<HubRow>(), w.in_chunks.as<HubChunk>(), hm + 0);
-  const bool same = c.rp == c.rrp && c.hub == c.bch;  // one list serves both
   if (with_sigma && !same)
     hipLaunchKernelGGL(mbc_hub_list_kernel, dim3(vgrid), dim3(256), 0, st, V, c.rp, c.bch,
                        w.hub_out.as<HubRow>(), w.out_chunks.as<HubChunk>(), hm + 2);
