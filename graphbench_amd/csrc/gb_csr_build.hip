@@ -39,7 +39,7 @@ constexpr int RS_BLOCK = 256;
 constexpr int RS_WAVES = RS_BLOCK / GB_WAVE;
 constexpr int RS_TILE = 8192;
 constexpr int RS_ITEMS = RS_TILE / RS_BLOCK;       // edges per thread
-// the scatter: 8 waves per tile, each over RS_SEG consecutive edges
+// the scatter: 16 waves per tile, each over RS_SEG consecutive edges
 constexpr int RS_SBLOCK = 1024;
 constexpr int RS_SWAVES = RS_SBLOCK / GB_WAVE;
 constexpr int RS_SITEMS = RS_TILE / RS_SBLOCK;
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(RS_BLOCK) void expand_rows_kernel(int32_t V, int64_
 // and freeing it took 1.5 ms of a 5.4 ms build).  One build uses it at a time,
 // on any thread and stream: a build waits for its stream before it lets go of
 // the scratch.  An allocation that would fail elsewhere takes it back first
-// (gb_csr_trim).
+// (gb_csr_trim), a build whose own allocations fail gives up what it does not use.
 constexpr size_t CSR_KEEP = (size_t)4 << 30;
 struct CsrWork {
   std::atomic<int> busy{0};
@@ -422,7 +422,11 @@ struct CsrWork {
            total.bytes + flag.bytes;
   }
   void release() {
-    for (DevBuf *b : {&rows, &k[0], &k[1], &v, &w, &hist, &gsum, &total, &flag}) b->release();
+    rows.release();
+    release_sort();
+  }
+  void release_sort() {  // all but the row ids of a transpose
+    for (DevBuf *b : {&k[0], &k[1], &v, &w, &hist, &gsum, &total, &flag}) b->release();
   }
 };
 // Holds the scratch for one build; at most CSR_KEEP bytes outlive it.
@@ -645,10 +649,19 @@ gb_status csr_build(CsrWork &k, int32_t V, int64_t E, const int32_t *d_src, cons
 gb_status csr_build_any(CsrWork &k, int32_t V, int64_t E, const int32_t *d_src,
                         const int32_t *d_dst, const void *d_w, int32_t w_bytes, int32_t *d_row_ptr,
                         int32_t *d_col, void *d_w_out, hipStream_t st) {
-  const gb_status s =
-      w_bytes == 8   ? csr_build<8>(k, V, E, d_src, d_dst, d_w, d_row_ptr, d_col, d_w_out, st)
-      : w_bytes == 4 ? csr_build<4>(k, V, E, d_src, d_dst, d_w, d_row_ptr, d_col, d_w_out, st)
-                     : csr_build<0>(k, V, E, d_src, d_dst, d_w, d_row_ptr, d_col, d_w_out, st);
+  auto build = [&]() {
+    return w_bytes == 8   ? csr_build<8>(k, V, E, d_src, d_dst, d_w, d_row_ptr, d_col, d_w_out, st)
+           : w_bytes == 4 ? csr_build<4>(k, V, E, d_src, d_dst, d_w, d_row_ptr, d_col, d_w_out, st)
+                          : csr_build<0>(k, V, E, d_src, d_dst, d_w, d_row_ptr, d_col, d_w_out, st);
+  };
+  gb_status s = build();
+  if (s == GB_ERR_NOMEM) {
+    // nothing is queued yet but a transpose's row ids: without what earlier
+    // builds left, once more
+    k.release_sort();
+    if (d_dst != k.rows.p) k.rows.release();
+    s = build();
+  }
   if (s != GB_OK) (void)hipStreamSynchronize(st);  // launches before an error end first
   return s;
 }
@@ -695,7 +708,12 @@ extern "C" gb_status gb_csr_transpose(int32_t V, int64_t E, const int32_t *d_row
   hipStream_t st = gb_stream(stream);
   CsrHold hold(csr_work());
   CsrWork &k = hold.k;
-  GB_TRY(k.rows.ensure(sizeof(int32_t) * ((size_t)E + 1)));
+  gb_status rs = k.rows.ensure(sizeof(int32_t) * ((size_t)E + 1));
+  if (rs == GB_ERR_NOMEM) {
+    k.release();
+    rs = k.rows.ensure(sizeof(int32_t) * ((size_t)E + 1));
+  }
+  GB_TRY(rs);
   if (E > 0 && V > 0) {
     hipLaunchKernelGGL(expand_rows_kernel, dim3((unsigned)((E + EX_TILE - 1) / EX_TILE)),
                        dim3(RS_BLOCK), 0, st, V, E, d_row_ptr, k.rows.as<int32_t>());
