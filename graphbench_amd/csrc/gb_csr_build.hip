@@ -410,12 +410,15 @@ __global__ __launch_bounds__(RS_BLOCK) void expand_rows_kernel(int32_t V, int64_
 
 // Scratch of the builds, kept between calls up to CSR_KEEP bytes (allocating
 // and freeing it took 1.5 ms of a 5.4 ms build).  One build uses it at a time,
-// on any thread and stream: a build waits for its stream before it lets go of
-// the scratch.  An allocation that would fail elsewhere takes it back first
-// (gb_csr_trim), a build whose own allocations fail gives up what it does not use.
+// on any thread, stream and device: a build waits for its stream before it lets
+// go of the scratch, and one on another device starts with none.  An allocation
+// that would fail elsewhere in the library takes it back first (gb_csr_trim), a
+// build whose own allocations fail gives up what it does not use;
+// gb_release_workspaces returns it to other allocators.
 constexpr size_t CSR_KEEP = (size_t)4 << 30;
 struct CsrWork {
   std::atomic<int> busy{0};
+  int device = -1;  // where the buffers are
   DevBuf rows, k[2], v, w, hist, gsum, total, flag;
   size_t held() const {
     return rows.bytes + k[0].bytes + k[1].bytes + v.bytes + w.bytes + hist.bytes + gsum.bytes +
@@ -438,6 +441,10 @@ struct CsrHold {
       idle = 0;
       std::this_thread::yield();
     }
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    if (dev != k.device) k.release();
+    k.device = dev;
   }
   ~CsrHold() {
     if (k.held() > CSR_KEEP) k.release();

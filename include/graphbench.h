@@ -55,7 +55,10 @@ const char *gb_last_error(void);
 gb_status gb_init(int32_t device);
 /* Cap on bytes the library itself allocates (0 = no cap). */
 void gb_set_mem_cap(uint64_t bytes);
-/* Release cached workspaces. */
+/* Release cached workspaces: the scratch of the solves and, up to 4 GiB, of the
+ * last CSR build (graph builds below).  They stay allocated between calls; an
+ * allocation of the library takes the CSR scratch back when it would fail, other
+ * allocators get it by this call. */
 void gb_release_workspaces(void);
 /* Library version string. */
 const char *gb_version(void);
