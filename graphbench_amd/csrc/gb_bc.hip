@@ -211,7 +211,8 @@ __global__ void bc_accum_kernel(int32_t V, int32_t nslots, const int32_t *__rest
 // distances: R-MAT 13 with 16 sources 22.5 ms, now 0.6 ms; 16384 vertices with
 // 196 K edges and 32 sources 28 ms, now 1.3 ms.  The steps and the operand
 // order of the dependencies are the kernels' above; sigma is added
-// instead of pulled (exact in any order below 2^53), a dependency is summed by
+// instead of pulled (exact in any order below 2^53; beyond, the last bits follow
+// the order in which lanes arrive, and vary between runs), a dependency is summed by
 // 8 lanes, or by a wave from BCS_HUB out-edges on, in a fixed order.
 constexpr int BCS_G = 8;        // lanes per vertex in the backward pass
 constexpr int BCS_HUB = 128;

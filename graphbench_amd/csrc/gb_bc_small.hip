@@ -14,8 +14,10 @@
 // Replaces comp_num_spath / comp_delta (csr_bc.c:70-96, 98-123) per source and
 // the accumulation of csr_bc.c:57-61, as gb_msbc.hip does; the sums of a
 // vertex's successors run in a fixed order (8 lanes, or a wave for a vertex
-// of 128 out-edges or more, then a butterfly), so results do not vary between
-// runs or with the batch.
+// of 128 out-edges or more, then a butterfly), so results do not vary with the
+// batch, nor between runs while path counts stay below 2^53 (they are whole
+// numbers added in the order the lanes arrive: exact up to there, rounded in that
+// order beyond, as in the pushes of gb_msbc.hip).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -76,7 +78,7 @@ __global__ __launch_bounds__(SM_BLOCK) void bc_small_kernel(SmGraph<void> G, SbS
   }
   __syncthreads();
   // forward: level [a, b) of the order discovers the next one.  sigma holds
-  // whole numbers, so its adds are exact in any order.
+  // whole numbers, so its adds are exact in any order (below 2^53).
   uint32_t a = 0, b = 1, depth = 1;
   for (;;) {
     sm_expand(
@@ -211,7 +213,7 @@ void gb_bc_small_release() { sbw().release(); }
 // sources 549 against 2453; 14336 vertices, 459 K edges, 256 / 1024 sources 597
 // / 2280 against 3165 / 4818.
 bool gb_bc_small_fits(gb_graph g) {
-  for (const char *k : {"GB_BC_GRID", "GB_BC_ALPHA", "GB_BC_HUB", "GB_BC_BCHUNK", "GB_BC_TUNE"}) {
+  for (const char *k : {"GB_BC_GRID", "GB_BC_ALPHA", "GB_BC_HUB", "GB_BC_BCHUNK"}) {
     const char *e = getenv(k);
     if (e && e[0]) return false;
   }

@@ -22,7 +22,7 @@
 //   * push: one wave per item of at most PUSH_CH out-edges of an L_d vertex;
 //     an edge to x carries the sources of the vertex's level-d mask that have
 //     not reached x: their sigma is added to x's by FP64 atomicAdd (integers:
-//     exact in any order), the bits are ORed into x's next-level mask, and the
+//     exact in any order below 2^53), the bits are ORed into x's next-level mask, and the
 //     lane whose OR found the mask empty appends x to L_{d+1};
 //   * pull: a scan lists the vertices with 1..hub in-edges that some source
 //     has not reached; one wave per listed vertex sums, lane s, sigma[u][s]

@@ -184,20 +184,21 @@ __device__ __forceinline__ MsIn ms_load(const MsCtx &c, const unsigned long long
   return r;
 }
 
-// Light phase: expand the entries of near queue a_in.  Entries are software
-// pipelined: entry i is expanded while entry i + nwaves's loads and entry
-// i + 2 nwaves's descriptor are in flight.
-// WIDE: the distance array is 4 GiB or more.  Below, its byte offsets are 32 bits.
-// What bounds the step beside its lines is instructions per (edge, source): with
-// a 64-bit multiply for the bucket of every new distance, 64-bit offsets and
-// counters per lane, R-MAT 24 with 32 sources took 48.9 ms; a compare with the
-// bucket's end 42.6; saturating adds, counts of ballots and 32-bit offsets 40.3.
+// The distance of source t at vertex x.  WIDE: the array is 4 GiB or more; below,
+// its byte offsets are 32 bits.
 template <int W, bool WIDE>
 __device__ __forceinline__ uint32_t *ms_dist(uint32_t *dist, int32_t x, int t) {
   if (WIDE) return dist + ((int64_t)x * W + t);
   return (uint32_t *)((char *)dist + ((uint32_t)x * (W * 4u) + (uint32_t)t * 4u));
 }
 
+// Light phase: expand the entries of near queue a_in.  Entries are software
+// pipelined: entry i is expanded while entry i + nwaves's loads and entry
+// i + 2 nwaves's descriptor are in flight.
+// What bounds the step beside its lines is instructions per (edge, source): with
+// a 64-bit multiply for the bucket of every new distance, 64-bit offsets and
+// counters per lane, R-MAT 24 with 32 sources took 48.9 ms; a compare with the
+// bucket's end 42.6; saturating adds, counts of ballots and 32-bit offsets 40.3.
 // The counters are the wave's (uniform).
 template <int W, bool SCAN, bool WIDE>
 __device__ __forceinline__ void ms_light(const MsCtx &c, const MsIo &io, uint64_t b, bool all,
@@ -748,8 +749,9 @@ __global__ void ms_count_kernel(int64_t V, int32_t nsrc, const int32_t *__restri
 // Step-kernel blocks per CU when the autotuner does not run: 4 below 2^23
 // edges (small phases: fewer idle blocks to launch and flush), 8 up to 2^25,
 // 16 beyond (more waves in flight in the large phases).  Measured at 4 / 8 /
-// 16 blocks per CU: R-MAT 16 with 8 sources 3.3 / 3.7-3.9 / 4.7 ms; R-MAT 22
-// with 32 sources 27.9 / 26.3-27.2 / 26.3-26.5 ms.
+// 16 blocks per CU: R-MAT 16 with 8 sources 1.13 / 1.67 / 2.29 ms; with 32 sources
+// R-MAT 20 20.2 / 15.8 / 15.7 ms, R-MAT 22 90 / 67.0 / 65.9, R-MAT 24 (learned width)
+// 42.2 / 33.0 / 32.5.
 int ms_rule_per_cu(int64_t E) {
   return E < ((int64_t)1 << 23) ? 4 : E < ((int64_t)1 << 25) ? 8 : 16;
 }
@@ -757,8 +759,11 @@ constexpr int MS_MAX_PER_CU = 16;
 
 // The scan form pays a pass over V per phase, the append form a returning
 // atomic and a row-bound read per newly marked target inside the step.
-// Measured with 8 sources of R-MAT 16 (185 phases): append 3.3 ms, scan
-// 4.3 ms; with 32 sources of R-MAT 24 (12 phases): append 61 ms, scan 54 ms.
+// Measured, append / scan, plain width: R-MAT 17 with 8 sources 1.45 / 1.94 ms,
+// 32 sources 3.19 / 3.26; R-MAT 19 4.34 / 4.75 and 7.51 / 6.30; R-MAT 20 5.36 /
+// 6.52 and 16.1 / 14.2; R-MAT 22 27.0 / 30.5 and 74.1 / 67.4; uniform graphs of
+// 2^18 vertices 2.11 / 2.10 and 4.12 / 3.74, of 2^20 7.50 / 6.36 and 16.6 / 11.1.
+// R-MAT 24 with the learned width: 8 sources 22.6 / 25.3 ms, 32 sources 40.0 / 34.5.
 // This is the rule when the autotuner does not run.
 bool ms_rule_scan(int64_t V) { return V >= ((int64_t)1 << 20); }
 
@@ -956,8 +961,8 @@ gb_status ms_group_shape(MsCtx c, const int32_t *d_src, int max_phases, const Ms
 // the group is solved in several shapes (every solve is exact, so each leaves
 // the same distances): the rules' shape, then one change at a time (the other
 // form, the other blocks-per-CU counts, the other chunk), keeping a change
-// when it is faster.  A shape's time is the wall time of its solve, graph
-// capture and host waits included; below 20 ms, the better of two solves.
+// when it is faster.  A shape's time is the wall time of its solve, host waits
+// included; below 20 ms, the better of two solves.
 // The stats returned are those of the kept shape's solve.
 template <int W>
 gb_status ms_group_tuned(gb_graph g, MsCtx c, const int32_t *d_src, int max_phases,
