@@ -245,7 +245,7 @@ __global__ __launch_bounds__(SM_BLOCK) void bcw_small_kernel(SmGraph<double> G, 
   const int32_t s0 = src.s[blockIdx.x];
   SmStats st;
   uint32_t sweep = 0;
-  sm_solve(s, G, s0, width, sweep, st);
+  sm_solve<false>(s, G, s0, width, 0, sweep, st);
   // s.dist is only read from here on
   for (int v = tid; v < G.V; v += SM_BLOCK) {
     sigma[v] = 0.0;

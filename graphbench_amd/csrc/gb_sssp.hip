@@ -775,13 +775,14 @@ struct SmSources {
 
 template <class Tr, int VCAP>
 __global__ __launch_bounds__(SM_BLOCK) void sssp_small_kernel(SmGraph<typename Tr::W> G,
-                                                              SmSources src, typename Tr::T width,
+                                                              SmSources src, typename Tr::T delta,
+                                                              uint64_t magic,
                                                               typename Tr::D *dist,
                                                               SmStats *out) {
   __shared__ SmLds<Tr, VCAP> s;
   SmStats st;
   uint32_t sweep = 0;
-  sm_solve(s, G, src.s[blockIdx.x], width, sweep, st);
+  sm_solve<true>(s, G, src.s[blockIdx.x], delta, magic, sweep, st);
   typename Tr::D *row = dist + (int64_t)blockIdx.x * G.V;
   for (int v = threadIdx.x; v < G.V; v += SM_BLOCK) row[v] = Tr::val(s.dist[v]);
   if (threadIdx.x == 0) out[blockIdx.x] = st;
@@ -804,17 +805,17 @@ bool sm_fits(int32_t V, int64_t E, int32_t nsrc) {
 }
 
 template <class Tr, int VCAP>
-void sm_launch(int n, const SmGraph<typename Tr::W> &G, const SmSources &src, typename Tr::T width,
+void sm_launch(int n, const SmGraph<typename Tr::W> &G, const SmSources &src, typename Tr::T delta,
                typename Tr::D *dist, SmStats *out, hipStream_t st) {
-  hipLaunchKernelGGL((sssp_small_kernel<Tr, VCAP>), dim3(n), dim3(SM_BLOCK), 0, st, G, src, width,
-                     dist, out);
+  hipLaunchKernelGGL((sssp_small_kernel<Tr, VCAP>), dim3(n), dim3(SM_BLOCK), 0, st, G, src, delta,
+                     Tr::host_magic(delta), dist, out);
 }
 
 // Solves all sources; *ovf set when some sum overflowed (the distances are
 // then not to be used: the caller repeats the solve with an engine, whose
 // narrower buckets decide whether the call fails).
 template <class Tr>
-gb_status sm_run(const SmGraph<typename Tr::W> &G, typename Tr::T width, const int32_t *h_sources,
+gb_status sm_run(const SmGraph<typename Tr::W> &G, typename Tr::T delta, const int32_t *h_sources,
                  int32_t nsrc, typename Tr::D *d_dist, gb_sssp_stats *stats, bool *ovf,
                  hipStream_t st) {
   static SmStats *res = nullptr;  // pinned, kept for the process's life
@@ -836,9 +837,9 @@ gb_status sm_run(const SmGraph<typename Tr::W> &G, typename Tr::T width, const i
     typename Tr::D *rows = d_dist + (int64_t)g0 * G.V;
     constexpr int BIG = sizeof(typename Tr::D) == 4 ? 32768 : 16384;
     if (G.V <= BIG / 4)
-      sm_launch<Tr, BIG / 4>(n, G, src, width, rows, res, st);
+      sm_launch<Tr, BIG / 4>(n, G, src, delta, rows, res, st);
     else
-      sm_launch<Tr, BIG>(n, G, src, width, rows, res, st);
+      sm_launch<Tr, BIG>(n, G, src, delta, rows, res, st);
     err = hipGetLastError();
     if (stats && g0 + n >= nsrc) (void)hipEventRecord(e1, st);
     if (err == hipSuccess) err = hipStreamSynchronize(st);

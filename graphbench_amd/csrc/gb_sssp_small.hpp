@@ -56,6 +56,14 @@ struct SmU32 {
   static __device__ __forceinline__ T widen(T width) {
     return width < (1ull << 32) ? width * 2 : width;
   }
+  // whether d + w stays in d's bucket of width delta (< 2^32); magic:
+  // floor((2^64 - 1) / delta) + 1, which makes the quotient exact (0: delta is 1)
+  static __device__ __forceinline__ bool stays(D d, W w, T delta, uint64_t magic) {
+    const uint32_t dl = (uint32_t)delta;
+    if (w >= dl) return false;
+    return magic == 0 || w < dl - (d - (uint32_t)__umul64hi(d, magic) * dl);
+  }
+  static uint64_t host_magic(T delta) { return delta > 1 ? (~0ull / delta) + 1 : 0; }
 };
 struct SmF64 {
   using D = double;
@@ -78,6 +86,10 @@ struct SmF64 {
     return t > lo ? t : __longlong_as_double(__double_as_longlong(lo) + 1);
   }
   static __device__ __forceinline__ T widen(T width) { return width * 2.0; }
+  static __device__ __forceinline__ bool stays(D d, W w, T delta, uint64_t) {
+    return (uint64_t)(long long)(__dadd_rn(d, w) / delta) == (uint64_t)(long long)(d / delta);
+  }
+  static uint64_t host_magic(T) { return 0; }
 };
 
 // W void: no weights
@@ -206,10 +218,13 @@ __device__ __forceinline__ void sm_expand(SmShare &s, const SmGraph<W> &G, uint3
   __syncthreads();
 }
 
-// Distances from src into s.dist (bits); every thread of the block.
-template <class Tr, int VCAP>
+// Distances from src into s.dist (bits); every thread of the block.  COUNT: the
+// improvements by whether they leave the bucket of the caller's width delta,
+// whatever the thresholds.
+template <bool COUNT, class Tr, int VCAP>
 __device__ __forceinline__ void sm_solve(SmLds<Tr, VCAP> &s, const SmGraph<typename Tr::W> &G,
-                                         int32_t src, typename Tr::T width, uint32_t &sweep, SmStats &st) {
+                                         int32_t src, const typename Tr::T delta, uint64_t magic,
+                                         uint32_t &sweep, SmStats &st) {
   using D = typename Tr::D;
   using Bits = typename Tr::Bits;
   const int tid = threadIdx.x, lane = gb_lane();
@@ -222,9 +237,9 @@ __device__ __forceinline__ void sm_solve(SmLds<Tr, VCAP> &s, const SmGraph<typen
     s.dist[src] = 0;
     s.pend[src >> 5] = 1u << (src & 31);
   }
-  typename Tr::T T = Tr::next((D)0, width);
+  typename Tr::T width = delta, T = Tr::next((D)0, width);
   uint32_t edges = 0;  // under the current threshold
-  uint32_t relax = 0, near = 0, far = 0;
+  uint32_t relax = 0, near = 0, imp = 0;
   bool ovf = false;
   st.buckets = 1;
   st.phases = 0;
@@ -309,9 +324,10 @@ __device__ __forceinline__ void sm_solve(SmLds<Tr, VCAP> &s, const SmGraph<typen
             if (in[u] & (nb < old[u])) {
               atomicMin(&s.dist[x[u]], nb);
               atomicOr(&s.pend[x[u] >> 5], 1u << (x[u] & 31));
-              const bool b = Tr::below(nd, T);
-              near += b;
-              far += !b;
+              if (COUNT) {
+                imp++;
+                near += Tr::stays(Tr::val(du[u]), w[u], delta, magic);
+              }
             }
           }
         });
@@ -334,7 +350,7 @@ __device__ __forceinline__ void sm_solve(SmLds<Tr, VCAP> &s, const SmGraph<typen
     }
   if (tid < 6) s.acc[tid] = 0;
   __syncthreads();
-  const unsigned long long mine[6] = {relax, near, far, reached, trav, ovf ? 1ull : 0ull};
+  const unsigned long long mine[6] = {relax, near, imp - near, reached, trav, ovf ? 1ull : 0ull};
 #pragma unroll
   for (int i = 0; i < 6; i++) {
     unsigned long long t = mine[i];
