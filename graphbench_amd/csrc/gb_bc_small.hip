@@ -207,18 +207,24 @@ SbWork &sbw() {
 
 void gb_bc_small_release() { sbw().release(); }
 
-// A CU takes about 0.6 ns per edge and direction, the engine some 2 ms of
-// launches per call.  Measured, workgroups against engine (us): 4096 vertices,
-// 131 K edges, 50 / 256 sources 225 / 242 against 2232 / 2514; 524 K edges, 50
-// sources 549 against 2453; 14336 vertices, 459 K edges, 256 / 1024 sources 597
-// / 2280 against 3165 / 4818.
-bool gb_bc_small_fits(gb_graph g) {
+// A launch of up to SB_SOURCES sources takes 1 to 2 ns an edge, as long as its
+// slowest CU, however few they are; the engine 0.3 to 0.5 ms of phases and less per
+// edge and source the more there are.  So the line lies at a product of launches and
+// edges.  Measured, workgroups against engine (us): uniform, R-MAT and a graph with
+// one vertex in two thirds of its edges; 4096 vertices, 131 K edges, 256 sources 181
+// / 243 / 281 against 579 / 828 / 468, 1024 sources 628 / 861 / 1026 against 1131 /
+// 1436 / 814; 262 K edges, 512 sources 464 / 678 / 946 against 829 / 984 / 661; 524 K
+// edges, 256 sources 553 / 586 / 896 against 721 / 930 / 633, 1024 sources 2082 / 2209
+// / 3504 against 1594 / 1681 / 1146.  14336 vertices, 524 K edges, 1024 sources 2014
+// / 2478 / 4137 against 2461 / 2137 / 1244.
+bool gb_bc_small_fits(gb_graph g, int32_t nsrc) {
   for (const char *k : {"GB_BC_GRID", "GB_BC_ALPHA", "GB_BC_HUB", "GB_BC_BCHUNK"}) {
     const char *e = getenv(k);
     if (e && e[0]) return false;
   }
   const char *e = getenv("GB_BC_SMALL");
-  return !(e && e[0] == '0') && g->V <= SB_MAX_V && g->E <= ((int64_t)1 << 19);
+  return !(e && e[0] == '0') && g->V <= SB_MAX_V &&
+         g->E * (((int64_t)nsrc + SB_SOURCES - 1) / SB_SOURCES) <= ((int64_t)1 << 19);
 }
 
 gb_status gb_bc_small_run(gb_graph g, const int32_t *h_sources, int32_t nsrc, double *d_bc,

@@ -205,7 +205,8 @@ void gb_bc_release();
 void gb_msbc_release();
 // Unweighted Brandes with one workgroup per source (gb_bc_small.hip): adds the
 // dependencies to d_bc, *depth the most levels of a source.
-bool gb_bc_small_fits(gb_graph g);
+// The form serves a call of nsrc sources (all of them, however batched).
+bool gb_bc_small_fits(gb_graph g, int32_t nsrc);
 gb_status gb_bc_small_run(gb_graph g, const int32_t *h_sources, int32_t nsrc, double *d_bc,
                           int32_t *depth, hipStream_t st);
 void gb_bc_small_release();

@@ -1076,14 +1076,15 @@ extern "C" gb_status gb_bc(gb_graph g, const int32_t *h_sources, int32_t nsrc, i
   if (V > 0 && per * (int64_t)V > cap_entries) per = std::max<int64_t>(64, (cap_entries / V) / 64 * 64);
   int32_t max_depth = 0, batches = 0;
   std::vector<int32_t> order;
-  if (V > 0 && nsrc > 0 && !gb_bc_small_fits(g)) {
+  const bool small = gb_bc_small_fits(g, nsrc);
+  if (V > 0 && nsrc > 0 && !small) {
     GB_TRY(bc_order(g, h_sources, nsrc, order, st));
     h_sources = order.data();
   }
   for (int32_t b0 = 0; b0 < nsrc && V > 0; b0 += (int32_t)per) {
     const int32_t ns = (int32_t)std::min<int64_t>(per, nsrc - b0);
     int32_t depth = 0;
-    if (gb_bc_small_fits(g)) {
+    if (small) {
       GB_TRY(gb_bc_small_run(g, h_sources + b0, ns, d_bc, &depth, st));
       max_depth = std::max(max_depth, depth - 1);
       batches++;
