@@ -245,7 +245,7 @@ __global__ __launch_bounds__(SM_BLOCK) void bcw_small_kernel(SmGraph<double> G, 
   const int32_t s0 = src.s[blockIdx.x];
   SmStats st;
   uint32_t sweep = 0;
-  sm_solve<false>(s, G, s0, width, 0, sweep, st);
+  sm_solve<false>(s, G, s0, width, width, 0, sweep, st);
   // s.dist is only read from here on
   for (int v = tid; v < G.V; v += SM_BLOCK) {
     sigma[v] = 0.0;
@@ -446,7 +446,15 @@ gb_status forward_levels(gb_graph g, int32_t nslots, hipStream_t st,
 }
 
 // Where the workgroup form serves: distances in LDS, and edges that one CU
-// reads in less time than the engine's launches take.
+// reads in about the time of the engine's launches.  The engine's time follows the
+// depth of the tight edges and the longest rows (a wave each), one workgroup's the
+// edges.  Measured, workgroups against engine (ms), 1 M edges, 1 / 16 / 64 sources:
+// uniform, 4000 vertices 2.56 / 2.58 / 2.63 against 1.15 / 2.14 / 5.36, 16384 vertices
+// 3.26 / 3.30 / 3.37 against 1.46 / 3.92 / 12.2; R-MAT 16384 3.39 / 3.49 / 3.61 against
+// 6.3 / 12.4 / 26.5; two thirds of the edges at one vertex 4.6 / 4.8 / 4.7 against 61 /
+// 94 / 142; 262 K edges, every graph and number of sources, 2 to 40 times.  Past 2^18
+// edges few sources of a uniform graph lose up to a factor of 2 by this line, what
+// others win by it is larger.
 constexpr int32_t BCS_MAX_V = 16384;
 constexpr int64_t BCS_MAX_E = (int64_t)1 << 20;
 

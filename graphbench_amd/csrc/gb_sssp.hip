@@ -775,14 +775,14 @@ struct SmSources {
 
 template <class Tr, int VCAP>
 __global__ __launch_bounds__(SM_BLOCK) void sssp_small_kernel(SmGraph<typename Tr::W> G,
-                                                              SmSources src, typename Tr::T delta,
-                                                              uint64_t magic,
+                                                              SmSources src, typename Tr::T width,
+                                                              typename Tr::T delta, uint64_t magic,
                                                               typename Tr::D *dist,
                                                               SmStats *out) {
   __shared__ SmLds<Tr, VCAP> s;
   SmStats st;
   uint32_t sweep = 0;
-  sm_solve<true>(s, G, src.s[blockIdx.x], delta, magic, sweep, st);
+  sm_solve<true>(s, G, src.s[blockIdx.x], width, delta, magic, sweep, st);
   typename Tr::D *row = dist + (int64_t)blockIdx.x * G.V;
   for (int v = threadIdx.x; v < G.V; v += SM_BLOCK) row[v] = Tr::val(s.dist[v]);
   if (threadIdx.x == 0) out[blockIdx.x] = st;
@@ -790,32 +790,51 @@ __global__ __launch_bounds__(SM_BLOCK) void sssp_small_kernel(SmGraph<typename T
 
 // One CU relaxes about one edge per ns, whatever the chip could do beside it,
 // so the form serves graphs of up to 2^18 edges, and up to 2^20 when enough
-// sources keep many CUs busy.  Measured against the engines (us, plain width /
-// width 128): R-MAT 12, 65 K edges, one source 193 against 1433 / 171 against
-// 737; 16384 vertices, 262 K edges 474 against 1669 / 462 against 758; 32768
-// vertices, 1 M edges, one source 1329 against 2309 / 1655 against 812 (the
-// engine), 64 sources 1939 against 13363 / 2450 against 2813.
+// sources keep many CUs busy.  Its thresholds start the plain rule's width apart
+// at most: with the caller's, a wide bucket relaxed edges again that no lanes were
+// free for (32768 uniform vertices, 1 M edges, 32 sources, width 100000: 3.6 ms,
+// now 1.16; plain width 1.17).  Measured against the engines (us, plain width / width
+// 100000; several sources: the engine once its shape is tuned, which takes 10 to 20
+// ms of a first call): one source, 8000 vertices, 65 K edges uniform 251 against 487
+// / 249 against 400, R-MAT 213 against 350 / 212 against 285; 262 K edges 347
+// against 477 / 344 against 410 and 359 against 369 / 355 against 287; 32768
+// vertices, 262 K edges 721 against 639 / 716 against 557 and 629 against 439 / 626
+// against 403; 1 M edges, 32 sources 1168 against 1273 / 1159 against 1089 and 1437
+// against 1454 / 1438 against 706, 300 sources 2381 against 9333 / 2386 against 7238
+// and 3202 against 10204 / 3215 against 4525.  So a width of many plain ones is the
+// engine's, past 2^17 edges with one source and past 2^19 with less than 64.
+// FP64 weights, whose thresholds start by a sample's mean weight: 16384 vertices, 1 M
+// edges, 64 sources 1059 uniform, 1296 R-MAT, whatever the width; engine, 32 sources,
+// 1205 to 2286 and 1892 to 2086.
 constexpr int64_t SM_MAX_E = (int64_t)1 << 18, SM_MAX_E_MANY = (int64_t)1 << 20;
 constexpr int32_t SM_MANY = 32;
+constexpr int64_t SM_MAX_E_WIDE = (int64_t)1 << 17, SM_MAX_E_WIDE_MANY = (int64_t)1 << 19;
+constexpr uint32_t SM_WIDE = 16;  // plain widths
 template <class Tr>
 bool sm_fits(int32_t V, int64_t E, int32_t nsrc) {
   const int32_t max_v = sizeof(typename Tr::D) == 4 ? 32768 : 16384;
   return nsrc > 0 && V <= max_v && E <= (nsrc >= SM_MANY ? SM_MAX_E_MANY : SM_MAX_E) &&
          gb_sssp_small_enabled();
 }
+// A width of many plain ones leaves the engine few phases.
+bool sm_few_phases(int64_t E, int32_t nsrc, uint32_t delta, uint32_t plain) {
+  return nsrc < 2 * SM_MANY && E > (nsrc == 1 ? SM_MAX_E_WIDE : SM_MAX_E_WIDE_MANY) &&
+         delta / SM_WIDE >= plain;
+}
 
 template <class Tr, int VCAP>
-void sm_launch(int n, const SmGraph<typename Tr::W> &G, const SmSources &src, typename Tr::T delta,
-               typename Tr::D *dist, SmStats *out, hipStream_t st) {
-  hipLaunchKernelGGL((sssp_small_kernel<Tr, VCAP>), dim3(n), dim3(SM_BLOCK), 0, st, G, src, delta,
-                     Tr::host_magic(delta), dist, out);
+void sm_launch(int n, const SmGraph<typename Tr::W> &G, const SmSources &src, typename Tr::T width,
+               typename Tr::T delta, typename Tr::D *dist, SmStats *out, hipStream_t st) {
+  hipLaunchKernelGGL((sssp_small_kernel<Tr, VCAP>), dim3(n), dim3(SM_BLOCK), 0, st, G, src, width,
+                     delta, Tr::host_magic(delta), dist, out);
 }
 
 // Solves all sources; *ovf set when some sum overflowed (the distances are
 // then not to be used: the caller repeats the solve with an engine, whose
 // narrower buckets decide whether the call fails).
 template <class Tr>
-gb_status sm_run(const SmGraph<typename Tr::W> &G, typename Tr::T delta, const int32_t *h_sources,
+gb_status sm_run(const SmGraph<typename Tr::W> &G, typename Tr::T width,
+                 typename Tr::T delta, const int32_t *h_sources,
                  int32_t nsrc, typename Tr::D *d_dist, gb_sssp_stats *stats, bool *ovf,
                  hipStream_t st) {
   static SmStats *res = nullptr;  // pinned, kept for the process's life
@@ -837,9 +856,9 @@ gb_status sm_run(const SmGraph<typename Tr::W> &G, typename Tr::T delta, const i
     typename Tr::D *rows = d_dist + (int64_t)g0 * G.V;
     constexpr int BIG = sizeof(typename Tr::D) == 4 ? 32768 : 16384;
     if (G.V <= BIG / 4)
-      sm_launch<Tr, BIG / 4>(n, G, src, delta, rows, res, st);
+      sm_launch<Tr, BIG / 4>(n, G, src, width, delta, rows, res, st);
     else
-      sm_launch<Tr, BIG>(n, G, src, delta, rows, res, st);
+      sm_launch<Tr, BIG>(n, G, src, width, delta, rows, res, st);
     err = hipGetLastError();
     if (stats && g0 + n >= nsrc) (void)hipEventRecord(e1, st);
     if (err == hipSuccess) err = hipStreamSynchronize(st);
@@ -943,10 +962,17 @@ extern "C" gb_status gb_sssp(gb_graph g, const gb_sssp_params *p, const int32_t 
   }
   if (lmax == 0) lmax = delta;
   if (!(p && p->max_phases > 0) && sm_fits<SmU32>(g->V, g->E, nsrc)) {
-    bool ovf = false;
-    GB_TRY(sm_run<SmU32>(SmGraph<uint32_t>{g->rp, g->col, g->w, g->V}, delta, h_sources, nsrc,
-                         d_dist, stats, &ovf, st));
-    if (!ovf) return GB_OK;
+    // thresholds no wider apart than the plain rule's: one workgroup has no
+    // lanes to spare for the edges that a wide bucket relaxes again
+    uint32_t mw = 0;
+    GB_TRY(gb_graph_max_w(g, &mw, st));
+    const uint32_t plain = plain_delta(mw, g->V, g->E);
+    if (!sm_few_phases(g->E, nsrc, delta, plain)) {
+      bool ovf = false;
+      GB_TRY(sm_run<SmU32>(SmGraph<uint32_t>{g->rp, g->col, g->w, g->V}, std::min(delta, plain),
+                           delta, h_sources, nsrc, d_dist, stats, &ovf, st));
+      if (!ovf) return GB_OK;
+    }
   }
   if (nsrc >= 2 && ms_enabled()) {
     // several sources: the batched engine (one entry per vertex and source mask)
@@ -998,8 +1024,8 @@ extern "C" gb_status gb_sssp_f64(gb_graph g, double delta, const int32_t *h_sour
   hipStream_t st = gb_stream(stream);
   if (sm_fits<SmF64>(g->V, g->E, nsrc)) {
     bool ovf = false;
-    return sm_run<SmF64>(SmGraph<double>{g->rp, g->col, g->w64, g->V}, delta, h_sources, nsrc,
-                         d_dist, stats, &ovf, st);
+    return sm_run<SmF64>(SmGraph<double>{g->rp, g->col, g->w64, g->V}, delta, delta, h_sources,
+                         nsrc, d_dist, stats, &ovf, st);
   }
   GB_TRY(check_degree(g, st));
   GB_TRY(gb_graph_split64(g, delta, st));

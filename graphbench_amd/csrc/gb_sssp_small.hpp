@@ -218,12 +218,13 @@ __device__ __forceinline__ void sm_expand(SmShare &s, const SmGraph<W> &G, uint3
   __syncthreads();
 }
 
-// Distances from src into s.dist (bits); every thread of the block.  COUNT: the
-// improvements by whether they leave the bucket of the caller's width delta,
-// whatever the thresholds.
+// Distances from src into s.dist (bits); every thread of the block.  The
+// thresholds start `width` apart.  COUNT: the improvements by whether they leave
+// the bucket of the caller's width delta, whatever the thresholds.
 template <bool COUNT, class Tr, int VCAP>
 __device__ __forceinline__ void sm_solve(SmLds<Tr, VCAP> &s, const SmGraph<typename Tr::W> &G,
-                                         int32_t src, const typename Tr::T delta, uint64_t magic,
+                                         int32_t src, typename Tr::T width,
+                                         const typename Tr::T delta, uint64_t magic,
                                          uint32_t &sweep, SmStats &st) {
   using D = typename Tr::D;
   using Bits = typename Tr::Bits;
@@ -232,12 +233,25 @@ __device__ __forceinline__ void sm_solve(SmLds<Tr, VCAP> &s, const SmGraph<typen
   for (int v = tid; v < V; v += SM_BLOCK) s.dist[v] = Tr::inf_bits();
   for (int i = tid; i < VCAP / 32; i += SM_BLOCK) s.pend[i] = 0;
   if (tid < SM_SWEEP / 64) s.start[sweep % 3][tid] = 0;
+  // FP64 weights: no wider than the plain rule's width, twice the mean weight over
+  // the mean degree, by a sample (the caller bounds the width of whole ones)
+  if constexpr (std::is_same<typename Tr::W, double>::value) {
+    const int64_t E = G.rp[V];
+    double *sum = (double *)s.own;
+    const double w = gb_wave_sum_f64(E > 0 ? G.w[tid * E / SM_BLOCK] : 0.0);
+    if (lane == 0) sum[tid >> 6] = w;
+    __syncthreads();
+    double mean = 0.0;
+    for (int q = 0; q < SM_WAVES; q++) mean += sum[q] / SM_BLOCK;
+    const double plain = E > 0 ? 2.0 * mean * V / E : 0.0;
+    if (plain > 0.0 && plain < width) width = plain;
+  }
   __syncthreads();
   if (tid == 0) {
     s.dist[src] = 0;
     s.pend[src >> 5] = 1u << (src & 31);
   }
-  typename Tr::T width = delta, T = Tr::next((D)0, width);
+  typename Tr::T T = Tr::next((D)0, width);
   uint32_t edges = 0;  // under the current threshold
   uint32_t relax = 0, near = 0, imp = 0;
   bool ovf = false;
