@@ -103,7 +103,7 @@ struct gb_graph_s {
   DevBuf pr_tile_row, pr_tile_edge;
   // PageRank on small graphs: the long rows' pieces for tiles of ps_tile items
   int32_t ps_tile = 0, ps_npieces = 0;
-  DevBuf ps_long, ps_pieces;
+  DevBuf ps_lists;
   // PageRank row blocks (row-block form), per edges-per-block and layout
   int32_t pr_rb_nb = 0;
   bool pr_rb_relabeled = false;

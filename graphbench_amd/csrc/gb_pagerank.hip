@@ -2084,17 +2084,18 @@ static gb_status pagerank_small(gb_graph g, const gb_pr_params *p, float *d_x, g
     g->pr_ntiles = nb;
   }
   PrWork &w = g_prw;
-  if (g->ps_tile != tile) {  // the long rows' pieces, once per handle
-    DevBuf count;
-    GB_TRY(g->ps_long.ensure(sizeof(PsLong) * nb));
-    GB_TRY(g->ps_pieces.ensure(sizeof(int2) * (2 * (g->E / PS_PIECE) + 1)));
-    GB_TRY(count.ensure(sizeof(int32_t)));
-    GB_HIP(hipMemsetAsync(count.p, 0, sizeof(int32_t), st));
+  GB_TRY(w.ps_done.ensure(2 * sizeof(int32_t)));  // the stop flag, a count
+  const int64_t most = 2 * (g->E / PS_PIECE) + 1;
+  if (g->ps_tile != tile && g->E > PS_ROW) {  // the long rows' pieces, once per handle
+    GB_TRY(g->ps_lists.ensure(sizeof(int2) * most + sizeof(PsLong) * nb));
+    int32_t *count = w.ps_done.as<int32_t>() + 1;
+    GB_HIP(hipMemsetAsync(count, 0, sizeof(int32_t), st));
+    int2 *pieces = g->ps_lists.as<int2>();
     hipLaunchKernelGGL(ps_long_list_kernel, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, st,
-                       (int32_t)nb, g->rrp, g->pr_tile_row.as<int32_t>(),
-                       g->ps_long.as<PsLong>(), g->ps_pieces.as<int2>(), count.as<int32_t>());
+                       (int32_t)nb, g->rrp, g->pr_tile_row.as<int32_t>(), (PsLong *)(pieces + most),
+                       pieces, count);
     GB_HIP(hipGetLastError());
-    GB_HIP(hipMemcpyAsync(&g->ps_npieces, count.p, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    GB_HIP(hipMemcpyAsync(&g->ps_npieces, count, sizeof(int32_t), hipMemcpyDeviceToHost, st));
     GB_HIP(hipStreamSynchronize(st));
     g->ps_tile = (int32_t)tile;
   }
@@ -2103,7 +2104,6 @@ static gb_status pagerank_small(gb_graph g, const gb_pr_params *p, float *d_x, g
   GB_TRY(w.ca.ensure(sizeof(float) * V));
   GB_TRY(w.cb.ensure(sizeof(float) * V));
   GB_TRY(w.pres.ensure(sizeof(double) * 4 * PS_MAX_BLOCKS));
-  GB_TRY(w.ps_done.ensure(sizeof(int32_t)));
   GbProgress *prog = nullptr;
   GB_TRY(gb_progress_begin(&prog));
   const int32_t *rows = g->pr_tile_row.as<int32_t>();
@@ -2114,13 +2114,13 @@ static gb_status pagerank_small(gb_graph g, const gb_pr_params *p, float *d_x, g
   hipLaunchKernelGGL(ps_init_kernel, dim3((unsigned)nb), dim3(PS_BLOCK), 0, st, V, p->d_x0, inv,
                      rows, d_x, c[0], part, done);
   GB_HIP(hipGetLastError());
-  const PsLong *longs = np > 0 ? g->ps_long.as<PsLong>() : nullptr;
+  const int2 *pieces = g->ps_lists.as<int2>();
+  const PsLong *longs = np > 0 ? (const PsLong *)(pieces + most) : nullptr;
   F2 *psum = np > 0 ? w.ps_sum.as<F2>() : nullptr;
   const gb_status gst = gb_drive_phases(prog, PS_AHEAD, st, [&](uint32_t k) {
     if (np > 0)
       hipLaunchKernelGGL(ps_long_kernel, dim3((unsigned)np), dim3(PS_BLOCK), 0, st,
-                         (const int2 *)g->ps_pieces.as<int2>(), g->rcol, (const float *)c[k & 1],
-                         psum);
+                         pieces, g->rcol, (const float *)c[k & 1], psum);
     hipLaunchKernelGGL(ps_iter_kernel, dim3((unsigned)nb), dim3(PS_BLOCK), 0, st, V, g->rrp,
                        g->rcol, rows, longs, (const F2 *)psum, inv, d_x, (const float *)c[k & 1],
                        c[(k + 1) & 1], part, done, (int32_t)k, p->max_iter, p->tol,
